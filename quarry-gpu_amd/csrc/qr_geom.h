@@ -336,23 +336,15 @@ QR_HD TriClosest closestOnTri(V3 p, const Tri& tri) {
     return {distTo(p, q), b1, b2, kRegionFace};
 }
 
-// distanceSquaredToAABB (geometry.h:262-277).
+// distanceSquaredToAABB (geometry.h:262-277), without its branches: at most one of
+// lo - v and v - hi is positive in a box with lo <= hi (and both are infinite in an
+// empty one), and adding a zero square leaves the sum's bits alone.  A NaN coordinate
+// adds nothing, as in the branches.
 QR_HD float boxDist2(V3 p, const Box& box) {
-    float d2 = 0.0f;
-#pragma unroll
-    for (int axis = 0; axis < 3; ++axis) {
-        const float v = comp(p, axis);
-        const float lo = comp(box.lo, axis);
-        const float hi = comp(box.hi, axis);
-        if (v < lo) {
-            const float d = lo - v;
-            d2 += d * d;
-        } else if (v > hi) {
-            const float d = v - hi;
-            d2 += d * d;
-        }
-    }
-    return d2;
+    const float dx = fmaxf(fmaxf(box.lo.x - p.x, p.x - box.hi.x), 0.0f);
+    const float dy = fmaxf(fmaxf(box.lo.y - p.y, p.y - box.hi.y), 0.0f);
+    const float dz = fmaxf(fmaxf(box.lo.z - p.z, p.z - box.hi.z), 0.0f);
+    return dx * dx + dy * dy + dz * dz;
 }
 
 // ---- Gaussians as solid ellipsoids (src/core/gaussian.h:23-131) ----------------

@@ -490,6 +490,17 @@ __host__ __device__ __forceinline__ int stackIdBitsDev(int idCount) {
     return bits <= 23 ? bits : 32;
 }
 
+// The same by mask (the low idBits bits; all 32 when there is no key): the float's bits,
+// shifted up over the sign, above the id.
+__host__ __device__ __forceinline__ uint32_t stackIdMask(int idCount) {
+    const int bits = stackIdBitsDev(idCount);
+    return bits >= 32 ? ~0u : (1u << bits) - 1u;
+}
+__device__ __forceinline__ uint32_t stackEntry(uint32_t id, uint32_t keyBits, uint32_t idMask) {
+    return ((keyBits << 1) & ~idMask) | id;
+}
+__device__ __forceinline__ uint32_t stackKey(uint32_t v, uint32_t idMask) { return (v & ~idMask) >> 1; }
+
 __device__ __forceinline__ int packEntry(int id, float key, int idBits) {
     if (idBits >= 32) return id;
     const uint32_t q = floatBits(key) >> (idBits - 1);
@@ -1103,21 +1114,6 @@ __device__ __forceinline__ void waveSortPairs(float& k, int& v, int lane, int wi
     }
 }
 
-// Bitonic merge of a bitonic sequence (one pair per lane, aligned groups of `width`
-// lanes) into ascending order.
-__device__ __forceinline__ void waveMergePairs(float& k, int& v, int lane, int width = 64) {
-    for (int stride = width >> 1; stride > 0; stride >>= 1) {
-        const float ok = waveXor(k, stride);
-        const int ov = waveXor(v, stride);
-        const bool low = (lane & stride) == 0;
-        const bool otherFirst = closer(ok, ov, k, v);
-        if (low == otherFirst) {
-            k = ok;
-            v = ov;
-        }
-    }
-}
-
 // Radius capture with one wave per query, for query sets too small to fill the
 // device four lanes per query.  The wave's 16 quads expand up to 16 nodes of the
 // query's walk per round (quad j takes the j-th entry from the top of a stack shared
@@ -1131,7 +1127,6 @@ __device__ __forceinline__ void waveMergePairs(float& k, int& v, int lane, int w
 // (the quad kernels' stack assumes the same depth).
 constexpr int kWaveStack = 1024;
 constexpr int kWaveHeadroom = 3 * 32 + 4;
-constexpr int kInsertMax = 16;  // a round's candidates inserted one by one up to this many (measured: 4 -> 0.473 ms, 16 -> 0.425, 64 -> 0.422 for C2 kNN16; the sort and merge 0.493)
 
 // Bitonic sort by (dist2, index) of up to 64 pairs held two per lane by a group of
 // 32 lanes (lane l holds elements l and l + 32; empty elements are (inf, INT_MAX)).
@@ -1283,225 +1278,298 @@ __global__ __launch_bounds__(kBlock) void radiusWaveKernel(
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
 }
 
-// Closest / kNN with one wave per query (the radius capture's layout: 16 quads expand
-// up to 16 nodes of one walk per round from a shared LDS stack, lane s of a quad
-// tests entry s).  The k-best list is spread one entry per lane (lanes 0..K-1,
-// sorted by (dist2, index), (inf, INT_MAX) when empty); a round's leaf candidates
-// that beat the list's K-th are sorted across the wave (bitonic network) and merged
-// in (the elementwise smaller of the list and the reversed candidates holds the K
-// best, a bitonic merge sorts it).  Interior children are pushed nearest-parent
-// first and, within a parent, nearest on top, so the next round expands about the
-// nearest 16 without a sort (for Gaussians: sorted by box distance across the wave).  The admission rule is the lane kernels' (n < K or
-// bound <= K-th), so the list ends as the K best by (dist2, index) whatever the
+// ---- steps of a group of G lanes (16, 32 or 64, aligned within the wave) ----------------
+// A group works on one query; the groups of a wave run the same instructions, so the
+// steps below keep to vector operations and wave-uniform branches.
+
+// The group's own bits of a ballot.  G <= 32: the half-wave word, masked to the group
+// and left in place (32-bit counts and shifts instead of 64-bit ones); G = 64: all.
+template <int G>
+struct GroupBits {
+    using Word = uint32_t;
+    Word mask;       // the group's lanes
+    Word lower;      // those below this lane
+    Word lowerQuad;  // those in lower quads than this lane's
+    bool high;       // the group lies in lanes 32..63
+    int base;        // lane of bit 0
+    __device__ __forceinline__ void init(int lane) {
+        const int at = lane & 31;
+        high = lane >= 32;
+        base = lane & 32;
+        mask = G == 32 ? ~0u : ((1u << (G & 31)) - 1u) << (at & ~(G - 1));
+        lower = mask & ((1u << at) - 1u);
+        lowerQuad = mask & ((1u << (at & ~3)) - 1u);
+    }
+    __device__ __forceinline__ Word of(unsigned long long ballot) const {
+        return (high ? static_cast<uint32_t>(ballot >> 32) : static_cast<uint32_t>(ballot)) & mask;
+    }
+    __device__ __forceinline__ static int count(Word w) { return __popc(w); }
+    __device__ __forceinline__ static int first(Word w) { return __ffs(static_cast<int>(w)) - 1; }
+};
+template <>
+struct GroupBits<64> {
+    using Word = unsigned long long;
+    Word lower, lowerQuad;
+    static constexpr int base = 0;
+    __device__ __forceinline__ void init(int lane) {
+        lower = (1ull << lane) - 1ull;
+        lowerQuad = (1ull << (lane & ~3)) - 1ull;
+    }
+    __device__ __forceinline__ Word of(unsigned long long ballot) const { return ballot; }
+    __device__ __forceinline__ static int count(Word w) { return __popcll(w); }
+    __device__ __forceinline__ static int first(Word w) { return __ffsll(static_cast<long long>(w)) - 1; }
+};
+
+__device__ __forceinline__ uint32_t minU(uint32_t a, uint32_t b) { return a < b ? a : b; }
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dppU(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(x), kCtrl, 0xF, 0xF, true));
+}
+// Smallest x over the group, in every lane: within rows of 16 by DPP (one instruction a
+// step, no LDS permute), across rows by the row and half swaps.
+template <int G>
+__device__ __forceinline__ uint32_t groupMin(uint32_t x) {
+    x = minU(x, dppU<0xB1>(x));   // quad_perm [1,0,3,2]
+    x = minU(x, dppU<0x4E>(x));   // quad_perm [2,3,0,1]
+    x = minU(x, dppU<0x141>(x));  // row_half_mirror
+    x = minU(x, dppU<0x140>(x));  // row_mirror
+    if constexpr (G >= 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+        x = minU(r[0], r[1]);
+    }
+    if constexpr (G == 64) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+        x = minU(r[0], r[1]);
+    }
+    return x;
+}
+// The group's lane i receives lane i - 1's x, its first lane 0.
+template <int G>
+__device__ __forceinline__ uint32_t groupShiftUp(uint32_t x, int gl) {
+    if constexpr (G == 16) {
+        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x111, 0xF, 0xF, false));
+    } else {
+        const int v = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xF, 0xF, false);
+        return static_cast<uint32_t>(G == 32 && gl == 0 ? 0 : v);
+    }
+}
+__device__ __forceinline__ uint32_t permuteU(int lane, uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(lane << 2, static_cast<int>(x)));
+}
+
+// A (dist2, index) pair as one ordered integer: dist2 is non-negative, so its bits order
+// as it does, and equal distances order by index.  (inf, INT_MAX) is an empty place; a
+// NaN distance lies behind it and is never taken.
+constexpr uint32_t kInfBits = 0x7f800000u;
+constexpr uint32_t kNoPrim = 0x7fffffffu;
+__device__ __forceinline__ unsigned long long pairKey(uint32_t d, uint32_t id) {
+    return (static_cast<unsigned long long>(d) << 32) | id;
+}
+
+// Rank of a lane's child among its quad's four by box distance (no child: rank 3, or
+// what is left).  The slot takes the key's two low bits, so no two keys are equal; the
+// order only steers the walk.
+__device__ __forceinline__ int quadRank(bool child, uint32_t dBits, int slot) {
+    const uint32_t key = child ? (dBits & ~3u) | static_cast<uint32_t>(slot) : 0xfffffffcu | static_cast<uint32_t>(slot);
+    int rank = dppU<0xB1>(key) < key ? 1 : 0;
+    rank += dppU<0x4E>(key) < key ? 1 : 0;
+    rank += dppU<0x1B>(key) < key ? 1 : 0;  // quad_perm [3,2,1,0]
+    return rank;
+}
+
+// Entry `slot` of 4-wide node `id`: its box and child code (>= 0 a node, < 0 a leaf
+// reference -(leaf slot + 1), kWideEmpty nothing).
+struct WideNodes {
+    const Wide4* __restrict__ wide;
+    __device__ __forceinline__ int entry(int id, int slot, Box& box) const {
+        const WideEntry e = wide[id].c[slot];
+        box = entryBox(e);
+        return e.child;
+    }
+};
+
+// Closest / kNN walk of one query by a group of G lanes.  The group's quads expand up to
+// G / 4 nodes of the walk per round from a stack in LDS, lane s of a quad testing entry s
+// of its node.  The k-best list is spread one entry per lane, sorted by (dist2, index)
+// (the group's lanes beyond K keep the entries that fell off the K best: they cost
+// nothing and are never read).  A round's leaf candidates closer than the K-th go in one
+// by one: each is broadcast to its group, and the entries behind its place move up one
+// lane (a DPP shift; no ballot or place count).  K = 1: the group's smallest candidate
+// by DPP.  Interior children are pushed nearest parent first and, within a parent,
+// nearest on top; for Gaussians, whose leaf test costs the most, in box-distance order
+// over the whole group.  A subtree or primitive is passed over only when its bound lies
+// beyond the K-th distance, so the list ends as the K best by (dist2, index) whatever the
 // walk order.
+//
+// Bound by VALU issue: the round is kept to as few instructions as possible.  The K-th
+// key stands for the list's fill (an empty list's is infinite), masks and counts are
+// 32-bit words of the group, the box test has no branches, reductions and shifts are DPP,
+// and a leaf's primitive is loaded once its box is admitted (a quarter of them are).
+// Against 64-bit masks, LDS permutes and short-circuit tests, kernel time on a
+// 2M-triangle terrain with 100k queries: closest 277 -> 205 us, kNN16 443 -> 308 us; one
+// path through all regions of the triangle distance instead of its exits: no faster here,
+// 15 % slower around an icosphere (1.01 -> 1.16 ms).
+template <typename L, int K, int G, bool kStats, typename Nodes>
+struct GroupNearest {
+    static_assert(G == 16 || G == 32 || G == 64, "lanes per query");
+    static_assert(K <= G, "the k-best list takes one lane per entry");
+    static constexpr bool kSortPushes = L::kKind == 2;
+    static constexpr int kQuads = G / 4;                 // nodes a query expands per round
+    static constexpr int kStack = kWaveStack / (64 / G);  // stack entries per query
+    uint32_t ld, lid;  // this lane's list entry (K = 1: the best, in every lane)
+    uint32_t kd, kid;  // the list's K-th (the same in every lane)
+
+    __device__ __forceinline__ void walk(const Nodes& nodes, const typename L::Item* __restrict__ prims,
+                                         const int* __restrict__ primIds, V3 p, LdsInt* stk, int lane,
+                                         uint32_t idMask, int& nodeTests, int& leafTests, int& overflow,
+                                         int& opened) {
+        const int gl = lane & (G - 1);  // lane within the group
+        const int quad = gl >> 2;
+        const int slot = lane & 3;
+        GroupBits<G> gb;
+        gb.init(lane);
+        ld = kd = kInfBits;
+        lid = kid = kNoPrim;
+        if (gl == 0) stk[0] = 0;
+        int sp = 1;
+        while (sp > 0) {
+            int take = takeOf(sp);
+            int node = -1;
+            bool cut = false;
+            if (quad < take) {
+                const uint32_t v = static_cast<uint32_t>(stk[sp - 1 - quad]);
+                cut = stackKey(v, idMask) > kd;
+                node = cut ? -1 : static_cast<int>(v & idMask);
+            }
+            const unsigned long long cuts = __ballot(cut);
+            if (cuts != 0 && gb.of(cuts) != 0) {
+                // the bound has overtaken entries the quads would take: drop those of
+                // the top G (order kept) and take again, so no quad idles on them
+                const int look = sp < G ? sp : G;
+                uint32_t v = 0;
+                bool keep = false;
+                if (gl < look) {
+                    v = static_cast<uint32_t>(stk[sp - look + gl]);
+                    keep = stackKey(v, idMask) <= kd;
+                }
+                const typename GroupBits<G>::Word kept = gb.of(__ballot(keep));
+                if (keep) stk[sp - look + gb.count(kept & gb.lower)] = static_cast<int>(v);
+                sp = sp - look + gb.count(kept);
+                take = takeOf(sp);
+                node = -1;
+                if (quad < take) node = static_cast<int>(static_cast<uint32_t>(stk[sp - 1 - quad]) & idMask);
+            }
+            sp -= take;
+            if (kStats && slot == 0 && node >= 0) ++opened;
+            Box box{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+            int ch = kWideEmpty;
+            if (node >= 0) ch = nodes.entry(node, slot, box);
+            const bool leaf = static_cast<uint32_t>(ch) > static_cast<uint32_t>(kWideEmpty);
+            const uint32_t d = floatBits(boxDist2(p, box));
+            const bool adm = (ch != kWideEmpty) & (d <= kd);
+            if (kStats && adm) ++nodeTests;
+            uint32_t cd = ~0u, cid = ~0u;
+            bool better = false;
+            if (adm & leaf) {
+                if (kStats) ++leafTests;
+                const uint32_t pid = static_cast<uint32_t>(primIds[-ch - 1]);
+                const uint32_t dd = floatBits(L::dist2(p, prims[-ch - 1]));
+                better = pairKey(dd, pid) < pairKey(kd, kid);
+                cd = better ? dd : ~0u;
+                cid = better ? pid : ~0u;
+            }
+            const unsigned long long bm = __ballot(better);
+            if (bm != 0) {
+                if constexpr (K == 1) {
+                    const uint32_t m = groupMin<G>(cd);
+                    const uint32_t mi = groupMin<G>(cd == m ? cid : ~0u);
+                    const bool got = m != ~0u;  // (a candidate is closer than the entry)
+                    kd = got ? m : kd;
+                    kid = got ? mi : kid;
+                } else {
+                    insertAll(gb, gb.of(bm), cd, cid, lane, gl);
+                }
+            }
+            // interior children that survive the updated bound: quad j popped the j-th
+            // nearest entry, so its children go above those of quads j+1..
+            const bool push = adm & !leaf & (d <= kd);
+            const unsigned long long pb = __ballot(push);
+            if (pb != 0) {
+                const typename GroupBits<G>::Word pm = gb.of(pb);
+                const int pushes = gb.count(pm);
+                const int top = sp + pushes;
+                if (top > kStack) {  // deeper than the stack bound allows
+                    if (gl == 0) overflow = 1;
+                    sp = 0;
+                } else {
+                    if constexpr (kSortPushes) {  // all of the round's children in box-distance order
+                        float pk = push ? bitsFloat(d) : kInf;
+                        int pv = push ? ch : 0x7fffffff;
+                        waveSortPairs(pk, pv, lane, G);
+                        if (gl < pushes) stk[top - 1 - gl] = static_cast<int>(stackEntry(static_cast<uint32_t>(pv), floatBits(pk), idMask));
+                    } else {
+                        const int rank = quadRank(push, d, slot);
+                        if (push) stk[top - 1 - gb.count(pm & gb.lowerQuad) - rank] = static_cast<int>(stackEntry(static_cast<uint32_t>(ch), d, idMask));
+                    }
+                    sp = top;
+                }
+            }
+        }
+    }
+
+    // Nodes to take from a stack of sp entries: one per quad, fewer when the stack could
+    // otherwise outgrow its room (see kWaveStack).
+    __device__ __forceinline__ static int takeOf(int sp) {
+        const int room = kStack - kWaveHeadroom - sp;
+        int width = kQuads;
+        if (room < 3 * kQuads) width = room < 3 ? 1 : room / 3;
+        return width < sp ? width : sp;
+    }
+
+    __device__ __forceinline__ void insertAll(const GroupBits<G>& gb, typename GroupBits<G>::Word rest, uint32_t cd,
+                                              uint32_t cid, int lane, int gl) {
+        while (__ballot(rest != 0) != 0) {
+            // a group that has none left broadcasts the key behind all others
+            const int src = rest != 0 ? gb.base + gb.first(rest) : lane;
+            uint32_t c = permuteU(src, cd), ci = permuteU(src, cid);
+            c = rest != 0 ? c : ~0u;
+            rest &= rest - 1;
+            const unsigned long long ck = pairKey(c, ci);
+            const uint32_t pd = groupShiftUp<G>(ld, gl), pi = groupShiftUp<G>(lid, gl);
+            const bool stays = pairKey(ld, lid) < ck;
+            const bool here = pairKey(pd, pi) < ck;  // the entry below is closer: the candidate's place
+            const uint32_t nd = here ? c : pd, ni = here ? ci : pi;
+            ld = stays ? ld : nd;
+            lid = stays ? lid : ni;
+        }
+        const int last = (lane & ~(G - 1)) + K - 1;
+        kd = permuteU(last, ld);
+        kid = permuteU(last, lid);
+    }
+
+    __device__ __forceinline__ void store(ClosestResult* __restrict__ dst, int k, int gl) const {
+        const uint32_t d = K == 1 ? kd : ld, i = K == 1 ? kid : lid;
+        if (gl < k) dst[gl] = i == kNoPrim ? ClosestResult{0u, -1} : ClosestResult{d, static_cast<int>(i)};
+    }
+};
+
+// The walk over a plain 4-wide tree: 64 / G queries per wave.
 template <typename L, int K, int G, bool kStats>
 __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
     const Wide4* __restrict__ wide, const typename L::Item* __restrict__ prims,
     const int* __restrict__ primIds, const V3* __restrict__ points, const uint32_t* __restrict__ order,
     int count, int k, int outStride, ClosestResult* __restrict__ out, unsigned long long* __restrict__ stats,
-    int idBits) {
-    // Gaussian leaves cost the most to test, so their walks pay for a sorted push
-    // order (fewer nodes opened); triangles and points push quad by quad.
-    constexpr bool kSortPushes = L::kKind == 2;
-    static_assert(G == 16 || G == 32 || G == 64, "lanes per query");
-    static_assert(K <= G, "the k-best list takes one lane per entry");
-    constexpr int kPerWave = 64 / G;              // queries per wave
-    constexpr int kQuads = G / 4;                 // nodes a query expands per round
-    constexpr int kStack = kWaveStack / kPerWave;  // stack entries per query
+    uint32_t idMask) {
     __shared__ int lds[kWaveStack * (kBlock / 64)];
-    __shared__ int ldsCmp[2 * 64 * (kBlock / 64)];  // per wave: candidate keys, values
     const int lane = threadIdx.x & 63;
-    const int gl = lane & (G - 1);   // lane within the query's group
-    const int gb = lane - gl;        // the group's first lane
-    const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1ull) << gb;
-    LdsInt* cmpK = (LdsInt*)(ldsCmp + (threadIdx.x >> 6) * 128) + gb;
-    LdsInt* cmpV = cmpK + 64;
-    const int quad = gl >> 2;
-    const int slot = lane & 3;
-    const int qi = (xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6)) * kPerWave + lane / G;
-    const unsigned long long below = ((1ull << lane) - 1ull) & gmask;
+    const int qi = (xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6)) * (64 / G) + lane / G;
     int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
     if (qi < count) {  // the same in the whole group
         const int q = order ? static_cast<int>(order[qi]) : qi;
-        const V3 p = points[q];
-        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * kStack);
-        float ld = kInf;  // this lane's list entry (group lanes 0..K-1)
-        int lid = 0x7fffffff;
-        float kd = kInf;  // the list's K-th (the same in every lane)
-        int kid = 0x7fffffff;
-        int n = 0;
-        auto admits = [&](float lb) { return n < K || lb <= kd; };
-        if (gl == 0) stk[0] = packEntry(0, 0.0f, idBits);
-        int sp = 1;
-        while (sp > 0) {
-            int width = (kStack - kWaveHeadroom - sp) / 3;
-            width = width < 1 ? 1 : (width > kQuads ? kQuads : width);
-            int take = width < sp ? width : sp;
-            int node = -1;
-            if (quad < take) {
-                const int v = stk[sp - 1 - quad];
-                if (admits(entryKey(v, idBits))) node = entryId(v, idBits);
-            }
-            if ((__ballot(quad < take && node < 0) & gmask) != 0) {
-                // the bound has overtaken entries the quads would take: drop those of
-                // the top G (order kept) and take again, so no quad idles on them
-                const int look = sp < G ? sp : G;
-                int v = 0;
-                bool keep = false;
-                if (gl < look) {
-                    v = stk[sp - look + gl];
-                    keep = admits(entryKey(v, idBits));
-                }
-                const unsigned long long km = __ballot(keep) & gmask;
-                if (keep) stk[sp - look + __popcll(km & below)] = v;
-                sp = sp - look + __popcll(km);
-                if (sp == 0) break;
-                width = (kStack - kWaveHeadroom - sp) / 3;
-                width = width < 1 ? 1 : (width > kQuads ? kQuads : width);
-                take = width < sp ? width : sp;
-                node = quad < take ? entryId(stk[sp - 1 - quad], idBits) : -1;
-            }
-            sp -= take;
-            if (kStats && slot == 0 && node >= 0) ++opened;
-            WideEntry e{};
-            int ch = kWideEmpty;
-            if (node >= 0) {
-                e = wide[node].c[slot];
-                ch = e.child;
-            }
-            const bool leaf = ch < 0 && ch != kWideEmpty;
-            typename L::Item it;
-            int pid = 0;
-            if (leaf) {
-                it = prims[-ch - 1];
-                pid = primIds[-ch - 1];
-            }
-            float d = kInf;
-            bool adm = false;
-            if (ch != kWideEmpty) {
-                d = boxDist2(p, entryBox(e));
-                adm = admits(d);
-            }
-            if (adm) ++nodeTests;
-            float cd = kInf;
-            int cid = 0x7fffffff;
-            bool better = false;
-            if (adm && leaf) {
-                ++leafTests;
-                cd = L::dist2(p, it);
-                cid = pid;
-                better = n < K || closer(cd, cid, kd, kid);
-            }
-            const unsigned long long bm = __ballot(better) & gmask;
-            if (K == 1 && bm != 0) {  // the group's smallest candidate replaces the entry
-                float ck = better ? cd : kInf;
-                int cv = better ? cid : 0x7fffffff;
-#pragma unroll
-                for (int off = G / 2; off > 0; off >>= 1) {
-                    const float ok = waveXor(ck, off);
-                    const int ov = waveXor(cv, off);
-                    if (closer(ok, ov, ck, cv)) {
-                        ck = ok;
-                        cv = ov;
-                    }
-                }
-                kd = ck;
-                kid = cv;
-                ld = gl == 0 ? ck : kInf;
-                lid = gl == 0 ? cv : 0x7fffffff;
-                n = 1;
-            } else if (bm != 0 && __popcll(bm) <= kInsertMax) {
-                // a few candidates: each in turn is broadcast to the group, finds its
-                // place by one ballot (the list entries closer than it) and the entries
-                // from there shift up one lane -- the same K best by (dist2, index)
-                // as the sort and merge below, for far fewer instructions
-                unsigned long long rest = bm;
-                const int nb = __popcll(bm);
-                for (int i = 0; i < nb; ++i) {
-                    const int src = __ffsll(static_cast<long long>(rest)) - 1;
-                    rest &= rest - 1ull;
-                    const float c = __shfl(cd, src, 64);
-                    const int ci = __shfl(cid, src, 64);
-                    const int pos = __popcll(__ballot(gl < K && closer(ld, lid, c, ci)) & gmask);
-                    const float pk = __shfl(ld, lane - 1, 64);
-                    const int pv = __shfl(lid, lane - 1, 64);
-                    if (gl < K && gl >= pos) {
-                        ld = gl == pos ? c : pk;
-                        lid = gl == pos ? ci : pv;
-                    }
-                }
-                n = n + nb;
-                n = n < K ? n : K;
-                kd = __shfl(ld, gb + K - 1, 64);
-                kid = __shfl(lid, gb + K - 1, 64);
-            } else if (bm != 0) {
-                // the nb candidates move to lanes 0..nb-1 (through LDS), are sorted
-                // over the smallest power-of-two width m >= max(nb, K), and merged:
-                // the list (lanes >= K hold (inf, INT_MAX)) against the reversed
-                // candidates, elementwise, is a bitonic sequence holding the K best
-                const int nb = __popcll(bm);
-                int m = K;
-                while (m < nb) m <<= 1;
-                if (better) {
-                    const int at = __popcll(bm & below);
-                    cmpK[at] = __float_as_int(cd);
-                    cmpV[at] = cid;
-                }
-                float ck = gl < nb ? __int_as_float(cmpK[gl]) : kInf;
-                int cv = gl < nb ? cmpV[gl] : 0x7fffffff;
-                waveSortPairs(ck, cv, lane, m);
-                const float rk = __shfl(ck, gb + m - 1 - (gl & (m - 1)), 64);
-                const int rv = __shfl(cv, gb + m - 1 - (gl & (m - 1)), 64);
-                float mk = ld;
-                int mv = lid;
-                if (gl < m && closer(rk, rv, mk, mv)) {
-                    mk = rk;
-                    mv = rv;
-                }
-                waveMergePairs(mk, mv, lane, m);
-                ld = gl < K ? mk : kInf;
-                lid = gl < K ? mv : 0x7fffffff;
-                n = n + __popcll(bm);
-                n = n < K ? n : K;
-                kd = __shfl(ld, gb + K - 1, 64);
-                kid = __shfl(lid, gb + K - 1, 64);
-            }
-            // interior children that survive the updated bound: quad j popped the j-th
-            // nearest entry, so its children go above those of quads j+1.., each
-            // quad's nearest child on top of its group
-            const bool push = adm && !leaf && admits(d);
-            const unsigned long long pm = __ballot(push) & gmask;
-            const int pushes = __popcll(pm);
-            if (pushes > 0) {
-                if (sp + pushes > kStack) {  // deeper than the stack bound allows
-                    if (gl == 0) overflow = 1;
-                    break;
-                }
-                if (kSortPushes) {  // all of the round's children in box-distance order
-                    float pk = push ? d : kInf;
-                    int pv = push ? ch : 0x7fffffff;
-                    waveSortPairs(pk, pv, lane, G);
-                    if (gl < pushes) stk[sp + pushes - 1 - gl] = packEntry(pv, pk, idBits);
-                } else {
-                    const float key = push ? d : kInf;
-                    const float k0 = quadGetF<0>(key), k1 = quadGetF<1>(key), k2 = quadGetF<2>(key), k3 = quadGetF<3>(key);
-                    int rank = 0;
-                    rank += (slot != 0) && (k0 < key || (k0 == key && 0 < slot));
-                    rank += (slot != 1) && (k1 < key || (k1 == key && 1 < slot));
-                    rank += (slot != 2) && (k2 < key || (k2 == key && 2 < slot));
-                    rank += (slot != 3) && (k3 < key || (k3 == key && 3 < slot));
-                    const int mine = __popcll((pm >> (gb + 4 * quad)) & 0xFull);
-                    const int deeper = quad < kQuads - 1 ? __popcll(pm >> (gb + 4 * (quad + 1))) : 0;
-                    if (push) stk[sp + deeper + (mine - 1 - rank)] = packEntry(ch, d, idBits);
-                }
-                sp += pushes;
-            }
-        }
-        if (gl < k) {
-            ClosestResult r{0u, -1};
-            if (gl < n) r = {floatBits(ld), lid};
-            out[static_cast<size_t>(q) * outStride + gl] = r;
-        }
+        GroupNearest<L, K, G, kStats, WideNodes> g;
+        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * g.kStack);
+        g.walk(WideNodes{wide}, prims, primIds, points[q], stk, lane, idMask, nodeTests, leafTests, overflow, opened);
+        g.store(out + static_cast<size_t>(q) * outStride, k, lane & (G - 1));
     }
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
 }
@@ -2145,12 +2213,12 @@ template <typename L, int K, int G>
 static void launchGroup(const TraverseArgs& a, const V3* pts, int count, int k, int outStride, ClosestResult* out,
                         unsigned long long* stats, hipStream_t s) {
     const auto* prims = static_cast<const typename L::Item*>(a.items);
-    const int idBits = stackIdBitsDev(a.wideCount);
+    const uint32_t idMask = stackIdMask(a.wideCount);
     const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
     if (stats)
-        nearestWaveKernel<L, K, G, true><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idBits);
+        nearestWaveKernel<L, K, G, true><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idMask);
     else
-        nearestWaveKernel<L, K, G, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idBits);
+        nearestWaveKernel<L, K, G, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idMask);
 }
 
 template <typename L, int K>

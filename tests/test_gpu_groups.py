@@ -1,0 +1,66 @@
+"""The walks that give a query a group of lanes, at the sizes where a group, a wave or the
+k-best list is only partly filled; results against the brute-force oracle, bit for bit."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import A, eq, random_gaussians, random_tris  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+
+def scene(kind, n, seed):
+    rng = np.random.default_rng(seed)
+    if kind == 0:
+        return random_tris(rng, n)
+    if kind == 1:
+        p = rng.uniform(-30, 30, (n, 3)).astype(np.float32)
+        p[n // 2:] = p[: n - n // 2]  # equal distances: ordered by index
+        return p
+    return random_gaussians(rng, n)
+
+
+@pytest.mark.parametrize("mode", [3, 5, 6])  # 64, 16 and 32 lanes per query
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_group_walk_edges(A, orc, kind, mode):  # noqa: F811
+    A.lib().qr_set_traversal_mode(mode)
+    try:
+        # (primitives, queries, k): fewer primitives than k, one query, the last group of a
+        # wave and the last wave of a workgroup partly filled, every capacity of the list
+        for n, nq, k in ((2, 1, 1), (5, 3, 32), (17, 5, 16), (300, 63, 2), (1000, 65, 4), (1000, 17, 5),
+                         (3000, 129, 8), (3000, 250, 15), (3000, 33, 17), (3000, 7, 32)):
+            print(f"kind={kind} mode={mode} n={n} nq={nq} k={k}", flush=True)
+            items = scene(kind, n, n + nq)
+            q = np.random.default_rng(k).uniform(-40, 40, (nq, 3)).astype(np.float32)
+            b = A.Bvh(kind, items)
+            b.build_wide()
+            want = orc.knn_brute(kind, items, q, k, threads=8)
+            assert eq(b.knn(q, k, order=A.ORDER_MORTON, wide=True)[0], want), (n, nq, k)
+            want = orc.knn_brute(kind, items, q, 0, threads=8)
+            assert eq(b.closest(q, order=A.ORDER_INPUT, wide=True)[0], want), (n, nq)
+    finally:
+        A.lib().qr_set_traversal_mode(0)
+
+
+@pytest.mark.parametrize("mode", [3, 5, 6])
+def test_group_walk_unusual_queries(A, orc, mode):  # noqa: F811
+    """NaN queries have no answer (index -1) and leave the others of their wave alone;
+    infinite ones are infinitely far from everything: the lowest indices."""
+    items = scene(1, 500, 3)
+    q = np.random.default_rng(4).uniform(-40, 40, (40, 3)).astype(np.float32)
+    bad, far = [3, 17, 18], [5, 30]
+    q[bad, 1] = np.nan
+    q[far, 0] = np.inf
+    rest = np.setdiff1d(np.arange(40), bad + far)
+    b = A.Bvh(1, items)
+    b.build_wide()
+    A.lib().qr_set_traversal_mode(mode)
+    try:
+        for k in (0, 4):
+            got = b.knn(q, k, order=A.ORDER_INPUT, wide=True)[0] if k else b.closest(q, order=A.ORDER_INPUT, wide=True)[0]
+            want = orc.knn_brute(1, items, q[rest], k, threads=8)
+            assert eq(got[rest], want)
+            assert np.all(got[bad, :, 1].view(np.int32) == -1)
+            assert np.all(got[far, :, 0].view(np.float32) == np.inf)
+            assert eq(got[far, :, 1], np.tile(np.arange(max(k, 1), dtype=np.uint32), (len(far), 1)))
+    finally:
+        A.lib().qr_set_traversal_mode(0)
