@@ -99,8 +99,8 @@ QR_API int qr_describe(char* buf, int len);
 QR_API int qr_warmup(void);
 /* Shape of the 4-wide traversal, process-wide: 0 automatic (closest / kNN below
  * 65,536 queries by query count, leaf kind and k; from 65,536 on, the first call
- * for a tree, k class and query-count octave times one lane, four lanes, 16 and 32
- * lanes and one wave per query on its own queries and keeps the fastest; radius 32
+ * for a tree, k class and query-count octave times 16 and 32 lanes and one wave per
+ * query on its own queries and keeps the fastest; radius 32
  * lanes per query (two queries per wave) below 131,072 queries, four lanes above;
  * rays one lane per ray), 1 one lane per query, 2 four lanes per query, 3 one wave
  * per query or ray, 4 as 0 but closest / kNN and rays tuned at every count, 5 / 6
@@ -292,7 +292,8 @@ QR_API int qr_batch_tree_hash(const qr_batch* b, int scene, uint64_t* out);
  * 1..32: kNN.  Kernel variants v: 0..3 walk the binary nodes, 4..7 the 4-wide nodes
  * (collapsed for every scene on first use), each with the traversal stack in LDS with
  * 256 or 64 lanes per workgroup (v % 4 = 0, 1), in scratch (2), or its top 8 entries in
- * registers (3).  tune = 1 times every variant with and without per-scene Morton order
+ * registers (3).  Variants 4 and 5 give each query a group of 16 to 64 lanes, the others
+ * one lane.  tune = 1 times every variant with and without per-scene Morton order
  * and keeps the fastest; tune = 0 takes variant 0 with Morton order; tune = 2 + 2 v + m
  * forces variant v with Morton order m.  The chosen pipeline is captured in a hipGraph.
  * The points must stay valid while the plan lives. */

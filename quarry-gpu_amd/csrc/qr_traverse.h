@@ -101,8 +101,8 @@ struct BatchQueryArgs {
     int* counter = nullptr;         // work-queue head (reset before each launch)
 };
 // Variants the autotuner chooses from: binary or 4-wide nodes; the stack in LDS
-// (256- or 64-lane workgroups, spilling to scratch), in scratch, or its top entries in
-// registers.
+// (256- or 64-lane workgroups; binary: one lane per query, spilling to scratch; 4-wide:
+// a group of lanes per query), in scratch, or its top entries in registers.
 enum BatchVariant : int {
     kBatchLds256 = 0, kBatchLds64 = 1, kBatchScratch64 = 2, kBatchReg64 = 3,
     kBatchWideLds256 = 4, kBatchWideLds64 = 5, kBatchWideScratch64 = 6, kBatchWideReg64 = 7,

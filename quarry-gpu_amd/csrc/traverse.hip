@@ -493,8 +493,8 @@ __host__ __device__ __forceinline__ int stackIdBitsDev(int idCount) {
 // The same by mask (the low idBits bits; all 32 when there is no key): the float's bits,
 // shifted up over the sign, above the id.
 __host__ __device__ __forceinline__ uint32_t stackIdMask(int idCount) {
-    const int bits = stackIdBitsDev(idCount);
-    return bits >= 32 ? ~0u : (1u << bits) - 1u;
+    const int bits = idCount <= 2 ? 1 : 32 - __builtin_clz(static_cast<unsigned>(idCount - 1));
+    return bits > 23 ? ~0u : (1u << bits) - 1u;
 }
 __device__ __forceinline__ uint32_t stackEntry(uint32_t id, uint32_t keyBits, uint32_t idMask) {
     return ((keyBits << 1) & ~idMask) | id;
@@ -601,6 +601,7 @@ __global__ __launch_bounds__(kBlock) void nearestBinaryKernel(
 }
 
 // ---- batched scenes: persistent work-queue traversal ------------------------------------
+// (The 4-wide variants with the stack in LDS are batchGroupKernel below.)
 // Queries of all scenes form one queue (scene-major, optionally Morton-ordered inside
 // each scene).  Each wave takes the next 64 queries with one atomic and walks, per
 // lane, the tree of that query's scene (scene s: items from primOff[s]; binary nodes
@@ -1390,18 +1391,18 @@ struct WideNodes {
 
 // Closest / kNN walk of one query by a group of G lanes.  The group's quads expand up to
 // G / 4 nodes of the walk per round from a stack in LDS, lane s of a quad testing entry s
-// of its node.  The k-best list is spread one entry per lane, sorted by (dist2, index)
-// (the group's lanes beyond K keep the entries that fell off the K best: they cost
-// nothing and are never read).  A round's leaf candidates closer than the K-th go in one
-// by one: each is broadcast to its group, and the entries behind its place move up one
-// lane (a DPP shift; no ballot or place count).  K = 1: the group's smallest candidate
-// by DPP.  Interior children are pushed nearest parent first and, within a parent,
+// of its node.  The k-best list is spread one entry per lane, sorted by (dist2, index),
+// for any k up to G (the group's lanes beyond k keep the entries that fell off the k
+// best: they cost nothing and are never read).  A round's leaf candidates closer than the
+// k-th go in one by one: each is broadcast to its group, and the entries behind its place
+// move up one lane (a DPP shift; no ballot or place count).  kOne (k = 1): the group's
+// smallest candidate by DPP.  Interior children are pushed nearest parent first and, within a parent,
 // nearest on top; for Gaussians, whose leaf test costs the most, in box-distance order
 // over the whole group.  A subtree or primitive is passed over only when its bound lies
-// beyond the K-th distance, so the list ends as the K best by (dist2, index) whatever the
+// beyond the k-th distance, so the list ends as the k best by (dist2, index) whatever the
 // walk order.
 //
-// Bound by VALU issue: the round is kept to as few instructions as possible.  The K-th
+// Bound by VALU issue: the round is kept to as few instructions as possible.  The k-th
 // key stands for the list's fill (an empty list's is infinite), masks and counts are
 // 32-bit words of the group, the box test has no branches, reductions and shifts are DPP,
 // and a leaf's primitive is loaded once its box is admitted (a quarter of them are).
@@ -1409,15 +1410,15 @@ struct WideNodes {
 // 2M-triangle terrain with 100k queries: closest 277 -> 205 us, kNN16 443 -> 308 us; one
 // path through all regions of the triangle distance instead of its exits: no faster here,
 // 15 % slower around an icosphere (1.01 -> 1.16 ms).
-template <typename L, int K, int G, bool kStats, typename Nodes>
+template <typename L, bool kOne, int G, bool kStats, typename Nodes>
 struct GroupNearest {
     static_assert(G == 16 || G == 32 || G == 64, "lanes per query");
-    static_assert(K <= G, "the k-best list takes one lane per entry");
     static constexpr bool kSortPushes = L::kKind == 2;
     static constexpr int kQuads = G / 4;                 // nodes a query expands per round
     static constexpr int kStack = kWaveStack / (64 / G);  // stack entries per query
-    uint32_t ld, lid;  // this lane's list entry (K = 1: the best, in every lane)
-    uint32_t kd, kid;  // the list's K-th (the same in every lane)
+    int k;             // list length, at most G (kOne: 1)
+    uint32_t ld, lid;  // this lane's list entry (k > 1)
+    uint32_t kd, kid;  // the list's k-th (the same in every lane)
 
     __device__ __forceinline__ void walk(const Nodes& nodes, const typename L::Item* __restrict__ prims,
                                          const int* __restrict__ primIds, V3 p, LdsInt* stk, int lane,
@@ -1480,7 +1481,7 @@ struct GroupNearest {
             }
             const unsigned long long bm = __ballot(better);
             if (bm != 0) {
-                if constexpr (K == 1) {
+                if constexpr (kOne) {
                     const uint32_t m = groupMin<G>(cd);
                     const uint32_t mi = groupMin<G>(cd == m ? cid : ~0u);
                     const bool got = m != ~0u;  // (a candidate is closer than the entry)
@@ -1542,19 +1543,19 @@ struct GroupNearest {
             ld = stays ? ld : nd;
             lid = stays ? lid : ni;
         }
-        const int last = (lane & ~(G - 1)) + K - 1;
+        const int last = (lane & ~(G - 1)) + k - 1;
         kd = permuteU(last, ld);
         kid = permuteU(last, lid);
     }
 
-    __device__ __forceinline__ void store(ClosestResult* __restrict__ dst, int k, int gl) const {
-        const uint32_t d = K == 1 ? kd : ld, i = K == 1 ? kid : lid;
-        if (gl < k) dst[gl] = i == kNoPrim ? ClosestResult{0u, -1} : ClosestResult{d, static_cast<int>(i)};
+    __device__ __forceinline__ void store(ClosestResult* __restrict__ dst, int gl) const {
+        const uint32_t d = kOne ? kd : ld, i = kOne ? kid : lid;
+        if (gl < (kOne ? 1 : k)) dst[gl] = i == kNoPrim ? ClosestResult{0u, -1} : ClosestResult{d, static_cast<int>(i)};
     }
 };
 
 // The walk over a plain 4-wide tree: 64 / G queries per wave.
-template <typename L, int K, int G, bool kStats>
+template <typename L, bool kOne, int G, bool kStats>
 __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
     const Wide4* __restrict__ wide, const typename L::Item* __restrict__ prims,
     const int* __restrict__ primIds, const V3* __restrict__ points, const uint32_t* __restrict__ order,
@@ -1566,12 +1567,40 @@ __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
     int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
     if (qi < count) {  // the same in the whole group
         const int q = order ? static_cast<int>(order[qi]) : qi;
-        GroupNearest<L, K, G, kStats, WideNodes> g;
+        GroupNearest<L, kOne, G, kStats, WideNodes> g;
+        g.k = k;
         LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * g.kStack);
         g.walk(WideNodes{wide}, prims, primIds, points[q], stk, lane, idMask, nodeTests, leafTests, overflow, opened);
-        g.store(out + static_cast<size_t>(q) * outStride, k, lane & (G - 1));
+        g.store(out + static_cast<size_t>(q) * outStride, lane & (G - 1));
     }
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
+}
+
+// Batched scenes by groups: G lanes walk one query of the batch's queue on its own
+// scene's 4-wide tree (scene s: items from primOff[s], nodes from wideRoot[s]).  Queries
+// lie scene by scene, so an XCD's contiguous range stays on a few scenes' nodes.
+template <typename L, bool kOne, int G, int kBT>
+__global__ __launch_bounds__(kBT) void batchGroupKernel(
+    const Wide4* __restrict__ wide, const int* __restrict__ wideRoot, const typename L::Item* __restrict__ prims,
+    const int* __restrict__ primIds, const int* __restrict__ primOff, const V3* __restrict__ points,
+    const int* __restrict__ qScene, const uint32_t* __restrict__ order, int count, int k, int outStride,
+    ClosestResult* __restrict__ out) {
+    __shared__ int lds[kWaveStack * (kBT / 64)];
+    const int lane = threadIdx.x & 63;
+    const int qi = (xcdBlock() * (kBT / 64) + (threadIdx.x >> 6)) * (64 / G) + lane / G;
+    int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
+    if (qi < count) {  // the same in the whole group
+        const int q = order ? static_cast<int>(order[qi]) : qi;
+        const int s = qScene[q];
+        const int ps = primOff[s], wr = wideRoot[s];
+        GroupNearest<L, kOne, G, false, WideNodes> g;
+        g.k = k;
+        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * g.kStack);
+        g.walk(WideNodes{wide + wr}, prims + ps, primIds + ps, points[q], stk, lane, stackIdMask(wideRoot[s + 1] - wr),
+               nodeTests, leafTests, overflow, opened);
+        g.store(out + static_cast<size_t>(q) * outStride, lane & (G - 1));
+    }
+    flushStats<false>(nullptr, nodeTests, leafTests, overflow, opened);
 }
 
 // Closest-hit rays with one wave per ray (the layout of the wave kernels above: 16
@@ -2027,14 +2056,13 @@ int gTraversalMode = 0;
 // (Group16 / Group32: 16 or 32 lanes per query, four or two queries per wave.)
 enum NearestShape : int { kShapeLane = 0, kShapeQuad = 1, kShapeWave = 2, kShapeGroup16 = 3, kShapeGroup32 = 4 };
 
-// Tuned shapes.  The best shape depends on how long and how uneven the walks are,
-// which the query count alone does not tell: on the terrain a million closest
-// queries run fastest four lanes per query (3.2 ms, one wave per query 4.0), while
-// 262,144 queries in and around an icosphere -- long walks of very different
-// lengths -- run 5.5x faster one wave per query (1.6 ms against 8.6 one lane per
-// query).  From kTuneFrom queries on, the first call for a (tree, k class, query
-// count octave) times the three shapes on its own queries and keeps the fastest;
-// every shape writes the same bits, so the trials' output is the call's output.
+// Tuned shapes.  The best shape depends on how long and how uneven the walks are, which
+// the query count alone does not tell: 262,144 closest queries on the terrain run fastest
+// 16 lanes per query (410 us, one wave per query 597), as many in and around an icosphere
+// -- long walks of very different lengths -- one wave per query (970 us against 1312).
+// From kTuneFrom queries on, the first call for a (tree, k class, query count octave)
+// times the three group shapes on its own queries and keeps the fastest; every shape
+// writes the same bits, so the trials' output is the call's output.
 constexpr int kTuneFrom = 65536;
 
 struct TuneKey {
@@ -2181,44 +2209,39 @@ void checkOverflow() {
                       "so some results are incomplete");
 }
 
-// kNN (k > 1): four lanes per query at every size -- the quad's spread k-best list
-// makes each offer a quarter of the per-lane work, and it measured faster from 20k
-// to 1M queries on the 2M-triangle terrain.  Closest (k = 1): four lanes per query
-// while the query set leaves most of the GPU idle one lane per query (fewer than 4
-// waves per SIMD: 256 CUs x 4 SIMDs x 4 waves x 64 lanes).
 // Radius capture one wave per query below this many queries, four lanes per query
 // above (traversal mode 2 forces four lanes per query).
 int gRadiusWaveBelow = 1 << 17;
 
-// Closest / kNN one wave per query below a leaf- and k-dependent count (automatic
-// mode, under kTuneFrom queries).  A small query set fills the device only with more
-// lanes per query, while past that the quad kernel needs fewer instructions per
-// query on short, even walks.
-// Measured crossovers (kernel time against the quad kernel, same bits): the
-// 2M-triangle terrain on a SAH tree -- closest about 200k queries, kNN16 about 150k
-// (100k: closest 0.45 vs 0.57 ms, kNN16 0.72 vs 0.80); 1M points -- closest about
-// 35k (20k: 0.08 vs 0.11 ms), kNN8 about 45k; 1M Gaussians -- closest about 45k,
-// kNN8 beyond 80k (80k: 0.81 vs 1.08 ms).
-template <typename L, int K>
-static bool useWave(int count) {
-    int below;
-    if (L::kKind == 0) below = K > 1 ? 131072 : 196608;
-    else if (L::kKind == 1) below = K > 1 ? 45056 : 32768;
-    else below = K > 1 ? 131072 : 45056;
-    return count < below;
+// Lanes per closest / kNN query (64, 32 or 16) by the number of queries.  A small set
+// fills the device only with more lanes per query; a large one is served with the fewest
+// instructions by 16.  Measured (kernel us at 64 / 32 / 16 lanes): the 2M-triangle terrain,
+// SAH tree, closest 8k 43 / 52 / 78, 16k 64 / 62 / 88, 60k 165 / 140 / 145, kNN16 32k
+// 160 / 143 / 159; around an icosphere, where walks are long and uneven, closest 16k
+// 155 / 284 / 473, 60k 264 / 364 / 561 -- so triangles change late, and from kTuneFrom
+// queries on the call times the three; 1M points kNN8 4k 33 / 32 / 41, 16k 69 / 52 / 53,
+// 60k 196 / 125 / 88; 1M Gaussians closest 4k 64 / 47 / 58, 32k 253 / 152 / 126.  One lane
+// and four lanes per query are behind at every count up to 1M (terrain closest 1M: 3253
+// and 2900 against 1361; points kNN8 1M: 1135 and 1338 against 810).
+template <typename L>
+static int lanesPerQuery(int count, int k) {
+    constexpr int kBelow64 = L::kKind == 0 ? 16384 : 3072;
+    constexpr int kBelow32 = L::kKind == 0 ? kTuneFrom : (L::kKind == 1 ? 12288 : 28672);
+    const int lanes = count < kBelow64 ? 64 : (count < kBelow32 ? 32 : 16);
+    return k > 16 && lanes < 32 ? 32 : lanes;  // the list takes a lane per entry
 }
 
-// G lanes per query (64: one wave per query).
-template <typename L, int K, int G>
+// G lanes per query (64: one wave per query), k at most G.
+template <typename L, bool kOne, int G>
 static void launchGroup(const TraverseArgs& a, const V3* pts, int count, int k, int outStride, ClosestResult* out,
                         unsigned long long* stats, hipStream_t s) {
     const auto* prims = static_cast<const typename L::Item*>(a.items);
     const uint32_t idMask = stackIdMask(a.wideCount);
     const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
     if (stats)
-        nearestWaveKernel<L, K, G, true><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idMask);
+        nearestWaveKernel<L, kOne, G, true><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idMask);
     else
-        nearestWaveKernel<L, K, G, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idMask);
+        nearestWaveKernel<L, kOne, G, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idMask);
 }
 
 template <typename L, int K>
@@ -2227,16 +2250,12 @@ static void launchShape(int shape, const TraverseArgs& a, const V3* pts, int cou
     const auto* prims = static_cast<const typename L::Item*>(a.items);
     const int idBits = stackIdBitsDev(a.wideCount);
     if (shape == kShapeWave) {
-        launchGroup<L, K, 64>(a, pts, count, k, outStride, out, stats, s);
+        launchGroup<L, K == 1, 64>(a, pts, count, k, outStride, out, stats, s);
     } else if (shape == kShapeGroup16 || shape == kShapeGroup32) {
-        if constexpr (K <= 16) {
-            if (shape == kShapeGroup16)
-                launchGroup<L, K, 16>(a, pts, count, k, outStride, out, stats, s);
-            else
-                launchGroup<L, K, 32>(a, pts, count, k, outStride, out, stats, s);
-        } else {
-            launchGroup<L, K, 32>(a, pts, count, k, outStride, out, stats, s);  // 32 entries need 32 lanes
-        }
+        if (shape == kShapeGroup16 && K <= 16)
+            launchGroup<L, K == 1, 16>(a, pts, count, k, outStride, out, stats, s);
+        else  // (more than 16 entries need 32 lanes)
+            launchGroup<L, K == 1, 32>(a, pts, count, k, outStride, out, stats, s);
     } else if (shape == kShapeQuad) {
         const int grid = blocksFor(4LL * count, kBlock);
         if (stats)
@@ -2255,8 +2274,8 @@ static void launchShape(int shape, const TraverseArgs& a, const V3* pts, int cou
 // The shape for a set of `count` queries by the measured crossovers (above).
 template <typename L, int K>
 static int defaultShape(int count) {
-    if (useWave<L, K>(count)) return kShapeWave;
-    return (K > 1 || count < 256 * 4 * 4 * 64) ? kShapeQuad : kShapeLane;
+    const int lanes = lanesPerQuery<L>(count, K);
+    return lanes == 64 ? kShapeWave : (lanes == 32 ? kShapeGroup32 : kShapeGroup16);
 }
 
 template <typename L, int K>
@@ -2272,10 +2291,10 @@ static int tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, in
     }
     // every candidate shape once, after one untimed walk that brings the tree into
     // the caches (so the first timed shape is not the only one reading it cold)
-    constexpr int kShapes = K <= 16 ? 5 : 4;
-    const int shapes[5] = {kShapeLane, kShapeQuad, kShapeWave, kShapeGroup32, kShapeGroup16};
-    EventSet<2 * 5> ev;
-    launchShape<L, K>(kShapeWave, a, pts, count, k, outStride, out, nullptr, s);
+    constexpr int kShapes = K <= 16 ? 3 : 2;
+    const int shapes[3] = {kShapeWave, kShapeGroup32, kShapeGroup16};
+    EventSet<2 * kShapes> ev;
+    launchShape<L, K>(kShapeGroup32, a, pts, count, k, outStride, out, nullptr, s);
     for (int i = 0; i < kShapes; ++i) {
         ev.record(2 * i, s);
         launchShape<L, K>(shapes[i], a, pts, count, k, outStride, out, nullptr, s);
@@ -2283,7 +2302,7 @@ static int tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, in
     }
     hipCheck(hipGetLastError(), "nearest tuning");
     ev.sync(2 * kShapes - 1);
-    int best = kShapeLane;
+    int best = kShapeWave;
     float bestMs = 0.0f;
     for (int i = 0; i < kShapes; ++i) {
         const float ms = ev.ms(2 * i, 2 * i + 1);
@@ -2634,6 +2653,27 @@ void launchBatchTKV(const BatchQueryArgs& a, hipStream_t s) {
                               a.primOff, a.points, a.qScene, a.order, a.count, a.k, a.outStride, a.out, a.counter);
 }
 
+template <typename L, int G, int kBT>
+void launchBatchGroup(const BatchQueryArgs& a, hipStream_t s) {
+    const int grid = blocksFor(a.count, (kBT / 64) * (64 / G));
+    const auto kern = a.k <= 1 ? batchGroupKernel<L, true, G, kBT> : batchGroupKernel<L, false, G, kBT>;
+    kern<<<grid, kBT, 0, s>>>(a.wide, a.wideRoot, static_cast<const typename L::Item*>(a.items), a.primIds, a.primOff,
+                              a.points, a.qScene, a.order, a.count, a.k, a.outStride, a.out);
+}
+
+// The 4-wide LDS-stack variants: as many lanes per query as a plain call of that many
+// queries takes.  One lane per query on a work queue, which these replaced, left the
+// device waiting for the longest walks: 51k closest / kNN8 queries over 64 scenes 646 /
+// 1012 us against 109 / 190, 1.73M over 2,048 scenes 1986 / 3329 against 1389 / 2563.
+template <typename L, int kBT>
+void launchBatchGroups(const BatchQueryArgs& a, hipStream_t s) {
+    switch (lanesPerQuery<L>(a.count, a.k)) {
+        case 64: launchBatchGroup<L, 64, kBT>(a, s); break;
+        case 32: launchBatchGroup<L, 32, kBT>(a, s); break;
+        default: launchBatchGroup<L, 16, kBT>(a, s); break;
+    }
+}
+
 template <typename L, int K>
 void launchBatchTK(const BatchQueryArgs& a, int variant, hipStream_t s) {
     switch (variant) {
@@ -2641,8 +2681,8 @@ void launchBatchTK(const BatchQueryArgs& a, int variant, hipStream_t s) {
         case kBatchLds64: launchBatchTKV<L, K, 64, kLdsDepth, false, false>(a, s); break;
         case kBatchScratch64: launchBatchTKV<L, K, 64, 0, false, false>(a, s); break;
         case kBatchReg64: launchBatchTKV<L, K, 64, 0, false, true>(a, s); break;
-        case kBatchWideLds256: launchBatchTKV<L, K, 256, kLdsDepth, true, false>(a, s); break;
-        case kBatchWideLds64: launchBatchTKV<L, K, 64, kLdsDepth, true, false>(a, s); break;
+        case kBatchWideLds256: launchBatchGroups<L, 256>(a, s); break;
+        case kBatchWideLds64: launchBatchGroups<L, 64>(a, s); break;
         case kBatchWideScratch64: launchBatchTKV<L, K, 64, 0, true, false>(a, s); break;
         default: launchBatchTKV<L, K, 64, 0, true, true>(a, s); break;
     }

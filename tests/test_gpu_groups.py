@@ -64,3 +64,28 @@ def test_group_walk_unusual_queries(A, orc, mode):  # noqa: F811
             assert eq(got[far, :, 1], np.tile(np.arange(max(k, 1), dtype=np.uint32), (len(far), 1)))
     finally:
         A.lib().qr_set_traversal_mode(0)
+
+
+# 64, 32 and 16 lanes per query (points change at 3,072 and 12,288 queries), on workgroups of
+# 256 and 64 lanes; k above 16 needs at least 32 lanes
+@pytest.mark.parametrize("variant", ["wide_lds256", "wide_lds64"])
+@pytest.mark.parametrize("nq,k", [(1, 0), (3071, 9), (3073, 0), (12287, 16), (12289, 0), (12290, 3), (12291, 20)])
+def test_batch_groups(A, orc, variant, nq, k):  # noqa: F811
+    print(f"variant={variant} nq={nq} k={k}", flush=True)
+    rng = np.random.default_rng(nq + k)
+    sizes = [2, 3, 700, 64, 5, 1500]
+    items = np.concatenate([scene(1, n, n) for n in sizes])
+    poff = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    cuts = np.sort(rng.integers(0, nq + 1, len(sizes) - 1))
+    qoff = np.concatenate([[0], cuts, [nq]]).astype(np.int32)
+    qoff[1] = 0  # a scene without queries
+    q = rng.uniform(-40, 40, (nq, 3)).astype(np.float32)
+    batch = A.Batch(1, items, poff)
+    plan = A.BatchPlan(batch, q, qoff, k, tune=(A.BATCH_VARIANTS.index(variant), bool(nq % 2)))
+    plan.run()
+    got = plan.read()
+    for s in range(len(sizes)):
+        a, b = qoff[s], qoff[s + 1]
+        if b > a:
+            want = orc.knn_brute(1, items[poff[s]:poff[s + 1]], q[a:b], k, threads=8)
+            assert eq(got[a:b], want), s
