@@ -102,8 +102,9 @@ QR_API int qr_warmup(void);
  * for a tree, k class and query-count octave times 16 and 32 lanes and one wave per
  * query on its own queries and keeps the fastest; radius 32
  * lanes per query (two queries per wave) below 131,072 queries, four lanes above;
- * rays one lane per ray), 1 one lane per query, 2 four lanes per query, 3 one wave
- * per query or ray, 4 as 0 but closest / kNN and rays tuned at every count, 5 / 6
+ * rays 64 to 8 lanes per ray by ray count, one lane from 393,216 on), 1 one lane per
+ * query or ray, 2 four lanes per query, 3 one wave per query or ray, 4 as 0 but closest
+ * / kNN and rays tuned at every count (rays: one lane or one wave), 5 / 6
  * closest and kNN with 16 / 32 lanes per query (four / two queries per wave; kNN
  * with k > 16 takes 32 lanes), radius as in mode 0 (5) or 32 lanes per query at
  * every count (6), other queries as in mode 0.  Results are identical in every

@@ -228,6 +228,7 @@ TraverseArgs argsFor(const BvhState& b, bool wide, bool arm = true) {
     a.wide = wide;
     a.nodes = b.nodes.p;
     a.nodeCount = b.nodeCount;
+    a.depth = b.depth;
     a.wideNodes = b.wide.p;
     a.wideCount = b.wideCount;
     a.items = b.items.p;

@@ -146,14 +146,15 @@ QR_HD bool rayBox(const Ray& ray, const Box& box, float tMax, float& tEnter) {
     return true;
 }
 
-// Same slab test with the per-axis reciprocal hoisted out of the traversal loop.
-// (lo - o) * inv with inv = 1/d is exactly what rayBox computes per call, so the
-// result bits are identical; the |d| < 1e-20 axes are flagged by inv == 0 sentinel
-// handling below (a separate mask keeps the skip rule exact).
+// The same slab test for one ray against many boxes: the reciprocals are formed once
+// (the values rayBox forms on each call), the slabs are intersected by min / max without
+// branches, and the ends are compared once -- t0 only grows and t1 only shrinks over the
+// axes, so the last comparison fails whenever an earlier one would have.
 struct RayPre {
     V3 o;
     V3 inv;
-    int flat;  // bit a set: |dir[a]| < 1e-20, the axis is tested by containment
+    bool flatX, flatY, flatZ;  // |dir| < 1e-20: the axis is tested by containment
+    bool anyFlat;
     float tMin;
 };
 
@@ -161,48 +162,34 @@ QR_HD RayPre rayPrepare(const Ray& ray) {
     RayPre p;
     p.o = ray.origin;
     p.tMin = ray.tMin;
-    p.flat = 0;
-    const float d[3] = {ray.dir.x, ray.dir.y, ray.dir.z};
-    float inv[3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        if (fabsf(d[a]) < 1e-20f) {
-            p.flat |= 1 << a;
-            inv[a] = 0.0f;
-        } else {
-            inv[a] = 1.0f / d[a];
-        }
-    }
-    p.inv = {inv[0], inv[1], inv[2]};
+    p.flatX = fabsf(ray.dir.x) < 1e-20f;
+    p.flatY = fabsf(ray.dir.y) < 1e-20f;
+    p.flatZ = fabsf(ray.dir.z) < 1e-20f;
+    p.anyFlat = p.flatX | p.flatY | p.flatZ;
+    p.inv = {1.0f / ray.dir.x, 1.0f / ray.dir.y, 1.0f / ray.dir.z};
     return p;
 }
 
 QR_HD bool rayBoxPre(const RayPre& r, const Box& box, float tMax, float& tEnter) {
-    float t0 = r.tMin;
-    float t1 = tMax * (1.0f + 1e-6f) + 1e-6f;
-#pragma unroll
-    for (int axis = 0; axis < 3; ++axis) {
-        const float o = comp(r.o, axis);
-        const float lo = comp(box.lo, axis);
-        const float hi = comp(box.hi, axis);
-        if (r.flat & (1 << axis)) {
-            if (o < lo || o > hi) return false;
-            continue;
-        }
-        const float inv = comp(r.inv, axis);
-        float ta = (lo - o) * inv;
-        float tb = (hi - o) * inv;
-        if (ta > tb) {
-            const float tmp = ta;
-            ta = tb;
-            tb = tmp;
-        }
-        t0 = ta > t0 ? ta : t0;
-        t1 = tb < t1 ? tb : t1;
-        if (t0 > t1 * (1.0f + 1e-6f) + 1e-6f) return false;
+    float ax = (box.lo.x - r.o.x) * r.inv.x, bx = (box.hi.x - r.o.x) * r.inv.x;
+    float ay = (box.lo.y - r.o.y) * r.inv.y, by = (box.hi.y - r.o.y) * r.inv.y;
+    float az = (box.lo.z - r.o.z) * r.inv.z, bz = (box.hi.z - r.o.z) * r.inv.z;
+    bool out = false;
+    if (r.anyFlat) {  // a flat axis bounds nothing, but a box beside the ray is missed
+        out = (r.flatX & ((r.o.x < box.lo.x) | (r.o.x > box.hi.x))) |
+              (r.flatY & ((r.o.y < box.lo.y) | (r.o.y > box.hi.y))) |
+              (r.flatZ & ((r.o.z < box.lo.z) | (r.o.z > box.hi.z)));
+        ax = r.flatX ? -kInf : ax;
+        bx = r.flatX ? kInf : bx;
+        ay = r.flatY ? -kInf : ay;
+        by = r.flatY ? kInf : by;
+        az = r.flatZ ? -kInf : az;
+        bz = r.flatZ ? kInf : bz;
     }
+    const float t0 = fmaxf(fmaxf(r.tMin, fminf(ax, bx)), fmaxf(fminf(ay, by), fminf(az, bz)));
+    const float t1 = fminf(fminf(tMax * (1.0f + 1e-6f) + 1e-6f, fmaxf(ax, bx)), fminf(fmaxf(ay, by), fmaxf(az, bz)));
     tEnter = t0;
-    return true;
+    return !(out | (t0 > t1 * (1.0f + 1e-6f) + 1e-6f));
 }
 
 // hitParamInsideBox (geometry.h:112-143).

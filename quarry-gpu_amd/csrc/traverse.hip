@@ -37,7 +37,7 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kLdsDepth = 32;
-constexpr int kSpill = 112;  // scratch entries beyond the LDS part (never reached by LBVH trees)
+constexpr int kSpill = 128;  // scratch entries beyond the LDS part (never reached by LBVH trees)
 
 // ---- XCD-aware block numbering ------------------------------------------------------
 // Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.  The
@@ -259,6 +259,45 @@ struct KnnList {
     }
 };
 
+// Stack entries of the closest / kNN walks carry the child's box distance above its id,
+// truncated to the bits the id leaves free: the leading bits of a non-negative
+// float are a lower bound of it.  A popped node whose bound already exceeds the
+// k-th distance is dropped without being opened -- opening it would find every
+// child beyond the k-th distance too (a child's box lies inside its parent's), so
+// the walk and its results are unchanged.  idBits = 32 turns the keys off (trees
+// whose wide ids need more than 23 bits).
+// Bits of a stack entry taken by a node id below `idCount` (the rest hold the
+// distance key); 32 = no key, when ids need more than 23 bits (fewer than 9 would
+// be left, too few for the float's exponent and a mantissa bit).
+__host__ __device__ __forceinline__ int stackIdBitsDev(int idCount) {
+    int bits = 1;
+    while (bits < 32 && (1LL << bits) < static_cast<long long>(idCount)) ++bits;
+    return bits <= 23 ? bits : 32;
+}
+
+// The same by mask (the low idBits bits; all 32 when there is no key): the float's bits,
+// shifted up over the sign, above the id.
+__host__ __device__ __forceinline__ uint32_t stackIdMask(int idCount) {
+    const int bits = idCount <= 2 ? 1 : 32 - __builtin_clz(static_cast<unsigned>(idCount - 1));
+    return bits > 23 ? ~0u : (1u << bits) - 1u;
+}
+__device__ __forceinline__ uint32_t stackEntry(uint32_t id, uint32_t keyBits, uint32_t idMask) {
+    return ((keyBits << 1) & ~idMask) | id;
+}
+__device__ __forceinline__ uint32_t stackKey(uint32_t v, uint32_t idMask) { return (v & ~idMask) >> 1; }
+
+__device__ __forceinline__ int packEntry(int id, float key, int idBits) {
+    if (idBits >= 32) return id;
+    const uint32_t q = floatBits(key) >> (idBits - 1);
+    return static_cast<int>((q << idBits) | static_cast<uint32_t>(id));
+}
+__device__ __forceinline__ int entryId(int v, int idBits) {
+    return idBits >= 32 ? v : static_cast<int>(static_cast<uint32_t>(v) & ((1u << idBits) - 1u));
+}
+__device__ __forceinline__ float entryKey(int v, int idBits) {
+    return idBits >= 32 ? 0.0f : bitsFloat((static_cast<uint32_t>(v) >> idBits) << (idBits - 1));
+}
+
 // ---- rays --------------------------------------------------------------------------
 // Each iteration opens one interior node: its children are tested, leaves are
 // intersected nearest first, and the nearest surviving interior child becomes the
@@ -402,6 +441,22 @@ __device__ __forceinline__ int descend(const int (&c)[4], const bool (&ok)[4], L
     return next;
 }
 
+// The farthest entry distance, as ray stacks keep them (not below zero), that a hit
+// nearer than `best` may still lie behind: the box tests' slack; a negative best (a ray
+// whose tMin is negative) drops nothing at zero.
+__device__ __forceinline__ float stackReach(float best) { return fmaxf(best * (1.0f + 1e-6f) + 1e-6f, 0.0f); }
+
+// One lane per ray over 4-wide nodes, for large ray sets.  The leaves of an opened node are
+// tested one per lane and step, not slot by slot: the wave runs the triangle test (the
+// longest piece of a step) as often as its busiest lane has leaves, not four times.  The
+// children's box tests share the ray's reciprocals and have no branches; the nearest
+// interior child is opened next and the others go on the stack farthest first by rank (no
+// sort moves them), with their entry distance above their id: a popped entry that lies
+// beyond the best hit is dropped unopened.  1M rays, kernel time before and after: city,
+// cosine 682 -> 477 us, down 300 -> 242; 131k terrain, cosine 1009 -> 678, down 352 -> 298;
+// icosphere 954 -> 705.  Opening nodes until some lane has a leaf before testing any was
+// slower (icosphere 1097).
+constexpr int kRayDepth = 16;  // stack entries per lane in LDS (8 workgroups a CU), the rest in scratch
 template <bool kStats, bool kSave>
 __global__ __launch_bounds__(kBlock) void rayWideKernel(const Wide4* __restrict__ wide,
                                                         const Tri* __restrict__ tris,
@@ -410,49 +465,81 @@ __global__ __launch_bounds__(kBlock) void rayWideKernel(const Wide4* __restrict_
                                                         int count, uint64_t* __restrict__ out,
                                                         unsigned long long* __restrict__ stats,
                                                         const int* __restrict__ primIds,
-                                                        int* __restrict__ hitPrim) {
-    __shared__ int lds[kLdsDepth * kBlock];
+                                                        int* __restrict__ hitPrim, uint32_t idMask) {
+    __shared__ int lds[kRayDepth * kBlock];
     const int i = xcdBlock() * kBlock + threadIdx.x;
     int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
     if (i < count) {
         const int q = order ? static_cast<int>(order[i]) : i;
         const Ray ray = rays[q];
+        const RayPre pre = rayPrepare(ray);
         float best = ray.tMax;
         bool any = false;
         int bestId = -1;
-        LaneStack st;
+        LaneStackT<kBlock, kRayDepth> st;
         SpillArea spill;
         st.init(lds);
-        int id = 0;
-        while (id >= 0) {
+        uint32_t next = 0;  // the entry to open (kDone: none left)
+        constexpr uint32_t kDone = ~0u;
+        while (next != kDone) {
+            int leaf[4];
+            uint32_t leaves = 0;
             if (kStats) ++opened;
-            WideEntry e[4];
-            loadWide(wide, id, e);
-            float key[4];
+            const Wide4& wn = wide[next & idMask];
+            next = kDone;
+            uint32_t key[4];
             int c[4];
+            bool in[4];
+            int m = 0;
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                c[s] = e[s].child;
-                key[s] = kInf;
+                const WideEntry e = wn.c[s];
                 float t;
-                if (c[s] != kWideEmpty && rayBox(ray, entryBox(e[s]), best, t)) {
-                    key[s] = t;
-                    ++nodeTests;
-                } else {
-                    c[s] = kWideEmpty;
-                }
+                c[s] = e.child;
+                const bool adm = rayBoxPre(pre, entryBox(e), best, t) & (c[s] != kWideEmpty);
+                if (kStats && adm) ++nodeTests;
+                in[s] = adm & (c[s] >= 0);
+                key[s] = in[s] ? (floatBits(fmaxf(t, 0.0f)) & ~3u) | s : 0xfffffffcu | s;
+                m += in[s] ? 1 : 0;
+                leaf[s] = -c[s] - 1;
+                leaves |= adm & (c[s] < 0) ? 1u << s : 0u;
             }
-            sort4(key, c);
-            bool ok[4];
+            if (m > 0) {
+                if (!st.room(3)) {
+                    overflow = 1;
+                    break;
+                }
+                const int a = key[1] < key[0], b = key[2] < key[0], d = key[3] < key[0];
+                const int e = key[2] < key[1], f = key[3] < key[1], g = key[3] < key[2];
+                const int rank[4] = {a + b + d, 1 - a + e + f, 2 - b - e + g, 3 - d - f - g};
+                const int top = st.sp + m - 1;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                ok[s] = c[s] != kWideEmpty;
-                if (ok[s] && c[s] < 0) {
-                    ++leafTests;
-                    rayLeaf<kSave>(ray, tris, primIds, -c[s] - 1, best, any, bestId);
+                for (int s = 0; s < 4; ++s) {
+                    const uint32_t v = stackEntry(static_cast<uint32_t>(c[s]), key[s], idMask);
+                    if (rank[s] == 0) next = v;
+                    if (in[s] & (rank[s] > 0)) {
+                        const int at = top - rank[s];
+                        if (at < kRayDepth) st.base[at * kBlock] = static_cast<int>(v);
+                        else *spill.at(at - kRayDepth) = static_cast<int>(v);
+                    }
+                }
+                st.sp = top;
+            } else {
+                const float reach = stackReach(best);
+                while (!st.empty()) {
+                    const uint32_t v = static_cast<uint32_t>(stackPop(st, spill));
+                    if (bitsFloat(stackKey(v, idMask)) <= reach) {
+                        next = v;
+                        break;
+                    }
                 }
             }
-            id = descend(c, ok, st, spill, overflow);
+            while (leaves != 0) {
+                const int slot = (leaves & 1u) ? leaf[0] : ((leaves & 2u) ? leaf[1] : ((leaves & 4u) ? leaf[2] : leaf[3]));
+                leaves &= leaves - 1u;
+                if (kStats) ++leafTests;
+                rayLeaf<kSave>(ray, tris, primIds, slot, best, any, bestId);
+            }
         }
         out[q] = any ? ((uint64_t{1} << 32) | floatBits(best)) : 0ull;
         if (kSave) hitPrim[q] = any ? bestId : -1;
@@ -472,45 +559,6 @@ __device__ __forceinline__ void writeList(const KnnList<K>& list, int k, Closest
             dst[s] = r;
         }
     }
-}
-
-// Stack entries of the closest / kNN walks carry the child's box distance above its id,
-// truncated to the bits the id leaves free: the leading bits of a non-negative
-// float are a lower bound of it.  A popped node whose bound already exceeds the
-// k-th distance is dropped without being opened -- opening it would find every
-// child beyond the k-th distance too (a child's box lies inside its parent's), so
-// the walk and its results are unchanged.  idBits = 32 turns the keys off (trees
-// whose wide ids need more than 23 bits).
-// Bits of a stack entry taken by a node id below `idCount` (the rest hold the
-// distance key); 32 = no key, when ids need more than 23 bits (fewer than 9 would
-// be left, too few for the float's exponent and a mantissa bit).
-__host__ __device__ __forceinline__ int stackIdBitsDev(int idCount) {
-    int bits = 1;
-    while (bits < 32 && (1LL << bits) < static_cast<long long>(idCount)) ++bits;
-    return bits <= 23 ? bits : 32;
-}
-
-// The same by mask (the low idBits bits; all 32 when there is no key): the float's bits,
-// shifted up over the sign, above the id.
-__host__ __device__ __forceinline__ uint32_t stackIdMask(int idCount) {
-    const int bits = idCount <= 2 ? 1 : 32 - __builtin_clz(static_cast<unsigned>(idCount - 1));
-    return bits > 23 ? ~0u : (1u << bits) - 1u;
-}
-__device__ __forceinline__ uint32_t stackEntry(uint32_t id, uint32_t keyBits, uint32_t idMask) {
-    return ((keyBits << 1) & ~idMask) | id;
-}
-__device__ __forceinline__ uint32_t stackKey(uint32_t v, uint32_t idMask) { return (v & ~idMask) >> 1; }
-
-__device__ __forceinline__ int packEntry(int id, float key, int idBits) {
-    if (idBits >= 32) return id;
-    const uint32_t q = floatBits(key) >> (idBits - 1);
-    return static_cast<int>((q << idBits) | static_cast<uint32_t>(id));
-}
-__device__ __forceinline__ int entryId(int v, int idBits) {
-    return idBits >= 32 ? v : static_cast<int>(static_cast<uint32_t>(v) & ((1u << idBits) - 1u));
-}
-__device__ __forceinline__ float entryKey(int v, int idBits) {
-    return idBits >= 32 ? 0.0f : bitsFloat((static_cast<uint32_t>(v) >> idBits) << (idBits - 1));
 }
 
 // Closest / kNN walk of one query over a binary tree whose node ids, leaf slots
@@ -1332,8 +1380,8 @@ template <int G>
 __device__ __forceinline__ uint32_t groupMin(uint32_t x) {
     x = minU(x, dppU<0xB1>(x));   // quad_perm [1,0,3,2]
     x = minU(x, dppU<0x4E>(x));   // quad_perm [2,3,0,1]
-    x = minU(x, dppU<0x141>(x));  // row_half_mirror
-    x = minU(x, dppU<0x140>(x));  // row_mirror
+    if constexpr (G >= 8) x = minU(x, dppU<0x141>(x));   // row_half_mirror
+    if constexpr (G >= 16) x = minU(x, dppU<0x140>(x));  // row_mirror
     if constexpr (G >= 32) {
         const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
         x = minU(r[0], r[1]);
@@ -1347,8 +1395,9 @@ __device__ __forceinline__ uint32_t groupMin(uint32_t x) {
 // The group's lane i receives lane i - 1's x, its first lane 0.
 template <int G>
 __device__ __forceinline__ uint32_t groupShiftUp(uint32_t x, int gl) {
-    if constexpr (G == 16) {
-        return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x111, 0xF, 0xF, false));
+    if constexpr (G <= 16) {
+        const int v = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x111, 0xF, 0xF, false);
+        return static_cast<uint32_t>(G < 16 && gl == 0 ? 0 : v);
     } else {
         const int v = __builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x138, 0xF, 0xF, false);
         return static_cast<uint32_t>(G == 32 && gl == 0 ? 0 : v);
@@ -1386,6 +1435,26 @@ struct WideNodes {
         const WideEntry e = wide[id].c[slot];
         box = entryBox(e);
         return e.child;
+    }
+};
+
+// The same over binary nodes: entry `slot` of the up to four grandchildren of interior
+// node `id` (a leaf child stands for itself in its first slot).
+struct BinaryNodes {
+    const Node2* __restrict__ nodes;
+    __device__ __forceinline__ int entry(int id, int slot, Box& box) const {
+        const int c = (slot & 2) != 0 ? nodes[id].right : nodes[id].left;
+        Node2 cn = nodes[c];
+        int code = c;
+        if (cn.left < 0) {
+            code = (slot & 1) != 0 ? kWideEmpty : cn.left;
+        } else {
+            code = (slot & 1) != 0 ? cn.right : cn.left;
+            cn = nodes[code];
+            code = cn.left < 0 ? cn.left : code;
+        }
+        box = nodeBox(cn);
+        return code;
     }
 };
 
@@ -1554,10 +1623,10 @@ struct GroupNearest {
     }
 };
 
-// The walk over a plain 4-wide tree: 64 / G queries per wave.
-template <typename L, bool kOne, int G, bool kStats>
+// The walk over a plain tree: 64 / G queries per wave.
+template <typename L, bool kOne, int G, bool kStats, typename Nodes>
 __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
-    const Wide4* __restrict__ wide, const typename L::Item* __restrict__ prims,
+    Nodes nodes, const typename L::Item* __restrict__ prims,
     const int* __restrict__ primIds, const V3* __restrict__ points, const uint32_t* __restrict__ order,
     int count, int k, int outStride, ClosestResult* __restrict__ out, unsigned long long* __restrict__ stats,
     uint32_t idMask) {
@@ -1567,10 +1636,10 @@ __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
     int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
     if (qi < count) {  // the same in the whole group
         const int q = order ? static_cast<int>(order[qi]) : qi;
-        GroupNearest<L, kOne, G, kStats, WideNodes> g;
+        GroupNearest<L, kOne, G, kStats, Nodes> g;
         g.k = k;
         LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * g.kStack);
-        g.walk(WideNodes{wide}, prims, primIds, points[q], stk, lane, idMask, nodeTests, leafTests, overflow, opened);
+        g.walk(nodes, prims, primIds, points[q], stk, lane, idMask, nodeTests, leafTests, overflow, opened);
         g.store(out + static_cast<size_t>(q) * outStride, lane & (G - 1));
     }
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
@@ -1603,112 +1672,107 @@ __global__ __launch_bounds__(kBT) void batchGroupKernel(
     flushStats<false>(nullptr, nodeTests, leafTests, overflow, opened);
 }
 
-// Closest-hit rays with one wave per ray (the layout of the wave kernels above: 16
-// quads expand up to 16 stacked nodes of one walk per round, lane s of a quad tests
-// entry s).  A round's hits reduce to the wave's smallest (t, then primitive index --
-// the lane kernels' rule for equal t), boxes are tested against the best t so far
-// with the lane kernels' slack, and popped entries whose entry distance (kept in the
-// stack entry, truncated: a lower bound) is beyond it are dropped.  Interior children
-// go on the stack nearest-parent first, each parent's nearest on top.
-template <bool kStats, bool kSave>
-__global__ __launch_bounds__(kBlock) void rayWaveKernel(const Wide4* __restrict__ wide,
-                                                        const Tri* __restrict__ tris,
+// Closest-hit walk of one ray by a group of G lanes (the layout of the query walks above).
+// A round's hits reduce to the group's smallest (t, then, when saved, primitive index --
+// the lane kernels' rule for equal t), boxes are tested against the best t so far with
+// the lane kernels' slack, and popped entries whose entry distance (kept in the stack
+// entry, truncated: a lower bound; not below zero there) is beyond it are dropped.
+// Interior children go on the stack nearest parent first, each parent's nearest on top.
+template <int G, bool kStats, bool kSave, typename Nodes>
+__global__ __launch_bounds__(kBlock) void rayWaveKernel(Nodes nodes, const Tri* __restrict__ tris,
                                                         const Ray* __restrict__ rays,
                                                         const uint32_t* __restrict__ order, int count,
                                                         uint64_t* __restrict__ out,
                                                         unsigned long long* __restrict__ stats,
                                                         const int* __restrict__ primIds,
-                                                        int* __restrict__ hitPrim, int idBits) {
-    __shared__ int lds[kWaveStack * (kBlock / 64)];
+                                                        int* __restrict__ hitPrim, uint32_t idMask) {
+    constexpr int kQuads = G / 4;
+    constexpr int kStack = G == 4 ? 96 : kWaveStack / (64 / G);
+    __shared__ int lds[kStack * (kBlock / G)];
     const int lane = threadIdx.x & 63;
-    const int quad = lane >> 2;
+    const int gl = lane & (G - 1);
+    const int quad = gl >> 2;
     const int slot = lane & 3;
-    const int qi = xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6);
+    const int qi = (xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6)) * (64 / G) + lane / G;
     int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
-    if (qi < count) {  // the same in the whole wave
+    if (qi < count) {  // the same in the whole group
         const int q = order ? static_cast<int>(order[qi]) : qi;
         const Ray ray = rays[q];
+        const RayPre pre = rayPrepare(ray);
+        GroupBits<G> gb;
+        gb.init(lane);
         float best = ray.tMax;
         bool any = false;
-        int bestId = 0x7fffffff;
-        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack);
-        if (lane == 0) stk[0] = packEntry(0, 0.0f, idBits);
+        uint32_t bestId = kNoPrim;
+        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x / G) * kStack);
+        if (gl == 0) stk[0] = 0;
         int sp = 1;
         while (sp > 0) {
-            int width = (kWaveStack - kWaveHeadroom - sp) / 3;
-            width = width < 1 ? 1 : (width > 16 ? 16 : width);
-            const int take = width < sp ? width : sp;
+            int take = kQuads;
+            if constexpr (G > 4) {
+                const int room = kStack - kWaveHeadroom - sp;
+                if (room < 3 * kQuads) take = room < 3 ? 1 : room / 3;
+                take = take < sp ? take : sp;
+            }
             int node = -1;
             if (quad < take) {
-                const int v = stk[sp - 1 - quad];
-                if (entryKey(v, idBits) <= best * (1.0f + 1e-6f) + 1e-6f) node = entryId(v, idBits);
+                const uint32_t v = static_cast<uint32_t>(stk[sp - 1 - quad]);
+                if (bitsFloat(stackKey(v, idMask)) <= stackReach(best)) node = static_cast<int>(v & idMask);
             }
             sp -= take;
             if (kStats && slot == 0 && node >= 0) ++opened;
-            WideEntry e{};
+            Box box{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
             int ch = kWideEmpty;
-            if (node >= 0) {
-                e = wide[node].c[slot];
-                ch = e.child;
-            }
-            float tEnter = kInf;
-            bool adm = false;
-            if (ch != kWideEmpty) adm = rayBox(ray, entryBox(e), best, tEnter);
-            if (adm) ++nodeTests;
-            const bool leaf = ch < 0 && ch != kWideEmpty;
+            if (node >= 0) ch = nodes.entry(node, slot, box);
+            const bool leaf = static_cast<uint32_t>(ch) > static_cast<uint32_t>(kWideEmpty);
+            float tEnter;
+            const bool adm = rayBoxPre(pre, box, best, tEnter) & (ch != kWideEmpty);
+            if (kStats && adm) ++nodeTests;
             float ht = kInf;
-            int hid = 0x7fffffff;
-            if (adm && leaf) {
-                ++leafTests;
+            uint32_t hid = ~0u;
+            bool hit = false;
+            if (adm & leaf) {
+                if (kStats) ++leafTests;
                 float t;
                 // the lane kernels' rule: a nearer hit, or an equal one once there is a hit
                 if (rayTri(ray, tris[-ch - 1], t) && (t < best || (any && t == best))) {
                     ht = t;
-                    hid = primIds[-ch - 1];
+                    hit = true;
+                    if (kSave) hid = static_cast<uint32_t>(primIds[-ch - 1]);
                 }
             }
-            if (__ballot(ht < kInf) != 0) {
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) {
-                    const float ot = waveXor(ht, off);
-                    const int oi = waveXor(hid, off);
-                    if (closer(ot, oi, ht, hid)) {
-                        ht = ot;
-                        hid = oi;
-                    }
+            const unsigned long long hb = __ballot(hit);
+            if (hb != 0) {
+                const uint32_t mine = hit ? orderedBits(ht) : ~0u;
+                const uint32_t m = groupMin<G>(mine);
+                const bool got = m != ~0u;
+                const float t = got ? fromOrderedBits(m) : best;
+                if (kSave) {
+                    const uint32_t mi = groupMin<G>(mine == m ? hid : ~0u);
+                    bestId = !got ? bestId : (t < best || mi < bestId ? mi : bestId);
                 }
-                if (ht < best) {
-                    best = ht;
-                    bestId = hid;
-                    any = true;
-                } else if (any && ht == best && hid < bestId) {
-                    bestId = hid;
-                }
+                best = t;
+                any |= got;
             }
-            const bool push = adm && !leaf && tEnter <= best * (1.0f + 1e-6f) + 1e-6f;
-            const unsigned long long pm = __ballot(push);
-            const int pushes = __popcll(pm);
-            if (pushes > 0) {
-                if (sp + pushes > kWaveStack) {  // deeper than the stack bound allows
-                    if (lane == 0) overflow = 1;
-                    break;
+            const bool push = adm & !leaf & (tEnter <= best * (1.0f + 1e-6f) + 1e-6f);
+            const unsigned long long pb = __ballot(push);
+            if (pb != 0) {
+                const typename GroupBits<G>::Word pm = gb.of(pb);
+                const int top = sp + gb.count(pm);
+                if (top > kStack) {  // deeper than the stack bound allows
+                    if (gl == 0) overflow = 1;
+                    sp = 0;
+                } else {
+                    const uint32_t key = floatBits(fmaxf(tEnter, 0.0f));
+                    const int rank = quadRank(push, key, slot);
+                    if (push) stk[top - 1 - gb.count(pm & gb.lowerQuad) - rank] = static_cast<int>(stackEntry(static_cast<uint32_t>(ch), key, idMask));
+                    sp = top;
                 }
-                const float key = push ? tEnter : kInf;
-                const float k0 = quadGetF<0>(key), k1 = quadGetF<1>(key), k2 = quadGetF<2>(key), k3 = quadGetF<3>(key);
-                int rank = 0;
-                rank += (slot != 0) && (k0 < key || (k0 == key && 0 < slot));
-                rank += (slot != 1) && (k1 < key || (k1 == key && 1 < slot));
-                rank += (slot != 2) && (k2 < key || (k2 == key && 2 < slot));
-                rank += (slot != 3) && (k3 < key || (k3 == key && 3 < slot));
-                const int mine = __popcll((pm >> (4 * quad)) & 0xFull);
-                const int deeper = quad < 15 ? __popcll(pm >> (4 * (quad + 1))) : 0;
-                if (push) stk[sp + deeper + (mine - 1 - rank)] = packEntry(ch, tEnter, idBits);
-                sp += pushes;
             }
         }
-        if (lane == 0) {
+        if (gl == 0) {
             out[q] = any ? ((uint64_t{1} << 32) | floatBits(best)) : 0ull;
-            if (kSave) hitPrim[q] = any ? bestId : -1;
+            if (kSave) hitPrim[q] = any ? static_cast<int>(bestId) : -1;
         }
     }
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
@@ -2053,8 +2117,15 @@ void mortonOrder(const float* base, int stride, int count, int boxMode, SortWork
 int gTraversalMode = 0;
 
 // Shapes of a walk over 4-wide nodes.
-// (Group16 / Group32: 16 or 32 lanes per query, four or two queries per wave.)
-enum NearestShape : int { kShapeLane = 0, kShapeQuad = 1, kShapeWave = 2, kShapeGroup16 = 3, kShapeGroup32 = 4 };
+// (Group8 / 16 / 32: that many lanes per query; Group8 serves rays only.)
+enum NearestShape : int {
+    kShapeLane = 0, kShapeQuad = 1, kShapeWave = 2, kShapeGroup16 = 3, kShapeGroup32 = 4, kShapeGroup8 = 5
+};
+
+// Deepest binary tree the group walks take: their stacks have room for three entries on
+// each of 32 4-wide levels above what a round pushes.  Deeper trees (none of the builders
+// makes one from distinct boxes) go one lane per query, whose stack spills to scratch.
+constexpr int kGroupDepth = 64;
 
 // Tuned shapes.  The best shape depends on how long and how uneven the walks are, which
 // the query count alone does not tell: 262,144 closest queries on the terrain run fastest
@@ -2079,41 +2150,70 @@ struct TuneKey {
 static std::mutex gTuneMutex;
 static std::map<TuneKey, int> gTuned;
 
+// G lanes per ray, over the 4-wide nodes or, with a.wide false, the binary ones.
+template <int G, bool kSave, typename Nodes>
+static void launchRayGroupOn(Nodes nodes, int idCount, const TraverseArgs& a, const Ray* rays, int count,
+                             uint64_t* out, int* hitPrim, unsigned long long* stats, hipStream_t s) {
+    const Tri* tris = static_cast<const Tri*>(a.items);
+    const uint32_t idMask = stackIdMask(idCount);
+    const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
+    if (stats)
+        rayWaveKernel<G, true, kSave><<<grid, kBlock, 0, s>>>(nodes, tris, rays, a.order, count, out, stats, a.primIds, hitPrim, idMask);
+    else
+        rayWaveKernel<G, false, kSave><<<grid, kBlock, 0, s>>>(nodes, tris, rays, a.order, count, out, nullptr, a.primIds, hitPrim, idMask);
+}
+template <int G, bool kSave>
+static void launchRayGroup(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,
+                           unsigned long long* stats, hipStream_t s) {
+    if (a.wide)
+        launchRayGroupOn<G, kSave>(WideNodes{a.wideNodes}, a.wideCount, a, rays, count, out, hitPrim, stats, s);
+    else
+        launchRayGroupOn<G, kSave>(BinaryNodes{a.nodes}, a.nodeCount, a, rays, count, out, hitPrim, stats, s);
+}
+
 template <bool kSave>
 static void launchRayShape(int shape, const TraverseArgs& a, const Ray* rays, int count, uint64_t* out,
                            int* hitPrim, unsigned long long* stats, hipStream_t s) {
     const Tri* tris = static_cast<const Tri*>(a.items);
     if (shape == kShapeWave) {
-        const int grid = blocksFor(count, kBlock / 64);
-        const int idBits = stackIdBitsDev(a.wideCount);
-        if (stats)
-            rayWaveKernel<true, kSave><<<grid, kBlock, 0, s>>>(a.wideNodes, tris, rays, a.order, count, out, stats,
-                                                              a.primIds, hitPrim, idBits);
-        else
-            rayWaveKernel<false, kSave><<<grid, kBlock, 0, s>>>(a.wideNodes, tris, rays, a.order, count, out, nullptr,
-                                                               a.primIds, hitPrim, idBits);
+        launchRayGroup<64, kSave>(a, rays, count, out, hitPrim, stats, s);
+    } else if (shape == kShapeGroup32) {
+        launchRayGroup<32, kSave>(a, rays, count, out, hitPrim, stats, s);
+    } else if (shape == kShapeGroup16) {
+        launchRayGroup<16, kSave>(a, rays, count, out, hitPrim, stats, s);
+    } else if (shape == kShapeGroup8) {
+        launchRayGroup<8, kSave>(a, rays, count, out, hitPrim, stats, s);
     } else {
         const int grid = blocksFor(count, kBlock);
         if (stats)
             rayWideKernel<true, kSave><<<grid, kBlock, 0, s>>>(a.wideNodes, tris, rays, a.order, count, out, stats,
-                                                              a.primIds, hitPrim);
+                                                              a.primIds, hitPrim, stackIdMask(a.wideCount));
         else
             rayWideKernel<false, kSave><<<grid, kBlock, 0, s>>>(a.wideNodes, tris, rays, a.order, count, out,
-                                                               nullptr, a.primIds, hitPrim);
+                                                               nullptr, a.primIds, hitPrim, stackIdMask(a.wideCount));
     }
 }
 
-// Rays over 4-wide nodes run one lane or one wave per ray (same bits).  One lane per
-// ray unless mode 3 forces one wave or mode 4 tunes (the first call for a tree, save
-// flag and ray-count octave times both and keeps the faster): closest-hit walks are
-// short and prune well one lane at a time -- one wave per ray measured 1.3-5x slower
-// on the down rays, the city and the icosphere (0.44 vs 2.17 ms, 0.75 vs 2.52, 1.06
-// vs 3.04 for 1M rays).
+// Lanes per ray by the number of rays (same bits).  Small sets are latency chains that
+// more lanes shorten; at a million the lane kernel needs the fewest instructions on
+// coherent rays.  Measured (kernel us, city SAH tree, cosine rays, 4-wide: 1 / 8 / 16 / 32 /
+// 64 lanes): 1k 140 / - / 16 / 14 / 13, 4k 117 / 25 / 18 / 14 / 15, 16k - / - / 24 / 25 /
+// 35, 64k 168 / 51 / 51 / 71 / 111, 262k 187 / 128 / 155 / 250 / 409, 1M 477 / 430 / 561 /
+// 939 / 1511; straight down, 262k 107 / 101 / 151, 1M 242 / 326 / 534; around an
+// icosphere 64k 186 / 61 / 68, 262k 245 / 191 / 220.  Binary nodes cross over alike.  Mode
+// 1 forces one lane, mode 3 one wave; mode 4 times one lane against one wave on the first
+// call for a 4-wide tree, save flag and ray-count octave.
 template <bool kSave>
 static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,
                     hipStream_t s) {
-    if (gTraversalMode == 3) return kShapeWave;
-    if (gTraversalMode != 4) return kShapeLane;
+    if (a.depth > kGroupDepth || gTraversalMode == 1) return kShapeLane;
+    if (gTraversalMode == 3) return a.wide ? kShapeWave : kShapeLane;
+    if (gTraversalMode != 4 || !a.wide) {
+        if (count < 3072) return kShapeWave;
+        if (count < 12288) return kShapeGroup32;
+        if (count < 49152) return kShapeGroup16;
+        return count < 393216 ? kShapeGroup8 : kShapeLane;
+    }
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
     const TuneKey key{a.wideNodes, a.wideCount, 100 + (kSave ? 1 : 0), 0, octave};
@@ -2144,9 +2244,9 @@ static void launchRaysT(const TraverseArgs& a, const Ray* rays, int count, uint6
     const int grid = blocksFor(count, kBlock);
     if (grid == 0) return;
     const Tri* tris = static_cast<const Tri*>(a.items);
-    if (a.wide) {
-        launchRayShape<kSave>(rayShape<kSave>(a, rays, count, out, hitPrim, s), a, rays, count, out, hitPrim,
-                              a.stats, s);
+    const int shape = rayShape<kSave>(a, rays, count, out, hitPrim, s);
+    if (a.wide || shape != kShapeLane) {
+        launchRayShape<kSave>(shape, a, rays, count, out, hitPrim, a.stats, s);
     } else {
         if (a.stats)
             rayBinaryKernel<true, kSave><<<grid, kBlock, 0, s>>>(a.nodes, tris, rays, a.order, count, out, a.stats,
@@ -2231,17 +2331,26 @@ static int lanesPerQuery(int count, int k) {
     return k > 16 && lanes < 32 ? 32 : lanes;  // the list takes a lane per entry
 }
 
-// G lanes per query (64: one wave per query), k at most G.
+// G lanes per query (64: one wave per query), k at most G; over the 4-wide nodes or, with
+// a.wide false, the binary ones.
+template <typename L, bool kOne, int G, typename Nodes>
+static void launchGroupOn(Nodes nodes, int idCount, const TraverseArgs& a, const V3* pts, int count, int k,
+                          int outStride, ClosestResult* out, unsigned long long* stats, hipStream_t s) {
+    const auto* prims = static_cast<const typename L::Item*>(a.items);
+    const uint32_t idMask = stackIdMask(idCount);
+    const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
+    if (stats)
+        nearestWaveKernel<L, kOne, G, true><<<grid, kBlock, 0, s>>>(nodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idMask);
+    else
+        nearestWaveKernel<L, kOne, G, false><<<grid, kBlock, 0, s>>>(nodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idMask);
+}
 template <typename L, bool kOne, int G>
 static void launchGroup(const TraverseArgs& a, const V3* pts, int count, int k, int outStride, ClosestResult* out,
                         unsigned long long* stats, hipStream_t s) {
-    const auto* prims = static_cast<const typename L::Item*>(a.items);
-    const uint32_t idMask = stackIdMask(a.wideCount);
-    const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
-    if (stats)
-        nearestWaveKernel<L, kOne, G, true><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, stats, idMask);
+    if (a.wide)
+        launchGroupOn<L, kOne, G>(WideNodes{a.wideNodes}, a.wideCount, a, pts, count, k, outStride, out, stats, s);
     else
-        nearestWaveKernel<L, kOne, G, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idMask);
+        launchGroupOn<L, kOne, G>(BinaryNodes{a.nodes}, a.nodeCount, a, pts, count, k, outStride, out, stats, s);
 }
 
 template <typename L, int K>
@@ -2269,6 +2378,17 @@ static void launchShape(int shape, const TraverseArgs& a, const V3* pts, int cou
         else
             nearestWideKernel<L, K, false><<<grid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, k, outStride, out, nullptr, idBits);
     }
+}
+
+// Binary nodes: the group walk tests a node's grandchildren as if it were 4-wide.  One lane
+// per query is behind at every count measured for triangles and Gaussians (8,192-triangle
+// terrain closest 257 queries 675 us against 22, 100k 937 against 221, 400k 1150 against
+// 656; 262k Gaussians kNN8 100k 1527 against 480) and ahead for points, whose leaf test is
+// the cheapest, from about 131,072 queries (1M points closest 100k 215 us against 171, 400k
+// 344 against 591).
+template <typename L>
+static int binaryLaneFrom() {
+    return L::kKind == 1 ? 131072 : INT_MAX;
 }
 
 // The shape for a set of `count` queries by the measured crossovers (above).
@@ -2336,6 +2456,11 @@ template <typename L, int K>
 static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int k, int outStride,
                             ClosestResult* out, hipStream_t s) {
     const auto* prims = static_cast<const typename L::Item*>(a.items);
+    const bool deep = a.depth > kGroupDepth;
+    if (!a.wide && !deep && count < binaryLaneFrom<L>()) {
+        launchShape<L, K>(defaultShape<L, K>(count), a, pts, count, k, outStride, out, a.stats, s);
+        return;
+    }
     if (!a.wide) {
         const int grid = blocksFor(count, kBlock);
         if (a.stats)
@@ -2345,7 +2470,7 @@ static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int
         return;
     }
     int shape;
-    switch (gTraversalMode) {
+    switch (deep ? 1 : gTraversalMode) {
         case 1: shape = kShapeLane; break;
         case 2: shape = kShapeQuad; break;
         case 3: shape = kShapeWave; break;

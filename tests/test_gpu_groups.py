@@ -89,3 +89,74 @@ def test_batch_groups(A, orc, variant, nq, k):  # noqa: F811
         if b > a:
             want = orc.knn_brute(1, items[poff[s]:poff[s + 1]], q[a:b], k, threads=8)
             assert eq(got[a:b], want), s
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_binary_group_walk(A, orc, kind):  # noqa: F811
+    """Binary nodes (wide=False) at every group width, a leaf directly below the root included."""
+    for n, nq, k in ((2, 1, 1), (3, 5, 4), (300, 63, 7), (2000, 3073, 16), (2000, 12289, 0), (700, 65537, 2),
+                     (700, 33, 32)):
+        print(f"kind={kind} n={n} nq={nq} k={k}", flush=True)
+        items = scene(kind, n, n + nq)
+        q = np.random.default_rng(k).uniform(-40, 40, (nq, 3)).astype(np.float32)
+        for builder in (0, 1):
+            b = A.Bvh(kind, items, builder)
+            got = (b.knn(q, k, order=A.ORDER_INPUT) if k else b.closest(q, order=A.ORDER_MORTON))[0]
+            assert eq(got, orc.knn_brute(kind, items, q, k, threads=16)), (n, nq, k, builder)
+
+
+def unusual_rays(rng, items, n):
+    """Rays from everywhere to everywhere: some along the axes, some from inside with a
+    negative tMin, some with a short tMax."""
+    o = rng.uniform(-40, 40, (n, 3))
+    d = items.reshape(-1, 9)[rng.integers(0, items.shape[0], n), 0:3] - o + rng.normal(0, 1, (n, 3))
+    axis = rng.integers(0, 9, n)
+    for a in range(3):
+        d[axis == a] = 0.0
+        d[axis == a, a] = rng.choice([-1.0, 1.0], (axis == a).sum())
+    r = np.concatenate([o, d, np.full((n, 1), 1e-6), np.full((n, 1), np.inf)], 1).astype(np.float32)
+    r[::7, 6] = -50.0
+    r[::5, 7] = 1.0
+    return r
+
+
+# the counts at which the lanes per ray change, and one ray
+@pytest.mark.parametrize("count", [1, 3071, 3072, 12289, 49153, 393217])
+def test_ray_group_edges(A, orc, count):  # noqa: F811
+    import ctypes
+
+    print(f"rays={count}", flush=True)
+    rng = np.random.default_rng(count)
+    items = random_tris(rng, 400, size=8.0)
+    rays = unusual_rays(rng, items, count)
+    want = orc.ray_brute(items, rays, threads=16)
+    L = A.lib()
+    dr, res, hit = A.DeviceArray(rays), A.DeviceArray.empty(count, np.uint64), A.DeviceArray.empty(count, np.int32)
+    prims, ms = [], ctypes.c_double()
+    for builder in (0, 1):
+        b = A.Bvh(0, items, builder)
+        b.build_wide()
+        for wide in (0, 1):
+            assert eq(b.raycast(rays, order=A.ORDER_MORTON, wide=bool(wide))[0], want), (builder, wide)
+            A.check(L.qr_raycast_save_device(b.h, dr.ptr, count, res.ptr, hit.ptr, A.ORDER_INPUT, wide, ctypes.byref(ms)))
+            assert eq(res.download(), want), (builder, wide)
+            prims.append(hit.download())
+    assert all(eq(p, prims[0]) for p in prims)
+    assert eq(prims[0] >= 0, (want >> np.uint64(32)) != 0)
+
+
+def test_deep_tree(A, orc):  # noqa: F811
+    """A SAH tree deeper than the groups' stacks allow for keeps one lane per query."""
+    x = np.exp2(np.linspace(-120, 0, 30000))
+    items = np.zeros((x.size, 3), np.float32)
+    items[:, 0] = x
+    b = A.Bvh(1, items, A.BUILDER_SAH)
+    b.build_wide()
+    print("depth", b.info().depth, flush=True)
+    q = np.zeros((100, 3), np.float32)
+    q[:, 0] = np.exp2(np.linspace(-100, 1, 100))
+    for k in (0, 5):
+        want = orc.knn_brute(1, items, q, k, threads=8)
+        for wide in (False, True):
+            got = (b.knn(q, k, wide=wide) if k else b.closest(q, wide=wide))[0]
+            assert eq(got, want), (k, wide)
