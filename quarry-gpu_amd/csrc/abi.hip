@@ -49,50 +49,9 @@ struct qr_points {
     int rKeysGuess = 0;
 };
 
-// Result buffers handed to the caller: stream-ordered allocations from the device's
-// default pool, kept warm (release threshold raised once), so a radius call does not
-// stall the device at hipMalloc.  Freed on the null stream: calls are synchronous,
-// nothing still runs on them when the caller destroys the result.
-void warmDefaultPool() {
-    static thread_local int warmed = -1;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return;
-    if (warmed == dev) return;
-    hipMemPool_t pool;
-    if (hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess) {
-        uint64_t keep = UINT64_MAX;
-        (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-    }
-    (void)hipGetLastError();
-    warmed = dev;
-}
-
-template <typename T>
-struct AsyncBuf {
-    T* p = nullptr;
-    AsyncBuf() = default;
-    AsyncBuf(const AsyncBuf&) = delete;
-    AsyncBuf& operator=(const AsyncBuf&) = delete;
-    ~AsyncBuf() { release(); }
-    void alloc(size_t count, hipStream_t s) {
-        release();
-        warmDefaultPool();
-        const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&p), (count > 0 ? count : 1) * sizeof(T), s);
-        if (e != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
-            throw OomError(std::string("hipMallocAsync failed: ") + hipGetErrorString(e));
-        }
-    }
-    void release() {
-        if (p) (void)hipFreeAsync(p, nullptr);
-        p = nullptr;
-    }
-};
-
 struct qr_csr {
-    AsyncBuf<int> offsets;
-    AsyncBuf<uint64_t> keys;
+    DevBuf<int> offsets;
+    DevBuf<uint64_t> keys;
     int count = 0;
     int total = 0;
 };
@@ -162,6 +121,14 @@ namespace {
 thread_local std::string tLastError;
 thread_local qr_traversal_stats tRayStats{};
 thread_local qr_traversal_stats tQueryStats{};
+
+// Deletes a handle: one wait for the device, then all of its buffers.
+template <typename H>
+void destroyHandle(H* h) {
+    if (!h) return;
+    QuietFree quiet(hipDeviceSynchronize() == hipSuccess);
+    delete h;
+}
 
 template <typename F>
 int guard(F&& f) {
@@ -370,14 +337,18 @@ int qr_dev_alloc(size_t bytes, void** out) {
     return guard([&] {
         need(out != nullptr, "null output pointer");
         *out = nullptr;
-        hipCheck(hipMalloc(out, bytes > 0 ? bytes : 1), "hipMalloc");
+        *out = devAlloc(bytes);
     });
 }
 
 int qr_dev_free(void* ptr) {
     return guard([&] {
-        if (ptr) hipCheck(hipFree(ptr), "hipFree");
+        hipCheck(devFree(ptr), "hipFree");
     });
+}
+
+int qr_dev_trim(void) {
+    return guard([&] { devTrim(); });
 }
 
 int qr_dev_upload(void* dst, const void* src, size_t bytes) {
@@ -472,7 +443,7 @@ int qr_bvh_build_device(int prim, int builder, const void* items, int n, qr_buil
 }
 
 int qr_bvh_destroy(qr_bvh* bvh) {
-    return guard([&] { delete bvh; });
+    return guard([&] { destroyHandle(bvh); });
 }
 
 int qr_bvh_get_info(const qr_bvh* bvh, qr_bvh_info* out) {
@@ -840,7 +811,7 @@ int qr_rays_upload(const void* rays, int n, qr_rays** out) {
 }
 
 int qr_rays_destroy(qr_rays* r) {
-    return guard([&] { delete r; });
+    return guard([&] { destroyHandle(r); });
 }
 
 namespace {
@@ -893,8 +864,10 @@ int qr_raycast_device(const qr_bvh* bvh, const void* rays, int n, uint64_t* resu
                       int wide, double* ms) {
     return guard([&] {
         need(n >= 0, "negative ray count");
+        QuietFree quiet;
         qr_rays scratch;
         const double t = raycastImpl(bvh, static_cast<const Ray*>(rays), n, results, &scratch, 0, order, wide);
+        quiet.begin();  // (the call has waited for its kernels)
         if (ms) *ms = t;
     });
 }
@@ -904,9 +877,11 @@ int qr_raycast_save_device(const qr_bvh* bvh, const void* rays, int n, uint64_t*
     return guard([&] {
         need(n >= 0, "negative ray count");
         need(n == 0 || (rays && results && hitPrim), "null device pointer");
+        QuietFree quiet;
         qr_rays scratch;
         const double t =
             raycastImpl(bvh, static_cast<const Ray*>(rays), n, results, &scratch, 0, order, wide, hitPrim);
+        quiet.begin();
         if (ms) *ms = t;
     });
 }
@@ -1034,7 +1009,7 @@ int qr_batch_build(int prim, const void* items, const int* offsets, int scenes, 
 }
 
 int qr_batch_destroy(qr_batch* b) {
-    return guard([&] { delete b; });
+    return guard([&] { destroyHandle(b); });
 }
 
 int qr_batch_info(const qr_batch* b, int* scenes, int* total, int* maxDepth) {
@@ -1195,7 +1170,7 @@ int qr_batch_plan_config(const qr_batch_plan* p, int* variant, int* morton, doub
 }
 
 int qr_batch_plan_destroy(qr_batch_plan* p) {
-    return guard([&] { delete p; });
+    return guard([&] { destroyHandle(p); });
 }
 
 int qr_rays_summarize(const qr_rays* r, uint64_t* perRay, qr_ray_stats* out) {
@@ -1255,7 +1230,7 @@ int qr_points_upload(const float* pts, int n, int rpp, qr_points** out) {
 }
 
 int qr_points_destroy(qr_points* p) {
-    return guard([&] { delete p; });
+    return guard([&] { destroyHandle(p); });
 }
 
 int qr_points_info(const qr_points* p, int* count, int* stride) {
@@ -1323,9 +1298,11 @@ int qr_knn(const qr_bvh* bvh, qr_points* p, int k, int collectStats, int order, 
 int qr_closest_device(const qr_bvh* bvh, const float* pts, int n, void* results, int order, int wide,
                       double* ms) {
     return guard([&] {
+        QuietFree quiet;
         qr_points work;
         const double t = pointQuery(bvh, reinterpret_cast<const V3*>(pts), n, 0, 1,
                                     static_cast<ClosestResult*>(results), &work, 0, order, wide);
+        quiet.begin();
         if (ms) *ms = t;
     });
 }
@@ -1334,9 +1311,11 @@ int qr_knn_device(const qr_bvh* bvh, const float* pts, int n, int k, void* resul
                   int wide, double* ms) {
     return guard([&] {
         need(k >= 1 && k <= 32, "kNearestGPU: k must be in [1, 32]");
+        QuietFree quiet;
         qr_points work;
         const double t = pointQuery(bvh, reinterpret_cast<const V3*>(pts), n, k, k,
                                     static_cast<ClosestResult*>(results), &work, 0, order, wide);
+        quiet.begin();
         if (ms) *ms = t;
     });
 }
@@ -1429,7 +1408,7 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             const int n = p->count;
             res->count = n;
             hipStream_t s = currentStream();
-            res->offsets.alloc(static_cast<size_t>(n) + 1, s);
+            res->offsets.alloc(static_cast<size_t>(n) + 1);
             if (n <= 0 || radius < 0.0f) {
                 // Empty CSR: every segment is empty (the reference returns no hits for r < 0).
                 std::vector<int> zeros(static_cast<size_t>(n) + 1, 0);
@@ -1473,7 +1452,7 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             // and the compaction is redone below at the exact size.
             const int guess = captured ? p->rKeysGuess : 0;
             if (guess > 0) {
-                res->keys.alloc(static_cast<size_t>(guess), s);
+                res->keys.alloc(static_cast<size_t>(guess));
                 radiusCompact(counts, res->offsets.p, p->rCapture.p, n, cap, res->keys.p, guess, s);
             }
             hipCheck(hipStreamSynchronize(s), "radius total sync");
@@ -1482,7 +1461,7 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             if (total < 0 || maxSeg < 0) throw DeviceError("radius: summary words not written");
             res->total = total;
             const bool compacted = guess > 0 && total <= guess;
-            if (!compacted) res->keys.alloc(static_cast<size_t>(total > 0 ? total : 1), s);
+            if (!compacted) res->keys.alloc(static_cast<size_t>(total > 0 ? total : 1));
             p->rKeysGuess = total + total / 8 + 64;
             kev.record(2, s);
             if (total > 0) {
@@ -1539,7 +1518,7 @@ int qr_radius_read(const qr_csr* r, int* offsets, uint64_t* keys) {
 }
 
 int qr_radius_destroy(qr_csr* r) {
-    return guard([&] { delete r; });
+    return guard([&] { destroyHandle(r); });
 }
 
 int qr_last_query_stats(qr_traversal_stats* out) {

@@ -328,6 +328,7 @@ __global__ void adjRayKernel(const Tri* __restrict__ items, const int* __restric
 int saveClosestAux(BvhState& b, const float* pts, int n, const void* results, int* aux, hipStream_t s) {
     if (n <= 0) return 0;
     ensurePrimSlot(b, s);
+    QuietFree quiet;
     DevBuf<int> mism(1);
     hipCheck(hipMemsetAsync(mism.p, 0, sizeof(int), s), "aux clear");
     const int grid = blocksFor(n, kBlock);
@@ -351,6 +352,7 @@ int saveClosestAux(BvhState& b, const float* pts, int n, const void* results, in
     int h = 0;
     hipCheck(hipMemcpyAsync(&h, mism.p, sizeof(int), hipMemcpyDeviceToHost, s), "aux check");
     hipCheck(hipStreamSynchronize(s), "aux sync");
+    quiet.begin();
     return h;
 }
 

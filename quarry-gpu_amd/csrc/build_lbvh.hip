@@ -1665,6 +1665,7 @@ static void buildBatchT(BatchState& b, const typename L::Item* dSrc, hipStream_t
     b.depth.alloc(static_cast<size_t>(S));
     b.sceneId.alloc(static_cast<size_t>(n));
     b.ws.reserve(static_cast<size_t>(n));
+    QuietFree quiet;
     DevBuf<uint32_t> cb(static_cast<size_t>(S) * 6), codes(n), tmpA(n), tmpB(n), s2(n), order2(n), codes2(n),
         idxLocal(n);
     DevBuf<int> farEnd(static_cast<size_t>(n - S)), winOff(static_cast<size_t>(S) + 1);
@@ -1740,6 +1741,7 @@ static void buildBatchT(BatchState& b, const typename L::Item* dSrc, hipStream_t
     hipCheck(hipMemcpyAsync(d.data(), b.depth.p, sizeof(int) * d.size(), hipMemcpyDeviceToHost, s), "batch depth");
     ev.record(4, s);
     ev.sync(4);
+    quiet.begin();  // the work buffers' kernels are done
     b.maxDepth = 0;
     for (int v : d) b.maxDepth = v > b.maxDepth ? v : b.maxDepth;
     if (t) {

@@ -427,6 +427,7 @@ __global__ __launch_bounds__(kBlock) void batchWideEmitKernel(const Node2* __res
 void buildBatchWide(BatchState& b, hipStream_t s) {
     if (b.wideValid) return;
     const int nc = 2 * b.total - b.scenes;
+    QuietFree quiet;
     DevBuf<unsigned long long> jump(static_cast<size_t>(nc));
     DevBuf<int> depth(static_cast<size_t>(nc)), flags(static_cast<size_t>(nc)),
         scan(static_cast<size_t>(scanScratchInts(nc)) + 1);
@@ -449,6 +450,7 @@ void buildBatchWide(BatchState& b, hipStream_t s) {
                                                                        flags.p, b.wideId.p, b.wideRoot.p, b.wide.p);
     hipCheck(hipGetLastError(), "batch wide");
     hipCheck(hipStreamSynchronize(s), "batch wide sync");
+    quiet.begin();
     b.wideValid = true;
 }
 

@@ -73,6 +73,29 @@ void hipCheck(hipError_t e, const char* what);
 
 inline int blocksFor(long long n, int block) { return static_cast<int>((n + block - 1) / block); }
 
+// Device memory through a bounded cache of freed blocks (dev_pool.hip).  devFree waits for
+// the device before the block can be handed out again, unless the thread is inside a
+// QuietFree that has begun: the caller has then seen all work that touches the blocks it
+// frees finish.
+void* devAlloc(size_t bytes);
+hipError_t devFree(void* p);
+void devTrim();  // gives the current device's cached blocks back
+struct QuietFree {
+    QuietFree() = default;
+    explicit QuietFree(bool now) {
+        if (now) begin();
+    }
+    ~QuietFree();
+    QuietFree(const QuietFree&) = delete;
+    QuietFree& operator=(const QuietFree&) = delete;
+    // From here to the end of the scope (declare it before the buffers, whose destructors
+    // then run inside it, and begin once their work is done).
+    void begin();
+
+  private:
+    bool on = false;
+};
+
 // Plain device allocation owned by a scope (or a borrowed view of memory someone
 // else owns: borrow() makes release() forget the pointer instead of freeing it).
 template <typename T>
@@ -106,12 +129,7 @@ struct DevBuf {
         release();
         owned = true;
         if (count == 0) count = 1;
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(&p), count * sizeof(T));
-        if (e != hipSuccess) {
-            p = nullptr;
-            (void)hipGetLastError();
-            throw OomError(std::string("hipMalloc failed: ") + hipGetErrorString(e));
-        }
+        p = static_cast<T*>(devAlloc(count * sizeof(T)));
         n = count;
     }
     // Grows to at least count elements; contents are not preserved.  A buffer that
@@ -125,7 +143,7 @@ struct DevBuf {
         }
     }
     void release() {
-        if (p && owned) (void)hipFree(p);
+        if (p && owned) (void)devFree(p);
         p = nullptr;
         n = 0;
         owned = true;

@@ -97,6 +97,7 @@ def lib():
             "qr_set_stream": ([_vp], _ip),
             "qr_dev_alloc": ([ctypes.c_size_t, _vp], _ip),
             "qr_dev_free": ([_vp], _ip),
+            "qr_dev_trim": ([], _ip),
             "qr_dev_upload": ([_vp, _vp, ctypes.c_size_t], _ip),
             "qr_dev_download": ([_vp, _vp, ctypes.c_size_t], _ip),
             "qr_dev_synchronize": ([], _ip),

@@ -146,7 +146,7 @@ def test_ray_group_edges(A, orc, count):  # noqa: F811
 
 
 def test_deep_tree(A, orc):  # noqa: F811
-    """A SAH tree deeper than the groups' stacks allow for keeps one lane per query."""
+    """Exponentially spaced points: a SAH tree twice as deep as a balanced one."""
     x = np.exp2(np.linspace(-120, 0, 30000))
     items = np.zeros((x.size, 3), np.float32)
     items[:, 0] = x
