@@ -82,6 +82,7 @@ struct qr_batch_plan {
     qr_batch* batch = nullptr;
     const V3* points = nullptr;
     int n = 0, k = 1, stride = 1, scenes = 0;
+    int maxPerScene = 0;
     int variant = kBatchLds256;
     bool morton = true;
     double tunedMs = 0.0;
@@ -922,7 +923,8 @@ namespace {
 void enqueuePlan(qr_batch_plan& p, int variant, bool morton, hipStream_t s) {
     const BatchState& b = p.batch->s;
     launchBatchReset(p.counter.p, s);
-    if (morton)
+    if (morton && !batchQueryOrder(p.points, p.qOff.p, p.n, p.scenes, p.maxPerScene, p.ws, p.codes.p, p.tmpA.p,
+                                   p.order.p, s))
         batchMortonOrder(kPrimPoint, p.points, p.n, p.qScene.p, p.scenes, p.ws, p.cb.p, p.codes.p, p.tmpA.p,
                          p.tmpB.p, p.sceneSorted.p, p.order.p, s);
     BatchQueryArgs a;
@@ -944,10 +946,10 @@ void enqueuePlan(qr_batch_plan& p, int variant, bool morton, hipStream_t s) {
     launchBatchNearest(a, variant, s);
 }
 
-double timePlan(qr_batch_plan& p, int variant, bool morton) {
+double timePlan(qr_batch_plan& p, int variant, bool morton, int runs) {
     EventSet<2> ev;
     double best = 1e30;
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < runs; ++r) {
         ev.record(0, p.stream);
         enqueuePlan(p, variant, morton, p.stream);
         ev.record(1, p.stream);
@@ -1073,6 +1075,7 @@ int qr_batch_plan_create(qr_batch* b, const float* points, const int* qoffsets, 
             p->k = k;
             p->stride = k < 1 ? 1 : k;
             p->scenes = S;
+            for (int i = 0; i < S; ++i) p->maxPerScene = std::max(p->maxPerScene, qoffsets[i + 1] - qoffsets[i]);
             p->qOff.alloc(static_cast<size_t>(S) + 1);
             hipCheck(hipMemcpy(p->qOff.p, qoffsets, sizeof(int) * (static_cast<size_t>(S) + 1), hipMemcpyHostToDevice),
                      "query offsets");
@@ -1094,12 +1097,12 @@ int qr_batch_plan_create(qr_batch* b, const float* points, const int* qoffsets, 
                 bestV = (tune - 2) / 2;
                 bestM = ((tune - 2) % 2) != 0;
                 if (batchVariantWide(bestV)) buildBatchWide(b->s, p->stream);
-                best = timePlan(*p, bestV, bestM);
+                best = timePlan(*p, bestV, bestM, 1);  // nothing to choose: one run warms it
             } else if (tune == 1) {
                 buildBatchWide(b->s, p->stream);  // the 4-wide variants are candidates too
                 for (int v = 0; v < kBatchVariants; ++v)
                     for (int m = 0; m < 2; ++m) {
-                        const double ms = timePlan(*p, v, m != 0);
+                        const double ms = timePlan(*p, v, m != 0, 2);
                         if (ms < best) {
                             best = ms;
                             bestV = v;
@@ -1107,7 +1110,7 @@ int qr_batch_plan_create(qr_batch* b, const float* points, const int* qoffsets, 
                         }
                     }
             } else {
-                best = timePlan(*p, bestV, bestM);
+                best = timePlan(*p, bestV, bestM, 1);
             }
             p->variant = bestV;
             p->morton = bestM;

@@ -2005,9 +2005,13 @@ __global__ void pointBoundsInitKernel(uint32_t* __restrict__ bb) {
 }
 
 // Bounds of points laid out with `stride` floats per element (3 for points, 8 for
-// rays: origin first, 8 + 3 for ray directions).
+// rays: origin first, 8 + 3 for ray directions).  Every workgroup's six atomics meet at
+// the same six words, so there is one set per workgroup and at most kBoundsGrid of them
+// (one per wave of up to 1,024 workgroups: 262k points 73 us).
+constexpr int kBoundsGrid = 256;
 __global__ void pointBoundsKernel(const float* __restrict__ base, int stride, int count,
                                   uint32_t* __restrict__ bb) {
+    __shared__ uint32_t part[6][kBlock / 64];
     float lo0 = kInf, lo1 = kInf, lo2 = kInf, hi0 = -kInf, hi1 = -kInf, hi2 = -kInf;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < count; i += kBlock * gridDim.x) {
         const float* p = base + static_cast<size_t>(i) * stride;
@@ -2018,22 +2022,20 @@ __global__ void pointBoundsKernel(const float* __restrict__ base, int stride, in
         hi1 = fmaxf(hi1, p[1]);
         hi2 = fmaxf(hi2, p[2]);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        lo0 = fminf(lo0, __shfl_xor(lo0, off, 64));
-        lo1 = fminf(lo1, __shfl_xor(lo1, off, 64));
-        lo2 = fminf(lo2, __shfl_xor(lo2, off, 64));
-        hi0 = fmaxf(hi0, __shfl_xor(hi0, off, 64));
-        hi1 = fmaxf(hi1, __shfl_xor(hi1, off, 64));
-        hi2 = fmaxf(hi2, __shfl_xor(hi2, off, 64));
-    }
+    const uint32_t v[6] = {reduce64<MinU>(orderedBits(lo0)), reduce64<MinU>(orderedBits(lo1)),
+                           reduce64<MinU>(orderedBits(lo2)), reduce64<MaxU>(orderedBits(hi0)),
+                           reduce64<MaxU>(orderedBits(hi1)), reduce64<MaxU>(orderedBits(hi2))};
     if ((threadIdx.x & 63) == 0) {
-        atomicMin(&bb[0], orderedBits(lo0));
-        atomicMin(&bb[1], orderedBits(lo1));
-        atomicMin(&bb[2], orderedBits(lo2));
-        atomicMax(&bb[3], orderedBits(hi0));
-        atomicMax(&bb[4], orderedBits(hi1));
-        atomicMax(&bb[5], orderedBits(hi2));
+#pragma unroll
+        for (int k = 0; k < 6; ++k) part[k][threadIdx.x >> 6] = v[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        const int k = static_cast<int>(threadIdx.x);
+        uint32_t x = part[k][0];
+        for (int w = 1; w < kBlock / 64; ++w) x = k < 3 ? MinU::op(x, part[k][w]) : MaxU::op(x, part[k][w]);
+        if (k < 3) atomicMin(&bb[k], x);
+        else atomicMax(&bb[k], x);
     }
 }
 
@@ -2059,6 +2061,68 @@ __global__ void mortonKeysKernel(const float* __restrict__ base, int stride, int
         atomicAdd(&h[1][(code >> 8) & 255u], 1u);
         atomicAdd(&h[2][(code >> 16) & 255u], 1u);
         atomicAdd(&h[3][code >> 24], 1u);
+    }
+    __syncthreads();
+    flushHistogram(&h[0][0], 4 * 256, hist);
+}
+
+// Sort keys of a batch's queries, one workgroup per scene: the bounds of the scene's points,
+// then (scene, Morton code within those bounds) per point, and the digit counts.  Queries
+// lie scene by scene, so no pass has to look a point's scene up and the bounds need no
+// atomics.
+constexpr int kBatchKeysBlock = 1024;
+__global__ __launch_bounds__(kBatchKeysBlock) void batchQueryKeysKernel(const V3* __restrict__ points,
+                                                                        const int* __restrict__ qOff, int codeBits,
+                                                                        uint32_t* __restrict__ keys,
+                                                                        uint32_t* __restrict__ hist) {
+    __shared__ uint32_t part[6][kBatchKeysBlock / 64];
+    __shared__ uint32_t h[4][256];
+    const int sc = static_cast<int>(blockIdx.x);
+    const int begin = qOff[sc], end = qOff[sc + 1];
+    if (begin == end) return;  // the same for the whole workgroup
+    for (int i = threadIdx.x; i < 4 * 256; i += kBatchKeysBlock) (&h[0][0])[i] = 0u;
+    uint32_t v[6] = {~0u, ~0u, ~0u, 0u, 0u, 0u};
+    for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kBatchKeysBlock) {
+        const V3 p = points[i];
+        const uint32_t o[3] = {orderedBits(p.x), orderedBits(p.y), orderedBits(p.z)};
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            v[a] = MinU::op(v[a], o[a]);
+            v[3 + a] = MaxU::op(v[3 + a], o[a]);
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        v[a] = reduce64<MinU>(v[a]);
+        v[3 + a] = reduce64<MaxU>(v[3 + a]);
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) part[k][wave] = v[k];
+    }
+    __syncthreads();
+    float lo[3], hi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        uint32_t l = ~0u, u = 0u;
+        for (int w = 0; w < kBatchKeysBlock / 64; ++w) {
+            l = MinU::op(l, part[a][w]);
+            u = MaxU::op(u, part[3 + a][w]);
+        }
+        lo[a] = fromOrderedBits(l);
+        hi[a] = fromOrderedBits(u);
+    }
+    for (int i = begin + static_cast<int>(threadIdx.x); i < end; i += kBatchKeysBlock) {
+        const V3 p = points[i];
+        const uint32_t code = (spread10b(quant10(p.x, lo[0], hi[0])) | (spread10b(quant10(p.y, lo[1], hi[1])) << 1) |
+                               (spread10b(quant10(p.z, lo[2], hi[2])) << 2)) >> (30 - codeBits);
+        const uint32_t key = (static_cast<uint32_t>(sc) << codeBits) | code;
+        keys[i] = key;
+        atomicAdd(&h[0][key & 255u], 1u);
+        atomicAdd(&h[1][(key >> 8) & 255u], 1u);
+        atomicAdd(&h[2][(key >> 16) & 255u], 1u);
+        atomicAdd(&h[3][key >> 24], 1u);
     }
     __syncthreads();
     flushHistogram(&h[0][0], 4 * 256, hist);
@@ -2104,12 +2168,30 @@ void mortonOrder(const float* base, int stride, int count, int boxMode, SortWork
     if (grid > 1024) grid = 1024;
     if (boxMode == kBoxMeasure) {
         pointBoundsInitKernel<<<1, 64, 0, s>>>(bb);
-        pointBoundsKernel<<<grid, kBlock, 0, s>>>(base, stride, count, bb);
+        pointBoundsKernel<<<grid < kBoundsGrid ? grid : kBoundsGrid, kBlock, 0, s>>>(base, stride, count, bb);
     }
     mortonKeysKernel<<<grid, kBlock, 0, s>>>(base, stride, count, bb, boxMode == kBoxUnit ? 1 : 0, drop,
                                              keys, ws.hist.p);
     hipCheck(hipGetLastError(), "morton keys");
     sortPairs(ws, keys, nullptr, keysSorted, orderOut, static_cast<size_t>(count), passes, s);
+}
+
+bool batchQueryOrder(const V3* points, const int* qOff, int n, int scenes, int maxPerScene, SortWorkspace& ws,
+                     uint32_t* keys, uint32_t* keysSorted, uint32_t* order, hipStream_t s) {
+    if (maxPerScene > kBatchOrderMax) return false;
+    if (n <= 0) return true;
+    // the scene's bits and as much of the Morton code as whole digits leave room for: the
+    // order steers locality only
+    int sceneBits = 1;
+    while ((1LL << sceneBits) < scenes) ++sceneBits;
+    const int passes = sceneBits <= 12 ? 3 : 4;
+    const int codeBits = 8 * passes - sceneBits;
+    ws.reserve(static_cast<size_t>(n));
+    sortClear(ws, static_cast<size_t>(n), passes, s);
+    batchQueryKeysKernel<<<scenes, kBatchKeysBlock, 0, s>>>(points, qOff, codeBits, keys, ws.hist.p);
+    hipCheck(hipGetLastError(), "batch query keys");
+    sortPairs(ws, keys, nullptr, keysSorted, order, static_cast<size_t>(n), passes, s);
+    return true;
 }
 
 // 0 automatic, 1 one lane per query, 2 four lanes per query, 3 one wave per query,

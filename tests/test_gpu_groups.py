@@ -160,3 +160,27 @@ def test_deep_tree(A, orc):  # noqa: F811
         for wide in (False, True):
             got = (b.knn(q, k, wide=wide) if k else b.closest(q, wide=wide))[0]
             assert eq(got, want), (k, wide)
+
+
+# one workgroup orders a scene of up to 16,384 queries, the general order takes more; above
+# 4,096 scenes the keys need a fourth digit; scenes without queries are passed over
+@pytest.mark.parametrize("counts", [[16384, 0, 5], [16385, 5, 0], [0, 1, 3] * 1500])
+def test_batch_query_order(A, orc, counts):  # noqa: F811
+    print(f"scenes={len(counts)} most={max(counts)}", flush=True)
+    rng = np.random.default_rng(len(counts))
+    S = len(counts)
+    items = rng.uniform(-30, 30, (S, 3, 3)).astype(np.float32)
+    qoff = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    q = rng.uniform(-40, 40, (int(qoff[-1]), 3)).astype(np.float32)
+    batch = A.Batch(1, items.reshape(-1, 3), np.arange(0, 3 * S + 1, 3, dtype=np.int32))
+    got = []
+    for variant in ("lds64", "wide_lds64"):
+        plan = A.BatchPlan(batch, q, qoff, 2, tune=(A.BATCH_VARIANTS.index(variant), True))
+        for graph in (True, False, True):
+            plan.run(graph=graph)
+            got.append(plan.read())
+    assert all(eq(g, got[0]) for g in got)
+    for s in range(0, S, max(1, S // 40)):
+        a, b = qoff[s], qoff[s + 1]
+        if b > a:
+            assert eq(got[0][a:b], orc.knn_brute(1, items[s], q[a:b], 2, threads=8)), s
