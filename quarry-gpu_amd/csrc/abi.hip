@@ -1441,14 +1441,18 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             if (cap > 0) p->rCapture.reserve(static_cast<size_t>(n) * cap);
             int* counts = p->rCounts.p;
             int* scratch = p->rScratch.p;
-            zeroInts(p->rMax.p, kMaxCopies, s);
+            const bool small = n <= kRadiusOffsetsMax;  // (the offsets pass finds the largest count itself)
+            if (!small) zeroInts(p->rMax.p, kMaxCopies, s);
             kev.record(0, s);
-            const bool captured = launchRadiusCapture(a, p->pts.p, n, r2, counts, p->rCapture.p, cap, p->rMax.p, s);
+            const bool captured =
+                launchRadiusCapture(a, p->pts.p, n, r2, counts, p->rCapture.p, cap, small ? nullptr : p->rMax.p, s);
             kev.record(1, s);
-            scanExclusive(counts, res->offsets.p, n, res->offsets.p + n, scratch, s);
             int* hw = hostWords();
             hw[0] = hw[1] = -1;
-            radiusSummary(res->offsets.p + n, p->rMax.p, hostWordsDevice(), s);
+            if (!radiusOffsets(counts, n, res->offsets.p, hostWordsDevice(), s)) {
+                scanExclusive(counts, res->offsets.p, n, res->offsets.p + n, scratch, s);
+                radiusSummary(res->offsets.p + n, p->rMax.p, hostWordsDevice(), s);
+            }
             // Compaction before the total is known on the host, into keys sized by the
             // last call on these queries: the common case then needs no host round
             // trip in the middle of the call.  A short guess skips the segments past it
@@ -1471,13 +1475,14 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
                 a.stats = nullptr;
                 if (captured && !compacted)
                     radiusCompact(counts, res->offsets.p, p->rCapture.p, n, cap, res->keys.p, total, s);
-                // a second walk only for the queries the capture could not hold
+                // a second walk only for the queries the capture could not hold (binary
+                // nodes: for all)
                 if (!captured || maxSeg > cap)
-                    launchRadiusFill(a, p->pts.p, n, r2, counts, captured ? cap : 0, res->offsets.p, res->keys.p, s);
+                    launchRadiusFill(a, p->pts.p, n, r2, counts, captured && a.wide ? cap : 0, res->offsets.p,
+                                     res->keys.p, s);
             }
             kev.record(3, s);
-            // segments of at most 64 captured hits come sorted from the one-wave capture
-            const bool sorted = captured && maxSeg <= 64 && maxSeg <= cap && radiusCapturePresorts(a, n);
+            const bool sorted = captured && radiusCompactSorts(maxSeg, cap);
             if (total > 0 && !sorted) segmentSort(res->offsets.p, res->keys.p, n, maxSeg, scratch, s);
             ev.record(2, s);
             ev.sync(2);

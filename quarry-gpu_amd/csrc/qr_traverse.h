@@ -66,14 +66,18 @@ constexpr int kMaxCopies = 64;
 int radiusCaptureCap(int count);  // hits kept per query: 64, fewer for huge query sets
 bool launchRadiusCapture(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
                          uint64_t* capture, int cap, int* maxCount, hipStream_t s);
-// True when the capture runs one wave per query, which leaves every captured segment
-// of at most 64 hits sorted by (dist2, index).
-bool radiusCapturePresorts(const TraverseArgs& a, int count);
 // Writes the CSR segments of the queries the capture does not hold (all queries when
 // nothing was captured: cap 0); counts are those of the capture / count pass.
 void launchRadiusFill(const TraverseArgs& a, const V3* pts, int count, float r2, const int* counts,
                       int cap, const int* offsets, uint64_t* keys, hipStream_t s);
-// Copies the captured segments into the CSR keys.
+// Offsets of the segments, and the total and the largest count straight into hostDev[0] and
+// hostDev[1] (device view of pinned host words), in one launch; false, doing nothing, above
+// kRadiusOffsetsMax queries (scanExclusive and radiusSummary serve those).
+constexpr int kRadiusOffsetsMax = 32768;
+bool radiusOffsets(const int* counts, int n, int* offsets, int* hostDev, hipStream_t s);
+// Whether radiusCompact leaves every segment sorted when the largest has maxSeg hits.
+bool radiusCompactSorts(int maxSeg, int cap);
+// Moves the captured segments into the CSR keys, sorting them on the way.
 void radiusCompact(const int* counts, const int* offsets, const uint64_t* capture, int count, int cap,
                    uint64_t* keys, long long capacity, hipStream_t s);
 // Writes the total (*total) and the largest of the kMaxCopies per-query maxima to

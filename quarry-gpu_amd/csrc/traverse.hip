@@ -1163,169 +1163,13 @@ __device__ __forceinline__ void waveSortPairs(float& k, int& v, int lane, int wi
     }
 }
 
-// Radius capture with one wave per query, for query sets too small to fill the
-// device four lanes per query.  The wave's 16 quads expand up to 16 nodes of the
-// query's walk per round (quad j takes the j-th entry from the top of a stack shared
-// in LDS, lane s tests entry s of it); admitted interior children are pushed in lane
-// order, hits are written at the query's cursor in lane order.  The walk order does
-// not matter: the segment sort orders the hits by (dist2, index).  Stack bound: a
-// round pops w entries and pushes at most 4w, and w is held to
-// (kWaveStack - kWaveHeadroom - sp) / 3 (at least 1), so sp stays below
-// kWaveStack - kWaveHeadroom except while popping one entry per round, which adds at
-// most 3 per 4-wide level -- within the headroom for trees up to 32 levels deep
-// (the quad kernels' stack assumes the same depth).
+// LDS stack of the walks that give a query a group of lanes: entries per wave, split among
+// its queries.  A round pops w entries and pushes at most 4w, and w is held to
+// (stack - kWaveHeadroom - sp) / 3 (at least 1), so sp stays below stack - kWaveHeadroom
+// except while popping one entry per round, which adds at most 3 per 4-wide level -- within
+// the headroom for trees up to 32 levels deep (the quad kernels' stack assumes the same).
 constexpr int kWaveStack = 1024;
 constexpr int kWaveHeadroom = 3 * 32 + 4;
-
-// Bitonic sort by (dist2, index) of up to 64 pairs held two per lane by a group of
-// 32 lanes (lane l holds elements l and l + 32; empty elements are (inf, INT_MAX)).
-__device__ __forceinline__ void groupSort64x2(float& ak, int& av, float& bk, int& bv, int gl) {
-    for (int size = 2; size <= 64; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            if (stride == 32) {  // (size 64) elements l and l + 32 meet in the lane
-                if (closer(bk, bv, ak, av)) {
-                    const float tk = ak;
-                    const int tv = av;
-                    ak = bk;
-                    av = bv;
-                    bk = tk;
-                    bv = tv;
-                }
-                continue;
-            }
-            const float oak = waveXor(ak, stride), obk = waveXor(bk, stride);
-            const int oav = waveXor(av, stride), obv = waveXor(bv, stride);
-            const bool low = (gl & stride) == 0;
-            const bool upA = (gl & size) == 0 || size == 64;
-            const bool upB = ((gl + 32) & size) == 0 || size == 64;
-            const bool aOther = closer(oak, oav, ak, av), bOther = closer(obk, obv, bk, bv);
-            if ((low == upA) ? aOther : !aOther) {
-                ak = oak;
-                av = oav;
-            }
-            if ((low == upB) ? bOther : !bOther) {
-                bk = obk;
-                bv = obv;
-            }
-        }
-    }
-}
-
-// G lanes per query (G = 64: one wave; G = 32: two queries per wave, their groups'
-// ballots and shuffles masked to the group, the LDS stack split between them): the
-// group's quads expand up to G / 4 nodes of the walk per round.  A captured segment of
-// at most 64 hits is left sorted (over the group's lanes, two per lane above G = 32).
-template <typename L, bool kStats, int G>
-__global__ __launch_bounds__(kBlock) void radiusWaveKernel(
-    const Wide4* __restrict__ wide, const typename L::Item* __restrict__ prims,
-    const int* __restrict__ primIds, const V3* __restrict__ points, const uint32_t* __restrict__ order,
-    int count, float r2, int* __restrict__ counts, uint64_t* __restrict__ capture,
-    unsigned long long* __restrict__ stats, int* __restrict__ maxCount, int cap) {
-    static_assert(G == 32 || G == 64, "lanes per query");
-    constexpr int kPerWave = 64 / G;
-    constexpr int kQuads = G / 4;
-    constexpr int kStack = kWaveStack / kPerWave;
-    __shared__ int lds[kWaveStack * (kBlock / 64)];
-    const int lane = threadIdx.x & 63;
-    const int gl = lane & (G - 1);
-    const int gb = lane - gl;
-    const unsigned long long gmask = G == 64 ? ~0ull : ((1ull << G) - 1ull) << gb;
-    const int quad = gl >> 2;
-    const int slot = lane & 3;
-    const int qi = (xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6)) * kPerWave + lane / G;
-    const unsigned long long below = ((1ull << lane) - 1ull) & gmask;
-    int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
-    int queryHits = 0;
-    if (qi < count) {  // the same in the whole group
-        const int q = order ? static_cast<int>(order[qi]) : qi;
-        const V3 p = points[q];
-        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x >> 6) * kWaveStack + (lane / G) * kStack);
-        uint64_t* seg = capture + static_cast<long long>(q) * cap;
-        if (gl == 0) stk[0] = 0;
-        int sp = 1;
-        int found = 0;
-        while (sp > 0) {
-            int width = (kStack - kWaveHeadroom - sp) / 3;
-            width = width < 1 ? 1 : (width > kQuads ? kQuads : width);
-            const int take = width < sp ? width : sp;
-            const int node = quad < take ? stk[sp - 1 - quad] : -1;
-            sp -= take;
-            if (kStats && slot == 0 && node >= 0) ++opened;
-            WideEntry e{};
-            int ch = kWideEmpty;
-            if (node >= 0) {
-                e = wide[node].c[slot];
-                ch = e.child;
-            }
-            const bool leaf = ch < 0 && ch != kWideEmpty;
-            typename L::Item it;
-            int pid = 0;
-            if (leaf) {
-                it = prims[-ch - 1];
-                pid = primIds[-ch - 1];
-            }
-            const bool adm = ch != kWideEmpty && boxDist2(p, entryBox(e)) <= r2;
-            if (adm) ++nodeTests;
-            const bool push = adm && !leaf;
-            const unsigned long long pm = __ballot(push) & gmask;
-            const int pushes = __popcll(pm);
-            if (sp + pushes > kStack) {  // deeper than the bound above allows
-                if (gl == 0) overflow = 1;
-                break;
-            }
-            if (push) stk[sp + __popcll(pm & below)] = ch;
-            sp += pushes;
-            bool hit = false;
-            float d2 = 0.0f;
-            if (adm && leaf) {
-                ++leafTests;
-                d2 = L::dist2(p, it);
-                hit = d2 <= r2;
-            }
-            const unsigned long long hm = __ballot(hit) & gmask;
-            if (hit) {
-                const int at = found + __popcll(hm & below);
-                if (at < cap) seg[at] = (static_cast<uint64_t>(floatBits(d2)) << 32) | static_cast<uint32_t>(pid);
-            }
-            found += __popcll(hm);
-        }
-        if (found > 1 && found <= G && found <= cap) {
-            // a segment of at most G hits leaves sorted by (dist2, index): the order
-            // of the 64-bit keys, dist2 being non-negative
-            int w = 2;
-            while (w < found) w <<= 1;
-            float sk = kInf;
-            int sv = 0x7fffffff;
-            if (gl < found) {
-                const uint64_t key = seg[gl];
-                sk = bitsFloat(static_cast<uint32_t>(key >> 32));
-                sv = static_cast<int>(static_cast<uint32_t>(key));
-            }
-            waveSortPairs(sk, sv, lane, w);
-            if (gl < found) seg[gl] = (static_cast<uint64_t>(floatBits(sk)) << 32) | static_cast<uint32_t>(sv);
-        } else if (G == 32 && found > G && found <= 64 && found <= cap) {
-            float ak = kInf, bk = kInf;
-            int av = 0x7fffffff, bv = 0x7fffffff;
-            {
-                const uint64_t key = seg[gl];
-                ak = bitsFloat(static_cast<uint32_t>(key >> 32));
-                av = static_cast<int>(static_cast<uint32_t>(key));
-            }
-            if (gl + 32 < found) {
-                const uint64_t key = seg[gl + 32];
-                bk = bitsFloat(static_cast<uint32_t>(key >> 32));
-                bv = static_cast<int>(static_cast<uint32_t>(key));
-            }
-            groupSort64x2(ak, av, bk, bv, gl);
-            seg[gl] = (static_cast<uint64_t>(floatBits(ak)) << 32) | static_cast<uint32_t>(av);
-            if (gl + 32 < found) seg[gl + 32] = (static_cast<uint64_t>(floatBits(bk)) << 32) | static_cast<uint32_t>(bv);
-        }
-        if (gl == 0) counts[q] = found;
-        queryHits = found;
-    }
-    waveMaxAtomic(maxCount, queryHits);
-    flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
-}
 
 // ---- steps of a group of G lanes (16, 32 or 64, aligned within the wave) ----------------
 // A group works on one query; the groups of a wave run the same instructions, so the
@@ -1645,6 +1489,87 @@ __global__ __launch_bounds__(kBlock) void nearestWaveKernel(
     flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
 }
 
+// Radius capture of one query by a group of G lanes (the layout above): every admitted
+// interior child goes on the stack in lane order, hits are counted and the first `cap` of
+// them kept in the query's slot of `capture`, in no particular order (radiusCompactKernel
+// sorts each segment as it moves it).
+template <typename L, bool kStats, int G, typename Nodes>
+__global__ __launch_bounds__(kBlock) void radiusGroupKernel(
+    Nodes nodes, const typename L::Item* __restrict__ prims, const int* __restrict__ primIds,
+    const V3* __restrict__ points, const uint32_t* __restrict__ order, int count, float r2,
+    int* __restrict__ counts, uint64_t* __restrict__ capture, unsigned long long* __restrict__ stats,
+    int* __restrict__ maxCount, int cap) {
+    constexpr int kQuads = G / 4;
+    constexpr int kStack = kWaveStack / (64 / G);
+    __shared__ int lds[kWaveStack * (kBlock / 64)];
+    const int lane = threadIdx.x & 63;
+    const int gl = lane & (G - 1);
+    const int quad = gl >> 2;
+    const int slot = lane & 3;
+    const int qi = (xcdBlock() * (kBlock / 64) + (threadIdx.x >> 6)) * (64 / G) + lane / G;
+    int nodeTests = 0, leafTests = 0, overflow = 0, opened = 0;
+    int found = 0;
+    if (qi < count) {  // the same in the whole group
+        const int q = order ? static_cast<int>(order[qi]) : qi;
+        const V3 p = points[q];
+        GroupBits<G> gb;
+        gb.init(lane);
+        LdsInt* stk = (LdsInt*)(lds + (threadIdx.x / G) * kStack);
+        uint64_t* seg = capture + static_cast<long long>(q) * cap;
+        if (gl == 0) stk[0] = 0;
+        int sp = 1;
+        while (sp > 0) {
+            const int room = kStack - kWaveHeadroom - sp;
+            int take = kQuads;
+            if (room < 3 * kQuads) take = room < 3 ? 1 : room / 3;
+            take = take < sp ? take : sp;
+            int node = -1;
+            if (quad < take) node = stk[sp - 1 - quad];
+            sp -= take;
+            if (kStats && slot == 0 && node >= 0) ++opened;
+            Box box{{0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+            int ch = kWideEmpty;
+            if (node >= 0) ch = nodes.entry(node, slot, box);
+            const bool leaf = static_cast<uint32_t>(ch) > static_cast<uint32_t>(kWideEmpty);
+            const bool adm = (ch != kWideEmpty) & (boxDist2(p, box) <= r2);
+            if (kStats && adm) ++nodeTests;
+            const bool push = adm & !leaf;
+            const unsigned long long pb = __ballot(push);
+            if (pb != 0) {
+                const typename GroupBits<G>::Word pm = gb.of(pb);
+                const int pushes = gb.count(pm);
+                if (sp + pushes > kStack) {  // deeper than the stack bound allows
+                    if (gl == 0) overflow = 1;
+                    break;
+                }
+                if (push) stk[sp + gb.count(pm & gb.lower)] = ch;
+                sp += pushes;
+            }
+            bool hit = false;
+            float d2 = 0.0f;
+            uint32_t pid = 0;
+            if (adm & leaf) {
+                if (kStats) ++leafTests;
+                pid = static_cast<uint32_t>(primIds[-ch - 1]);
+                d2 = L::dist2(p, prims[-ch - 1]);
+                hit = d2 <= r2;
+            }
+            const unsigned long long hb = __ballot(hit);
+            if (hb != 0) {
+                const typename GroupBits<G>::Word hm = gb.of(hb);
+                if (hit) {
+                    const int at = found + gb.count(hm & gb.lower);
+                    if (at < cap) seg[at] = (static_cast<uint64_t>(floatBits(d2)) << 32) | pid;
+                }
+                found += gb.count(hm);
+            }
+        }
+        if (gl == 0) counts[q] = found;
+    }
+    waveMaxAtomic(maxCount, found);
+    flushStats<kStats>(stats, nodeTests, leafTests, overflow, opened);
+}
+
 // Batched scenes by groups: G lanes walk one query of the batch's queue on its own
 // scene's 4-wide tree (scene s: items from primOff[s], nodes from wideRoot[s]).  Queries
 // lie scene by scene, so an XCD's contiguous range stays on a few scenes' nodes.
@@ -1876,29 +1801,52 @@ __global__ __launch_bounds__(kBlock) void radiusKernel(
 constexpr int kWaveCap = 256;
 constexpr int kBlockCap = 8192;
 
-__device__ __forceinline__ void bitonicLds(uint64_t* buf, int cap, int lane, int lanes,
-                                           bool blockSync) {
+// Bitonic sort of cap (a power of two, at least 4) keys in LDS by `lanes` threads (a wave,
+// or a whole workgroup), ascending.  A chain of LDS round trips: a round therefore does two
+// steps, strides 2 h and h, on four keys in registers (the last stride alone when their
+// number is odd), and a thread's four loads are in flight together -- about 30 rounds for
+// 1,024 keys instead of 55.  A wave's 64 consecutive quads lie in 256 consecutive keys
+// while h <= 64, so only rounds of longer strides and the round after them need the
+// workgroup's barrier; within a wave LDS accesses run in order (the fence keeps the
+// compiler to it).
+__device__ __forceinline__ void orderKeys(uint64_t& a, uint64_t& b, bool up) {
+    const bool swap = (a > b) == up;  // (equal keys: either way)
+    const uint64_t x = swap ? b : a, y = swap ? a : b;
+    a = x;
+    b = y;
+}
+__device__ __forceinline__ void bitonicLds(uint64_t* buf, int cap, int lane, int lanes) {
+    bool far = false;  // the round before reached across waves
     for (int size = 2; size <= cap; size <<= 1) {
-        for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int i = lane; i < cap; i += lanes) {
-                const int partner = i ^ stride;
-                if (partner > i) {
-                    const uint64_t a = buf[i];
-                    const uint64_t b = buf[partner];
-                    const bool up = (i & size) == 0;
-                    if (up ? (a > b) : (a < b)) {
-                        buf[i] = b;
-                        buf[partner] = a;
-                    }
+        int stride = size >> 1;
+        while (stride > 0) {
+            const bool two = stride > 1;
+            const int h = two ? stride >> 1 : 1;
+            const bool reach = h > 64;
+            if (lanes > 64 && (reach || far)) __syncthreads();
+            else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            far = reach;
+            for (int p = lane; p < cap >> 2; p += lanes) {
+                const int i = ((p & ~(h - 1)) << 2) | (p & (h - 1));
+                uint64_t k0 = buf[i], k1 = buf[i + h], k2 = buf[i + 2 * h], k3 = buf[i + 3 * h];
+                const bool up = (i & size) == 0 || size == cap;
+                const bool up2 = ((i + 2 * h) & size) == 0 || size == cap;  // (differs at size 2 only)
+                if (two) {
+                    orderKeys(k0, k2, up);
+                    orderKeys(k1, k3, up);
                 }
+                orderKeys(k0, k1, up);
+                orderKeys(k2, k3, up2);
+                buf[i] = k0;
+                buf[i + h] = k1;
+                buf[i + 2 * h] = k2;
+                buf[i + 3 * h] = k3;
             }
-            if (blockSync) {
-                __syncthreads();
-            } else {
-                __builtin_amdgcn_wave_barrier();
-            }
+            stride >>= two ? 2 : 1;
         }
     }
+    if (lanes > 64) __syncthreads();
+    else __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 __global__ __launch_bounds__(kBlock) void segSortWaveKernel(const int* __restrict__ offsets,
@@ -1912,12 +1860,12 @@ __global__ __launch_bounds__(kBlock) void segSortWaveKernel(const int* __restric
     const int begin = offsets[seg];
     const int m = offsets[seg + 1] - begin;
     if (m <= 1 || m > kWaveCap) return;
-    int cap = 2;
+    int cap = 4;
     while (cap < m) cap <<= 1;
     uint64_t* buf = smem[w];
     for (int i = lane; i < cap; i += 64) buf[i] = i < m ? keys[begin + i] : ~0ull;
     __builtin_amdgcn_wave_barrier();
-    bitonicLds(buf, cap, lane, 64, false);
+    bitonicLds(buf, cap, lane, 64);
     for (int i = lane; i < m; i += 64) keys[begin + i] = buf[i];
 }
 
@@ -1937,7 +1885,7 @@ __global__ __launch_bounds__(kBlock) void segSortBlockKernel(const int* __restri
         while (cap < m) cap <<= 1;
         for (int i = threadIdx.x; i < cap; i += kBlock) dyn[i] = i < m ? keys[begin + i] : ~0ull;
         __syncthreads();
-        bitonicLds(dyn, cap, threadIdx.x, kBlock, true);
+        bitonicLds(dyn, cap, threadIdx.x, kBlock);
         for (int i = threadIdx.x; i < m; i += kBlock) keys[begin + i] = dyn[i];
         __syncthreads();
     }
@@ -2391,9 +2339,6 @@ void checkOverflow() {
                       "so some results are incomplete");
 }
 
-// Radius capture one wave per query below this many queries, four lanes per query
-// above (traversal mode 2 forces four lanes per query).
-int gRadiusWaveBelow = 1 << 17;
 
 // Lanes per closest / kNN query (64, 32 or 16) by the number of queries.  A small set
 // fills the device only with more lanes per query; a large one is served with the fewest
@@ -2606,11 +2551,9 @@ void launchKnn(const TraverseArgs& a, const V3* pts, int count, int k, int outSt
     launchNearest(a, pts, count, k, outStride, out, s);
 }
 
-// Radius on four lanes per query measured faster at every query count from 20k to
-// 1M on the 2M-triangle terrain (the lanes of a quad test the four children of a
-// node and its leaves together instead of walking them one after another); it
-// serves 4-wide trees unless one lane per query is forced.
-static bool radiusOnQuads(const TraverseArgs& a) { return a.wide && gTraversalMode != 1; }
+// Whether a radius call captures its hits in one walk (by groups of lanes, or on quads):
+// unless one lane per query is forced or the tree is deeper than those walks' stacks take.
+static bool radiusCaptures(const TraverseArgs& a) { return gTraversalMode != 1 && a.depth <= kGroupDepth; }
 
 // cap > 0: a fill on quads after a capture (only the queries the capture could not
 // hold are walked); cap == 0: the per-lane count / fill kernels.
@@ -2636,30 +2579,57 @@ static void launchRadiusT(const TraverseArgs& a, const V3* pts, int count, float
     }
 }
 
+// Lanes per radius query (4: the quad kernel, when mode 2 forces it).  Measured (kernel us at
+// 64 / 32 / 16 / 4 lanes): 1M points r = 1, 5k 29 / 44 / 76 / 333, 20k 56 / 66 / 100 / 398,
+// 60k 586 / 466 / 440 / 686, 400k 2326 / 1389 / 966 / 950; the 2M-triangle terrain r = 2,
+// 20k 31 / 28 / 29 / 74, 100k 131 / 98 / 75 / 86, 400k 453 / 324 / 222 / 214; 262k
+// Gaussians 20k 117 / 108 / 121 / 290, 131k 707 / 471 / 504 / 788.
+static int radiusLanes(int count) {
+    if (gTraversalMode == 2) return 4;
+    if (gTraversalMode == 3) return 64;
+    if (gTraversalMode == 6) return 32;
+    return count < 16384 ? 64 : (count < 40960 ? 32 : 16);
+}
+
+template <typename L, int G, typename Nodes>
+static void launchCaptureGroup(Nodes nodes, const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
+                               uint64_t* capture, int cap, int* maxCount, hipStream_t s) {
+    const auto* prims = static_cast<const typename L::Item*>(a.items);
+    const int grid = blocksFor(count, (kBlock / 64) * (64 / G));
+    if (a.stats)
+        radiusGroupKernel<L, true, G><<<grid, kBlock, 0, s>>>(nodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, a.stats, maxCount, cap);
+    else
+        radiusGroupKernel<L, false, G><<<grid, kBlock, 0, s>>>(nodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, nullptr, maxCount, cap);
+}
+
+template <typename L, int G>
+static void launchCaptureOn(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
+                            uint64_t* capture, int cap, int* maxCount, hipStream_t s) {
+    if (a.wide)
+        launchCaptureGroup<L, G>(WideNodes{a.wideNodes}, a, pts, count, r2, counts, capture, cap, maxCount, s);
+    else
+        launchCaptureGroup<L, G>(BinaryNodes{a.nodes}, a, pts, count, r2, counts, capture, cap, maxCount, s);
+}
+
 template <typename L>
 static void launchCaptureT(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
                            uint64_t* capture, int cap, int* maxCount, hipStream_t s) {
+    const int lanes = radiusLanes(count);
+    if (lanes == 64) {
+        launchCaptureOn<L, 64>(a, pts, count, r2, counts, capture, cap, maxCount, s);
+        return;
+    }
+    if (lanes == 32) {
+        launchCaptureOn<L, 32>(a, pts, count, r2, counts, capture, cap, maxCount, s);
+        return;
+    }
+    if (lanes == 16 || !a.wide) {
+        launchCaptureOn<L, 16>(a, pts, count, r2, counts, capture, cap, maxCount, s);
+        return;
+    }
     const int qgrid = blocksFor(4LL * count, kBlock);
     const auto* prims = static_cast<const typename L::Item*>(a.items);
-    // below gRadiusWaveBelow two queries per wave (measured ahead of one per wave at
-    // every count tried: terrain r = 2 at 20k-115k queries 0.045-0.127 ms against
-    // 0.049-0.161, the 1M-point cloud r = 1 at 20k / 65k 0.106 / 0.605 against
-    // 0.124 / 0.745; its segments of up to 64 hits leave sorted, so the quads' segment
-    // sort is not needed either); mode 3 forces one wave per query
-    if ((count < gRadiusWaveBelow && (gTraversalMode == 0 || gTraversalMode == 4 || gTraversalMode == 5)) ||
-        gTraversalMode == 6) {
-        const int wgrid = blocksFor(count, 2 * (kBlock / 64));
-        if (a.stats)
-            radiusWaveKernel<L, true, 32><<<wgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, a.stats, maxCount, cap);
-        else
-            radiusWaveKernel<L, false, 32><<<wgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, nullptr, maxCount, cap);
-    } else if (gTraversalMode == 3) {
-        const int wgrid = blocksFor(count, kBlock / 64);
-        if (a.stats)
-            radiusWaveKernel<L, true, 64><<<wgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, a.stats, maxCount, cap);
-        else
-            radiusWaveKernel<L, false, 64><<<wgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, capture, nullptr, maxCount, cap);
-    } else if (a.stats)
+    if (a.stats)
         radiusQuadKernel<L, kRadiusCaptureMode, true><<<qgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, nullptr, capture, a.stats, maxCount, cap);
     else
         radiusQuadKernel<L, kRadiusCaptureMode, false><<<qgrid, kBlock, 0, s>>>(a.wideNodes, prims, a.primIds, pts, a.order, count, r2, counts, nullptr, capture, nullptr, maxCount, cap);
@@ -2679,16 +2649,10 @@ int radiusCaptureCap(int count) {
     return tight < 8 ? 0 : static_cast<int>(tight);
 }
 
-bool radiusCapturePresorts(const TraverseArgs& a, int count) {
-    return radiusOnQuads(a) &&
-           ((count < gRadiusWaveBelow && (gTraversalMode == 0 || gTraversalMode == 4 || gTraversalMode == 5)) ||
-            gTraversalMode == 3 || gTraversalMode == 6);
-}
-
 bool launchRadiusCapture(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
                          uint64_t* capture, int cap, int* maxCount, hipStream_t s) {
     if (count <= 0) return false;
-    if (!radiusOnQuads(a) || cap <= 0) {
+    if (!radiusCaptures(a) || cap <= 0) {
         switch (a.kind) {
             case 0: launchRadiusT<TriLeaf, false>(a, pts, count, r2, counts, nullptr, nullptr, maxCount, 0, s); break;
             case 1: launchRadiusT<PointLeaf, false>(a, pts, count, r2, counts, nullptr, nullptr, maxCount, 0, s); break;
@@ -2719,21 +2683,63 @@ void launchRadiusFill(const TraverseArgs& a, const V3* pts, int count, float r2,
 }
 
 namespace {
-// One wave per query copies its captured hits (queries with more than `cap` hits are
-// left to the fill walk); a segment that would end past `capacity` keys is skipped
-// (the caller compacts again into a buffer of the exact size).
-__global__ void radiusCompactKernel(const int* __restrict__ counts, const int* __restrict__ offsets,
-                                    const uint64_t* __restrict__ capture, int count, int cap,
-                                    uint64_t* __restrict__ keys, long long capacity) {
-    const long long q = static_cast<long long>(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6);
-    if (q >= count) return;
-    const int c = counts[q];
-    if (c > cap) return;
-    const long long off = offsets[q];
-    if (off + c > capacity) return;
+// Moves the captured hits into the result, each segment sorted by (dist2, index) -- the
+// order of the 64-bit keys, dist2 being non-negative.  A workgroup serves four queries:
+// segments of up to 64 hits in one wave's registers (a hit per lane), then the longer ones
+// one after another by the whole workgroup through a bitonic network in LDS (one wave
+// alone took 100 us over the longest of them); beyond kCompactSort they move as they are.
+// Queries with more than `cap` hits are left to the fill walk; a segment that would end
+// past `capacity` keys is skipped (the caller moves again into a buffer of the exact size).
+// Sorting here takes the place of a pass over all segments and of three launches for the
+// long ones: 20k segments of 16 hits on average, 2 % above 64 and up to 566 long, took
+// 84 us in those launches and take 31 here.
+constexpr int kCompactSort = 2048;
+__global__ __launch_bounds__(kBlock) void radiusCompactKernel(const int* __restrict__ counts,
+                                                              const int* __restrict__ offsets,
+                                                              const uint64_t* __restrict__ capture, int count,
+                                                              int cap, uint64_t* __restrict__ keys,
+                                                              long long capacity) {
+    constexpr int kWaves = kBlock / 64;
+    __shared__ uint64_t buf[kCompactSort];
+    __shared__ int longCount[kWaves];  // the wave's segment, when the workgroup is to sort it
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const long long first = static_cast<long long>(blockIdx.x) * kWaves;
+    const long long q = first + wave;
+    int c = q < count ? counts[q] : 0;
+    const long long off = c > 0 ? offsets[q] : 0;
+    if (c > cap || off + c > capacity) c = 0;
+    if (lane == 0) longCount[wave] = c > 64 && c <= kCompactSort ? c : 0;
     const uint64_t* src = capture + q * cap;
     uint64_t* dst = keys + off;
-    for (int j = threadIdx.x & 63; j < c; j += 64) dst[j] = src[j];
+    if (c <= 64) {
+        float d = kInf;
+        int id = 0x7fffffff;
+        if (lane < c) {
+            const uint64_t k = src[lane];
+            d = bitsFloat(static_cast<uint32_t>(k >> 32));
+            id = static_cast<int>(static_cast<uint32_t>(k));
+        }
+        int w = 2;
+        while (w < c) w <<= 1;
+        if (c > 1) waveSortPairs(d, id, lane, w);
+        if (lane < c) dst[lane] = (static_cast<uint64_t>(floatBits(d)) << 32) | static_cast<uint32_t>(id);
+    } else if (c > kCompactSort) {
+        for (int j = lane; j < c; j += 64) dst[j] = src[j];
+    }
+    __syncthreads();
+    for (int s = 0; s < kWaves; ++s) {
+        const int m = longCount[s];  // the same in every thread
+        if (m == 0) continue;
+        const uint64_t* from = capture + (first + s) * cap;
+        uint64_t* to = keys + offsets[first + s];
+        int w = 128;
+        while (w < m) w <<= 1;
+        for (int j = threadIdx.x; j < w; j += kBlock) buf[j] = j < m ? from[j] : ~0ull;
+        __syncthreads();
+        bitonicLds(buf, w, threadIdx.x, kBlock);
+        for (int j = threadIdx.x; j < m; j += kBlock) to[j] = buf[j];
+        __syncthreads();
+    }
 }
 
 // The radius call's two host-side figures in one step: the total hit count and the
@@ -2761,6 +2767,93 @@ void radiusCompact(const int* counts, const int* offsets, const uint64_t* captur
     radiusCompactKernel<<<blocksFor(count, kBlock / 64), kBlock, 0, s>>>(counts, offsets, capture, count, cap,
                                                                         keys, capacity);
     hipCheck(hipGetLastError(), "radius compact");
+}
+
+bool radiusCompactSorts(int maxSeg, int cap) { return maxSeg <= cap && maxSeg <= kCompactSort; }
+
+// Offsets, total and largest count of a small query set in one workgroup: thread t takes
+// a run of up to kOffsetsRun counts (a multiple of four: 16-byte loads, all in flight at
+// once, kept in registers for the second use), the workgroup scans the runs' sums.
+namespace {
+constexpr int kOffsetsBlock = 1024, kOffsetsRun = kRadiusOffsetsMax / kOffsetsBlock;
+static_assert(kOffsetsRun % 4 == 0, "runs of int4");
+__global__ __launch_bounds__(kOffsetsBlock) void radiusOffsetsKernel(const int* __restrict__ counts, int n, int run,
+                                                                     int* __restrict__ offsets,
+                                                                     int* __restrict__ host) {
+    __shared__ int sums[kOffsetsBlock / 64], most[kOffsetsBlock / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int begin = static_cast<int>(threadIdx.x) * run;
+    int4 c[kOffsetsRun / 4];
+    int sum = 0, big = 0;
+#pragma unroll
+    for (int k = 0; k < kOffsetsRun / 4; ++k) {
+        const int i = begin + 4 * k;
+        c[k] = {0, 0, 0, 0};
+        if (4 * k < run) {
+            if (i + 3 < n) {
+                c[k] = *reinterpret_cast<const int4*>(counts + i);
+            } else {
+                if (i < n) c[k].x = counts[i];
+                if (i + 1 < n) c[k].y = counts[i + 1];
+                if (i + 2 < n) c[k].z = counts[i + 2];
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kOffsetsRun / 4; ++k) {
+        sum += c[k].x + c[k].y + c[k].z + c[k].w;
+        const int a = c[k].x > c[k].y ? c[k].x : c[k].y, b = c[k].z > c[k].w ? c[k].z : c[k].w;
+        big = a > big ? a : big;
+        big = b > big ? b : big;
+    }
+    int x = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+        const int o = __shfl_xor(big, off, 64);
+        big = o > big ? o : big;
+    }
+    if (lane == 63) {
+        sums[wave] = x;
+        most[wave] = big;
+    }
+    __syncthreads();
+    int at = x - sum, total = 0;
+    for (int w = 0; w < kOffsetsBlock / 64; ++w) {
+        at += w < wave ? sums[w] : 0;
+        total += sums[w];
+        big = most[w] > big ? most[w] : big;
+    }
+#pragma unroll
+    for (int k = 0; k < kOffsetsRun / 4; ++k) {
+        const int i = begin + 4 * k;
+        const int4 o = {at, at + c[k].x, at + c[k].x + c[k].y, at + c[k].x + c[k].y + c[k].z};
+        if (4 * k < run) {
+            if (i + 3 < n) {
+                *reinterpret_cast<int4*>(offsets + i) = o;
+            } else {
+                if (i < n) offsets[i] = o.x;
+                if (i + 1 < n) offsets[i + 1] = o.y;
+                if (i + 2 < n) offsets[i + 2] = o.z;
+            }
+        }
+        at = o.w + c[k].w;
+    }
+    if (threadIdx.x == 0) {
+        offsets[n] = total;
+        __hip_atomic_store(&host[0], total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&host[1], big, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+}  // namespace
+
+bool radiusOffsets(const int* counts, int n, int* offsets, int* hostDev, hipStream_t s) {
+    if (n > kRadiusOffsetsMax) return false;
+    const int run = (blocksFor(n, kOffsetsBlock) + 3) & ~3;
+    radiusOffsetsKernel<<<1, kOffsetsBlock, 0, s>>>(counts, n, run, offsets, hostDev);
+    hipCheck(hipGetLastError(), "radius offsets");
+    return true;
 }
 
 void radiusSummary(const int* total, const int* maxCopies, int* hostDev, hipStream_t s) {

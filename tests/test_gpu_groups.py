@@ -184,3 +184,33 @@ def test_batch_query_order(A, orc, counts):  # noqa: F811
         a, b = qoff[s], qoff[s + 1]
         if b > a:
             assert eq(got[0][a:b], orc.knn_brute(1, items[s], q[a:b], 2, threads=8)), s
+
+
+# lanes per query change at 16,384 and 40,960 queries, the one-workgroup offsets end at 32,768
+@pytest.mark.parametrize("nq", [1, 14, 16384, 32768, 32769, 40961])
+def test_radius_segment_lengths(A, orc, nq):  # noqa: F811
+    """Segments at the edges of every way of sorting them: registers (64), the workgroup's
+    network (2,048), the capture's room (2,048 for few queries), none at all."""
+    sizes = [0, 1, 2, 63, 64, 65, 127, 128, 129, 1024, 1025, 2047, 2048, 2049]
+    print(f"nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    centers = np.zeros((len(sizes), 3), np.float32)
+    centers[:, 0] = 10.0 * np.arange(len(sizes))
+    parts = [c + rng.uniform(-0.3, 0.3, (m, 3)) for c, m in zip(centers, sizes)]
+    items = np.concatenate(parts).astype(np.float32)[rng.permutation(sum(sizes))]
+    q = centers[np.arange(nq) % len(sizes)].copy()
+    if nq > 14:  # mostly short segments: the rest of the queries near nothing or few points
+        q[14:] = rng.uniform(-5, 25, (nq - 14, 3)) * np.float32([1, 0.02, 0.02])
+    want = orc.radius_brute(1, items, q, 1.0, threads=16)
+    for builder in (0, 1):
+        b = A.Bvh(1, items, builder)
+        for wide in (False, True):
+            for order in (A.ORDER_INPUT, A.ORDER_MORTON):
+                offs, keys, _, _ = b.radius(q, 1.0, order=order, wide=wide) if not wide else (
+                    b.build_wide(), b.radius(q, 1.0, order=order, wide=True))[1]
+                assert eq(offs, want[0]), (builder, wide, order)
+                assert eq(keys, want[1]), (builder, wide, order)
+        pb = A.PointBuffer(q)
+        for _ in range(2):  # the second call moves the hits before the host knows their number
+            _, offs, keys = pb.radius(b, 1.0, keep=True)
+            assert eq(offs, want[0]) and eq(keys, want[1])
