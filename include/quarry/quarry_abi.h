@@ -335,6 +335,15 @@ QR_API int qr_adjoint_closest(qr_bvh* bvh, const float* points_dev, int n, const
 QR_API int qr_adjoint_ray(qr_bvh* bvh, const void* rays_dev, int n, const uint64_t* results_dev,
                           const int* hit_prim_dev, const float* grad_t_dev, float* grad_origins_dev,
                           float* grad_dirs_dev, float* grad_tris_dev);
+/* The same for a mesh of shared vertices: faces_dev holds three vertex indices per
+ * triangle (prim_count x 3 i32, scene order, in range), and the triangles' gradients go
+ * straight to grad_vertices_dev (3 floats per vertex, accumulated, may be NULL). */
+QR_API int qr_adjoint_closest_mesh(qr_bvh* bvh, const float* points_dev, int n, const void* results_dev,
+                                   const int* aux_dev, const float* grad_dist2_dev, const int* faces_dev,
+                                   float* grad_points_dev, float* grad_vertices_dev);
+QR_API int qr_adjoint_ray_mesh(qr_bvh* bvh, const void* rays_dev, int n, const uint64_t* results_dev,
+                               const int* hit_prim_dev, const float* grad_t_dev, const int* faces_dev,
+                               float* grad_origins_dev, float* grad_dirs_dev, float* grad_vertices_dev);
 
 #ifdef __cplusplus
 }

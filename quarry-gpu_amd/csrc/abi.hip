@@ -904,7 +904,19 @@ int qr_adjoint_closest(qr_bvh* bvh, const float* points, int n, const void* resu
         need(n >= 0, "negative point count");
         need(n == 0 || (points && results && grad_dist2), "null device pointer");
         need(n == 0 || bvh->s.kind == kPrimPoint || aux != nullptr, "saved region / root required");
-        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_items, currentStream());
+        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_items, nullptr, currentStream());
+    });
+}
+
+int qr_adjoint_closest_mesh(qr_bvh* bvh, const float* points, int n, const void* results, const int* aux,
+                            const float* grad_dist2, const int* faces, float* grad_points, float* grad_vertices) {
+    return guard([&] {
+        checkTree(bvh, false);
+        need(n >= 0, "negative point count");
+        need(bvh->s.kind == kPrimTri, "mesh adjoint needs a triangle BVH");
+        need(faces != nullptr, "null face array");
+        need(n == 0 || (points && results && aux && grad_dist2), "null device pointer");
+        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_vertices, faces, currentStream());
     });
 }
 
@@ -914,7 +926,20 @@ int qr_adjoint_ray(qr_bvh* bvh, const void* rays, int n, const uint64_t* results
         checkTree(bvh, false);
         need(n >= 0, "negative ray count");
         need(n == 0 || (rays && results && hit_prim && grad_t), "null device pointer");
-        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_tris,
+        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_tris, nullptr,
+                   currentStream());
+    });
+}
+
+int qr_adjoint_ray_mesh(qr_bvh* bvh, const void* rays, int n, const uint64_t* results, const int* hit_prim,
+                        const float* grad_t, const int* faces, float* grad_origins, float* grad_dirs,
+                        float* grad_vertices) {
+    return guard([&] {
+        checkTree(bvh, false);
+        need(n >= 0, "negative ray count");
+        need(faces != nullptr, "null face array");
+        need(n == 0 || (rays && results && hit_prim && grad_t), "null device pointer");
+        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_vertices, faces,
                    currentStream());
     });
 }

@@ -25,7 +25,7 @@
 //   ray hit t with n = (b - a) x (c - a), w the hit's barycentrics:
 //     dt/do = -n / (n.d),  dt/dd = -t n / (n.d),  dt/dv_i = w_i n / (n.d).
 // Scene-order gradient arrays are accumulated with atomics (several queries may
-// share a primitive).
+// share a primitive), for a mesh straight into its shared vertices.
 #include "qr_adjoint.h"
 
 namespace qr {
@@ -38,6 +38,23 @@ __device__ __forceinline__ void atomicAdd3(float* dst, V3 v) {
     atomicAdd(dst + 0, v.x);
     atomicAdd(dst + 1, v.y);
     atomicAdd(dst + 2, v.z);
+}
+
+// Adds a triangle's three vertex gradients: to the triangle's nine words, or, with faces
+// (three vertex indices per triangle, scene order), to the shared vertices.  A vertex
+// without weight -- two of the three when the closest point is a vertex -- adds zeros and
+// is passed over: the atomics bound these kernels (262k queries around an icosphere 231
+// us with all nine, 82 into its vertices).
+__device__ __forceinline__ void addVertices(float* __restrict__ dst, const int* __restrict__ faces, int prim, V3 a,
+                                            V3 b, V3 c) {
+    const V3 v[3] = {a, b, c};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const bool zero = (v[k].x == 0.0f) & (v[k].y == 0.0f) & (v[k].z == 0.0f);
+        if (zero) continue;
+        const size_t at = static_cast<size_t>(prim) * 3 + k;
+        atomicAdd3(dst + 3 * (faces ? static_cast<size_t>(faces[at]) : at), v[k]);
+    }
 }
 
 // Barycentric weights (of a, b, c) of the closest point for a known region,
@@ -127,7 +144,8 @@ __global__ void saveAuxKernel(const typename L::Item* __restrict__ items, const 
 __global__ void adjTriKernel(const Tri* __restrict__ items, const int* __restrict__ primSlot,
                              const V3* __restrict__ pts, const ClosestResult* __restrict__ res,
                              const int* __restrict__ aux, const float* __restrict__ gout, int n,
-                             float* __restrict__ gpts, float* __restrict__ gitems) {
+                             float* __restrict__ gpts, float* __restrict__ gitems,
+                             const int* __restrict__ faces) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const ClosestResult r = res[i];
@@ -141,12 +159,7 @@ __global__ void adjTriKernel(const Tri* __restrict__ items, const int* __restric
         const V3 p = add(add(scale(tri.a, wa), scale(tri.b, wb)), scale(tri.c, wc));
         const V3 d = scale(sub(q, p), 2.0f * g);
         gq = d;
-        if (gitems) {
-            float* dst = gitems + static_cast<size_t>(r.prim) * 9;
-            atomicAdd3(dst + 0, scale(d, -wa));
-            atomicAdd3(dst + 3, scale(d, -wb));
-            atomicAdd3(dst + 6, scale(d, -wc));
-        }
+        if (gitems) addVertices(gitems, faces, r.prim, scale(d, -wa), scale(d, -wb), scale(d, -wc));
     }
     if (gpts) {
         gpts[3 * i + 0] = gq.x;
@@ -278,7 +291,8 @@ __global__ void adjGaussKernel(const Gaussian* __restrict__ items, const int* __
 __global__ void adjRayKernel(const Tri* __restrict__ items, const int* __restrict__ primSlot,
                              const Ray* __restrict__ rays, const uint64_t* __restrict__ res,
                              const int* __restrict__ hitPrim, const float* __restrict__ gout, int n,
-                             float* __restrict__ gorig, float* __restrict__ gdir, float* __restrict__ gitems) {
+                             float* __restrict__ gorig, float* __restrict__ gdir, float* __restrict__ gitems,
+                             const int* __restrict__ faces) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const uint64_t rv = res[i];
@@ -304,12 +318,7 @@ __global__ void adjRayKernel(const Tri* __restrict__ items, const int* __restric
         const V3 k = scale(nrm, g / nd);
         go = scale(k, -1.0f);
         gd = scale(k, -t);
-        if (gitems) {
-            float* dst = gitems + static_cast<size_t>(prim) * 9;
-            atomicAdd3(dst + 0, scale(k, 1.0f - bu - bv));
-            atomicAdd3(dst + 3, scale(k, bu));
-            atomicAdd3(dst + 6, scale(k, bv));
-        }
+        if (gitems) addVertices(gitems, faces, prim, scale(k, 1.0f - bu - bv), scale(k, bu), scale(k, bv));
     }
     if (gorig) {
         gorig[3 * i + 0] = go.x;
@@ -357,8 +366,9 @@ int saveClosestAux(BvhState& b, const float* pts, int n, const void* results, in
 }
 
 void adjointClosest(BvhState& b, const float* pts, int n, const void* results, const int* aux,
-                    const float* gout, float* gpts, float* gitems, hipStream_t s) {
+                    const float* gout, float* gpts, float* gitems, const int* faces, hipStream_t s) {
     if (n <= 0) return;
+    if (faces && b.kind != kPrimTri) throw ArgError("mesh adjoint: the tree does not hold triangles");
     ensurePrimSlot(b, s);
     const int grid = blocksFor(n, kBlock);
     const auto* P = reinterpret_cast<const V3*>(pts);
@@ -366,7 +376,7 @@ void adjointClosest(BvhState& b, const float* pts, int n, const void* results, c
     switch (b.kind) {
         case kPrimTri:
             adjTriKernel<<<grid, kBlock, 0, s>>>(reinterpret_cast<const Tri*>(b.items.p), b.primSlot.p, P, R, aux,
-                                                 gout, n, gpts, gitems);
+                                                 gout, n, gpts, gitems, faces);
             break;
         case kPrimPoint:
             adjPointKernel<<<grid, kBlock, 0, s>>>(reinterpret_cast<const V3*>(b.items.p), b.primSlot.p, P, R, gout,
@@ -381,13 +391,13 @@ void adjointClosest(BvhState& b, const float* pts, int n, const void* results, c
 }
 
 void adjointRay(BvhState& b, const void* rays, int n, const uint64_t* results, const int* hitPrim,
-                const float* gout, float* gorig, float* gdir, float* gitems, hipStream_t s) {
+                const float* gout, float* gorig, float* gdir, float* gitems, const int* faces, hipStream_t s) {
     if (n <= 0) return;
     if (b.kind != kPrimTri) throw ArgError("ray adjoint: the tree does not hold triangles");
     ensurePrimSlot(b, s);
     adjRayKernel<<<blocksFor(n, kBlock), kBlock, 0, s>>>(reinterpret_cast<const Tri*>(b.items.p), b.primSlot.p,
                                                          static_cast<const Ray*>(rays), results, hitPrim, gout, n,
-                                                         gorig, gdir, gitems);
+                                                         gorig, gdir, gitems, faces);
     hipCheck(hipGetLastError(), "adjoint ray");
 }
 

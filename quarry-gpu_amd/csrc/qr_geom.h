@@ -418,6 +418,9 @@ QR_HD GaussClosest gaussClosest(V3 p, const Gaussian& g) {
             const float newton = t - f / fp;
             if (newton > lo && newton < hi) next = newton;
         }
+        // a step that returns to t would return to it in every further step: f, fp and the
+        // bracket's end at t come out the same (20k kNN8 on 1M Gaussians 154 -> 142 us)
+        if (next == t) break;
         t = next;
     }
     const float ir0 = 1.0f / (t + aa), ir1 = 1.0f / (t + bb), ir2 = 1.0f / (t + cc);

@@ -156,6 +156,8 @@ def lib():
             "qr_closest_save_aux": ([_vp, _vp, _ip, _vp, _vp], _ip),
             "qr_adjoint_closest": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp], _ip),
             "qr_adjoint_ray": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
+            "qr_adjoint_closest_mesh": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
+            "qr_adjoint_ray_mesh": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
         }
         for name, (args, res) in sig.items():
             fn = getattr(L, name)

@@ -58,22 +58,36 @@ def _build(kind: int, items: torch.Tensor, wide: bool, builder: int) -> A.Bvh:
     return bvh
 
 
+def _gather(vertices: torch.Tensor, faces: torch.Tensor):
+    """Triangles (F, 9) of a mesh, and its faces as the adjoint kernels read them (int32,
+    in range: a negative index counts from the end, as in the gather)."""
+    idx = faces.long()
+    tris = vertices[idx].reshape(-1, 9).contiguous()
+    idx = idx.to(vertices.device)
+    return tris, torch.where(idx < 0, idx + vertices.shape[0], idx).to(torch.int32).contiguous()
+
+
+def _closest_forward(ctx, points, items, kind, order, wide, builder):
+    n = points.shape[0]
+    bvh = _build(kind, items.detach(), wide, builder)
+    res = torch.empty((n, 2), dtype=torch.int32, device=points.device)
+    aux = torch.empty(n, dtype=torch.int32, device=points.device)
+    ms = ctypes.c_double()
+    _on_stream()
+    A.check(A.lib().qr_closest_device(bvh.h, _p(points), n, _p(res), order, int(wide), ctypes.byref(ms)))
+    A.check(A.lib().qr_closest_save_aux(bvh.h, _p(points), n, _p(res), _p(aux)))
+    ctx.bvh = bvh
+    dist2 = res[:, 0].view(torch.float32).clone()
+    index = res[:, 1].to(torch.int64)
+    ctx.mark_non_differentiable(index)
+    return dist2, index, res, aux
+
+
 class _ClosestDist2(torch.autograd.Function):
     @staticmethod
     def forward(ctx, points, items, kind, order, wide, builder):
-        n = points.shape[0]
-        bvh = _build(kind, items.detach(), wide, builder)
-        res = torch.empty((n, 2), dtype=torch.int32, device=points.device)
-        aux = torch.empty(n, dtype=torch.int32, device=points.device)
-        ms = ctypes.c_double()
-        _on_stream()
-        A.check(A.lib().qr_closest_device(bvh.h, _p(points), n, _p(res), order, int(wide), ctypes.byref(ms)))
-        A.check(A.lib().qr_closest_save_aux(bvh.h, _p(points), n, _p(res), _p(aux)))
-        ctx.bvh = bvh
+        dist2, index, res, aux = _closest_forward(ctx, points, items, kind, order, wide, builder)
         ctx.save_for_backward(points, items, res, aux)
-        dist2 = res[:, 0].view(torch.float32).clone()
-        index = res[:, 1].to(torch.int64)
-        ctx.mark_non_differentiable(index)
         return dist2, index
 
     @staticmethod
@@ -88,11 +102,38 @@ class _ClosestDist2(torch.autograd.Function):
         return gp, gi, None, None, None, None
 
 
-class _RayHitT(torch.autograd.Function):
+class _MeshDist2(torch.autograd.Function):
+    """Closest points on a mesh of shared vertices: gathers the triangles itself, and the
+    adjoint adds each query's gradient straight to the vertices (a per-triangle gradient
+    and the gather's own sorted backward took three times as long as the adjoint)."""
+
     @staticmethod
-    def forward(ctx, origins, dirs, tris, tmax, order, wide, builder):
+    def forward(ctx, points, vertices, faces, order, wide, builder):
+        tris, idx = _gather(vertices, faces)
+        dist2, index, res, aux = _closest_forward(ctx, points, tris, A.PRIM_TRI, order, wide, builder)
+        ctx.save_for_backward(points, idx, res, aux)
+        ctx.vertices = vertices.shape  # (not the tensor: it may change in place before the backward)
+        return dist2, index
+
+    @staticmethod
+    def backward(ctx, g_dist2, g_index):
+        points, idx, res, aux = ctx.saved_tensors
+        n = points.shape[0]
+        g = g_dist2.contiguous().to(torch.float32)
+        gp = torch.empty_like(points) if ctx.needs_input_grad[0] else None
+        gv = torch.zeros(ctx.vertices, dtype=torch.float32, device=points.device) if ctx.needs_input_grad[1] else None
+        _on_stream()
+        A.check(A.lib().qr_adjoint_closest_mesh(ctx.bvh.h, _p(points), n, _p(res), _p(aux), _p(g), _p(idx), _p(gp),
+                                                _p(gv)))
+        return gp, gv, None, None, None, None
+
+
+class _MeshRayHitT(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, origins, dirs, vertices, faces, tmax, order, wide, builder):
         n = origins.shape[0]
-        bvh = _build(A.PRIM_TRI, tris.detach(), wide, builder)
+        tris, idx = _gather(vertices, faces)
+        bvh = _build(A.PRIM_TRI, tris, wide, builder)
         rays = torch.empty((n, 8), dtype=torch.float32, device=origins.device)
         rays[:, 0:3] = origins.detach()
         rays[:, 3:6] = dirs.detach()
@@ -105,7 +146,8 @@ class _RayHitT(torch.autograd.Function):
         A.check(A.lib().qr_raycast_save_device(bvh.h, _p(rays), n, _p(res), _p(hit), order, int(wide),
                                                ctypes.byref(ms)))
         ctx.bvh = bvh
-        ctx.save_for_backward(rays, tris, res, hit)
+        ctx.save_for_backward(rays, idx, res, hit)
+        ctx.vertices = vertices.shape
         hit_mask = (res >> 32) != 0
         t = (res & 0xFFFFFFFF).to(torch.int32).view(torch.float32).clone()
         t = torch.where(hit_mask, t, torch.full_like(t, float("inf")))
@@ -115,30 +157,31 @@ class _RayHitT(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_t, g_index):
-        rays, tris, res, hit = ctx.saved_tensors
+        rays, idx, res, hit = ctx.saved_tensors
         n = rays.shape[0]
         g = torch.nan_to_num(g_t.contiguous().to(torch.float32), nan=0.0, posinf=0.0, neginf=0.0)
         go = torch.empty((n, 3), dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[0] else None
         gd = torch.empty((n, 3), dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[1] else None
-        gt = torch.zeros_like(tris) if ctx.needs_input_grad[2] else None
+        gv = torch.zeros(ctx.vertices, dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[2] else None
         _on_stream()
-        A.check(A.lib().qr_adjoint_ray(ctx.bvh.h, _p(rays), n, _p(res), _p(hit), _p(g), _p(go), _p(gd), _p(gt)))
-        return go, gd, gt, None, None, None, None
+        A.check(A.lib().qr_adjoint_ray_mesh(ctx.bvh.h, _p(rays), n, _p(res), _p(hit), _p(g), _p(idx), _p(go), _p(gd),
+                                            _p(gv)))
+        return go, gd, gv, None, None, None, None, None
 
 
-def _tris(vertices: torch.Tensor, faces: torch.Tensor) -> torch.Tensor:
+def _mesh(vertices: torch.Tensor, faces: torch.Tensor) -> torch.Tensor:
     v = _f32(vertices, 3, "vertices")
     if faces.dim() != 2 or faces.shape[1] != 3:
         raise ValueError("faces must have shape (F, 3)")
-    return v[faces.long()].reshape(-1, 9).contiguous()
+    return v
 
 
 def closest_point_dist2(points, vertices, faces, order: str = "morton", wide: bool = True,
                         builder: str = "lbvh"):
     """Squared distance from each point to the mesh and the closest face index."""
     p = _f32(points, 3, "points")
-    return _ClosestDist2.apply(p, _tris(vertices, faces), A.PRIM_TRI, _ORDER[order], wide,
-                               A.BUILDER_SAH if builder == "sah" else A.BUILDER_LBVH)
+    return _MeshDist2.apply(p, _mesh(vertices, faces), faces, _ORDER[order], wide,
+                            A.BUILDER_SAH if builder == "sah" else A.BUILDER_LBVH)
 
 
 def ray_hit_t(origins, dirs, vertices, faces, tmax: float = float("inf"), order: str = "input",
@@ -149,8 +192,8 @@ def ray_hit_t(origins, dirs, vertices, faces, tmax: float = float("inf"), order:
     if o.shape[0] != d.shape[0]:
         raise ValueError("origins and dirs must match")
     orders = {"input": A.ORDER_INPUT, "morton": A.ORDER_MORTON, "morton_direction": A.ORDER_MORTON_DIRECTION}
-    return _RayHitT.apply(o, d, _tris(vertices, faces), float(tmax), orders[order], wide,
-                          A.BUILDER_SAH if builder == "sah" else A.BUILDER_LBVH)
+    return _MeshRayHitT.apply(o, d, _mesh(vertices, faces), faces, float(tmax), orders[order], wide,
+                              A.BUILDER_SAH if builder == "sah" else A.BUILDER_LBVH)
 
 
 def point_closest_dist2(points, cloud, order: str = "morton", wide: bool = True):
