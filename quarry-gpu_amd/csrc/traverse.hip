@@ -2162,8 +2162,7 @@ constexpr int kGroupDepth = 64;
 // 16 lanes per query (410 us, one wave per query 597), as many in and around an icosphere
 // -- long walks of very different lengths -- one wave per query (970 us against 1312).
 // From kTuneFrom queries on, the first call for a (tree, k class, query count octave)
-// times the three group shapes on its own queries and keeps the fastest; every shape
-// writes the same bits, so the trials' output is the call's output.
+// times the three group shapes on its own queries and keeps the fastest (tunedShape).
 constexpr int kTuneFrom = 65536;
 
 struct TuneKey {
@@ -2425,34 +2424,55 @@ static int defaultShape(int count) {
     return lanes == 64 ? kShapeWave : (lanes == 32 ? kShapeGroup32 : kShapeGroup16);
 }
 
+// The shape for this tree and size class, timed on the first call's own queries; that call's
+// results are then written already (done), every shape writing the same.  From
+// kTuneSplitFrom queries on each shape walks a third of the queries, so that the first call
+// on a new tree costs about what a later one does -- a mesh that moves is a new tree every
+// step; below, a third would not fill the device and say little, and each shape walks all.
+// The first to run finds the tree outside the caches; 32 lanes, seldom far from the better
+// of the other two, goes first.
+constexpr int kTuneSplitFrom = 3 * 65536;
+struct TunedShape {
+    int shape;
+    bool done;
+};
 template <typename L, int K>
-static int tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, int outStride, ClosestResult* out,
-                      hipStream_t s) {
+static TunedShape tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, int outStride,
+                             ClosestResult* out, hipStream_t s) {
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
     const TuneKey key{a.wideNodes, a.wideCount, L::kKind, K, octave};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
         const auto it = gTuned.find(key);
-        if (it != gTuned.end()) return it->second;
+        if (it != gTuned.end()) return {it->second, false};
     }
-    // every candidate shape once, after one untimed walk that brings the tree into
-    // the caches (so the first timed shape is not the only one reading it cold)
     constexpr int kShapes = K <= 16 ? 3 : 2;
-    const int shapes[3] = {kShapeWave, kShapeGroup32, kShapeGroup16};
-    EventSet<2 * kShapes> ev;
-    launchShape<L, K>(kShapeGroup32, a, pts, count, k, outStride, out, nullptr, s);
+    const int shapes[3] = {kShapeGroup32, kShapeWave, kShapeGroup16};
+    const bool split = count >= kTuneSplitFrom;
+    EventSet<kShapes + 1> ev;
+    ev.record(0, s);
     for (int i = 0; i < kShapes; ++i) {
-        ev.record(2 * i, s);
-        launchShape<L, K>(shapes[i], a, pts, count, k, outStride, out, nullptr, s);
-        ev.record(2 * i + 1, s);
+        const int begin = split ? static_cast<int>(static_cast<long long>(count) * i / kShapes) : 0;
+        const int end = split ? static_cast<int>(static_cast<long long>(count) * (i + 1) / kShapes) : count;
+        TraverseArgs part = a;
+        const V3* p = pts;
+        ClosestResult* o = out;
+        if (a.order) {
+            part.order = a.order + begin;
+        } else {
+            p += begin;
+            o += static_cast<size_t>(begin) * outStride;
+        }
+        launchShape<L, K>(shapes[i], part, p, end - begin, k, outStride, o, nullptr, s);
+        ev.record(i + 1, s);
     }
     hipCheck(hipGetLastError(), "nearest tuning");
-    ev.sync(2 * kShapes - 1);
-    int best = kShapeWave;
+    ev.sync(kShapes);
+    int best = shapes[0];
     float bestMs = 0.0f;
     for (int i = 0; i < kShapes; ++i) {
-        const float ms = ev.ms(2 * i, 2 * i + 1);
+        const float ms = ev.ms(i, i + 1);
         if (i == 0 || ms < bestMs) {
             best = shapes[i];
             bestMs = ms;
@@ -2461,7 +2481,7 @@ static int tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, in
     std::lock_guard<std::mutex> lock(gTuneMutex);
     if (gTuned.size() >= 4096) gTuned.clear();  // trees come and go; keep the table small
     gTuned[key] = best;
-    return best;
+    return {best, true};
 }
 
 // The shape an earlier tuning chose for this tree and size class, else the measured
@@ -2497,6 +2517,7 @@ static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int
         return;
     }
     int shape;
+    bool tune = false;
     switch (deep ? 1 : gTraversalMode) {
         case 1: shape = kShapeLane; break;
         case 2: shape = kShapeQuad; break;
@@ -2504,12 +2525,17 @@ static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int
         case 5: shape = kShapeGroup16; break;
         case 6: shape = kShapeGroup32; break;
         case 4:
-            shape = a.tune ? tunedShape<L, K>(a, pts, count, k, outStride, out, s) : cachedShape<L, K>(a, count);
+            tune = a.tune;
+            shape = cachedShape<L, K>(a, count);
             break;
         default:
-            shape = count < kTuneFrom ? defaultShape<L, K>(count)
-                    : a.tune          ? tunedShape<L, K>(a, pts, count, k, outStride, out, s)
-                                      : cachedShape<L, K>(a, count);
+            tune = a.tune && count >= kTuneFrom;
+            shape = count < kTuneFrom ? defaultShape<L, K>(count) : cachedShape<L, K>(a, count);
+    }
+    if (tune) {
+        const TunedShape t = tunedShape<L, K>(a, pts, count, k, outStride, out, s);
+        if (t.done && !a.stats) return;
+        shape = t.shape;
     }
     launchShape<L, K>(shape, a, pts, count, k, outStride, out, a.stats, s);
 }
