@@ -1458,11 +1458,11 @@ static void buildLbvhT(BvhState& b, const typename L::Item* dSrc, int n, hipStre
     }
     ev.record(4, s);
 
-    int depth = 0;
-    hipCheck(hipMemcpyAsync(&depth, b.height.p, sizeof(int), hipMemcpyDeviceToHost, s), "depth");
+    int* depth = pinnedInts();
+    hipCheck(hipMemcpyAsync(depth, b.height.p, sizeof(int), hipMemcpyDeviceToHost, s), "depth");
     ev.record(5, s);
     ev.sync(5);
-    b.depth = depth;
+    b.depth = *depth;
 
     if (t) {
         t->mortonMs = phases ? ev.ms(0, 1) : 0.0;
@@ -1581,6 +1581,54 @@ __global__ void depthJumpKernel(const int* __restrict__ parent, int nodeCount,
     depth[i] = dist;
 }
 
+// Whether each internal node 0..n-2 lies at an even depth, one bit a node, in two steps.
+// Nodes are numbered by leaf ranges, so the lower levels of a path stay within a block of
+// kJumpBlock neighbouring ids: the first step walks those in LDS (pointer doubling) and
+// leaves every node its first ancestor outside its block and the distance; the second
+// hops from block to block through those pairs, which no longer change (plain cached
+// loads).  2M triangles: 74 us for all nodes' depths through agent-scope jumps, 12 for
+// initialising them and 6 for the flags; 41 for these two.
+constexpr int kJumpBlock = 1024;
+__global__ __launch_bounds__(kJumpBlock) void blockJumpKernel(const int* __restrict__ parent, int internalCount,
+                                                              unsigned long long* __restrict__ jump) {
+    __shared__ int anc[kJumpBlock], dist[kJumpBlock];
+    const int first = static_cast<int>(blockIdx.x) * kJumpBlock;
+    const int t = static_cast<int>(threadIdx.x), i = first + t;
+    int a = i < internalCount ? parent[i] : -1;
+    int d = a < 0 ? 0 : 1;
+    anc[t] = a;
+    dist[t] = d;
+    __syncthreads();
+    while (true) {  // each round doubles the levels passed: at most 11
+        const bool inside = a >= first && a < first + kJumpBlock;
+        const int a2 = inside ? anc[a - first] : a;
+        const int d2 = inside ? d + dist[a - first] : d;
+        if (!__syncthreads_or(inside)) break;
+        anc[t] = a = a2;
+        dist[t] = d = d2;
+        __syncthreads();
+    }
+    if (i < internalCount)
+        jump[i] = (static_cast<unsigned long long>(static_cast<uint32_t>(d)) << 32) | static_cast<uint32_t>(a);
+}
+
+__global__ void evenDepthKernel(const unsigned long long* __restrict__ jump, int internalCount,
+                                unsigned long long* __restrict__ mask, int* __restrict__ counts) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    const bool live = i < internalCount;
+    int a = live ? i : -1, d = 0;
+    while (a >= 0) {  // (the root's block ends with -1)
+        const unsigned long long j = jump[a];
+        d += static_cast<int>(j >> 32);
+        a = static_cast<int>(j & 0xffffffffu);
+    }
+    const unsigned long long even = __ballot(live && (d & 1) == 0);
+    if ((threadIdx.x & 63) == 0 && live) {
+        mask[i >> 6] = even;
+        counts[i >> 6] = __popcll(even);
+    }
+}
+
 __global__ void depthJumpInitKernel(const int* __restrict__ parent, int nodeCount,
                                     unsigned long long* __restrict__ jump) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
@@ -1593,6 +1641,14 @@ __global__ void depthJumpInitKernel(const int* __restrict__ parent, int nodeCoun
               static_cast<uint32_t>(anc);
 }
 }  // namespace
+
+void evenDepthMask(BvhState& b, int* counts, hipStream_t s) {
+    const int internal = b.n - 1;
+    b.jump.reserve(static_cast<size_t>(internal));
+    blockJumpKernel<<<blocksFor(internal, kJumpBlock), kJumpBlock, 0, s>>>(b.parent.p, internal, b.jump.p);
+    evenDepthKernel<<<blocksFor(internal, kBlock), kBlock, 0, s>>>(b.jump.p, internal, b.wideMask.p, counts);
+    hipCheck(hipGetLastError(), "even depths");
+}
 
 void computeDepth(BvhState& b, hipStream_t s) {
     if (b.depthValid) return;

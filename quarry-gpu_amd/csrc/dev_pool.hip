@@ -212,4 +212,16 @@ void devTrim() {
     giveBack(back);
 }
 
+int* pinnedInts() {
+    static thread_local int* w = nullptr;
+    if (!w) hipCheck(hipHostMalloc(reinterpret_cast<void**>(&w), 16 * sizeof(int), hipHostMallocDefault), "pinned words");
+    return w;
+}
+
+int* pinnedIntsDevice() {
+    static thread_local int* d = nullptr;
+    if (!d) hipCheck(hipHostGetDevicePointer(reinterpret_cast<void**>(&d), pinnedInts(), 0), "pinned words map");
+    return d;
+}
+
 }  // namespace qr

@@ -1,6 +1,9 @@
 // Tree maintenance: 4-wide collapse, refit (full and dirty-only), structural
 // validation and the node-array hash.
 #include "qr_bvh.h"
+#include "qr_traverse.h"
+
+#include <algorithm>
 
 namespace qr {
 
@@ -40,10 +43,10 @@ __device__ __forceinline__ Box readBoxAgent(const Node2* nd) {
 // at odd depth (direct children) or even depth (grandchildren), so every leaf is
 // referenced exactly once.
 
-__global__ void wideFlagKernel(const int* __restrict__ depth, int internalCount,
-                               int* __restrict__ flags) {
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < internalCount) flags[i] = (depth[i] & 1) == 0 ? 1 : 0;
+// Wide index of internal node i, which is a 4-wide node (its bit is set).
+__device__ __forceinline__ int wideIndex(const unsigned long long* __restrict__ mask, const int* __restrict__ base,
+                                         int i) {
+    return base[i >> 6] + __popcll(mask[i >> 6] & ((1ull << (i & 63)) - 1ull));
 }
 
 __device__ __forceinline__ void setEntry(WideEntry& e, const Node2& box, int child) {
@@ -64,35 +67,42 @@ __device__ __forceinline__ void clearEntry(WideEntry& e) {
     e.pad = 0;
 }
 
-// Four lanes per internal node: lane s writes entry s (32 B) of the node's 4-wide
-// node, so a wide node is one contiguous 128 B write.  Even-depth internal node i
-// holds its children, with each interior child replaced by its two children.
-// A node id >= n - 1 is a leaf, so the entry layout needs no node reads.
+// Even-depth internal node i becomes a 4-wide node: its children, with each interior child
+// replaced by its two children.  A wave takes the nodes of one mask word: it lists those
+// whose bit is set, then four lanes write each (lane s entry s, 32 B), 16 nodes a step, so
+// every lane works and a step writes 2 KB in one run (a quad per node, set or not: 2M
+// triangles 85 us, 77 here; reads and writes of 134 MB each).  A node id >= n - 1 is a
+// leaf, so the entry layout needs no node reads.
 __global__ __launch_bounds__(kBlock) void wideEmitKernel(const Node2* __restrict__ nodes, int n,
-                                                         const int* __restrict__ depth,
-                                                         const int* __restrict__ wideId,
+                                                         const unsigned long long* __restrict__ mask,
+                                                         const int* __restrict__ base,
                                                          Wide4* __restrict__ wide) {
-    const long long t = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-    const int i = static_cast<int>(t >> 2);
-    const int slot = static_cast<int>(t & 3);
-    if (i >= n - 1 || (depth[i] & 1) != 0) return;
-    const Node2 nd = nodes[i];
-    const int a0 = nd.left >= n - 1 ? 1 : 2;
-    const int a1 = nd.right >= n - 1 ? 1 : 2;
-    WideEntry e;
-    clearEntry(e);
-    int src = -1;
-    if (slot < a0) {
-        src = a0 == 1 ? nd.left : (slot == 0 ? nodes[nd.left].left : nodes[nd.left].right);
-    } else if (slot - a0 < a1) {
-        const int j = slot - a0;
-        src = a1 == 1 ? nd.right : (j == 0 ? nodes[nd.right].left : nodes[nd.right].right);
+    __shared__ int list[kBlock / 64][64];  // per wave: the word's 4-wide nodes, in order
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int word = static_cast<int>(blockIdx.x) * (kBlock / 64) + wave;
+    const unsigned long long m = word < (n - 1 + 63) / 64 ? mask[word] : 0ull;
+    if ((m >> lane) & 1ull) list[wave][__popcll(m & ((1ull << lane) - 1ull))] = word * 64 + lane;
+    __syncthreads();
+    const int slot = lane & 3, count = __popcll(m);
+    for (int j = lane >> 2; j < count; j += 16) {
+        const Node2 nd = nodes[list[wave][j]];
+        const int a0 = nd.left >= n - 1 ? 1 : 2;
+        const int a1 = nd.right >= n - 1 ? 1 : 2;
+        WideEntry e;
+        clearEntry(e);
+        int src = -1;
+        if (slot < a0) {
+            src = a0 == 1 ? nd.left : (slot == 0 ? nodes[nd.left].left : nodes[nd.left].right);
+        } else if (slot - a0 < a1) {
+            const int k = slot - a0;
+            src = a1 == 1 ? nd.right : (k == 0 ? nodes[nd.right].left : nodes[nd.right].right);
+        }
+        if (src >= 0) {
+            const Node2 sn = nodes[src];
+            setEntry(e, sn, src >= n - 1 ? sn.left : wideIndex(mask, base, src));
+        }
+        wide[base[word] + j].c[slot] = e;
     }
-    if (src >= 0) {
-        const Node2 sn = nodes[src];
-        setEntry(e, sn, src >= n - 1 ? sn.left : wideId[src]);
-    }
-    wide[wideId[i]].c[slot] = e;
 }
 
 // ---- refit --------------------------------------------------------------------------
@@ -289,28 +299,32 @@ __global__ void checkDepthKernel(const Node2* __restrict__ nodes, const int* __r
 void reserveWide(BvhState& b) {
     if (b.n < 2) throw ArgError("buildWideNodes: tree is empty");
     const int internal = b.n - 1;
-    b.depthArr.reserve(static_cast<size_t>(b.nodeCount));
-    b.jump.reserve(static_cast<size_t>(b.nodeCount));
-    b.wideId.reserve(static_cast<size_t>(internal));
-    b.wideFlags.reserve(static_cast<size_t>(internal));
-    b.wideScan.reserve(static_cast<size_t>(scanScratchInts(internal)) + 1);
+    const int words = blocksFor(internal, 64);
+    b.jump.reserve(static_cast<size_t>(internal));
+    b.wideMask.reserve(static_cast<size_t>(words));
+    b.wideBase.reserve(static_cast<size_t>(words) + 1);
+    b.wideScan.reserve(static_cast<size_t>(std::max(scanScratchInts(words) + 1, words)));
     // at most one wide node per internal node: no count round trip before the emit
     b.wide.reserve(static_cast<size_t>(internal));
 }
 
 void buildWide(BvhState& b, hipStream_t s) {
     reserveWide(b);
-    computeDepth(b, s);
-    const int internal = b.n - 1;
-    wideFlagKernel<<<blocksFor(internal, kBlock), kBlock, 0, s>>>(b.depthArr.p, internal, b.wideFlags.p);
-    int* total = b.wideScan.p + scanScratchInts(internal);
-    scanExclusive(b.wideFlags.p, b.wideId.p, internal, total, b.wideScan.p, s);
-    wideEmitKernel<<<blocksFor(4LL * internal, kBlock), kBlock, 0, s>>>(b.nodes.p, b.n, b.depthArr.p,
-                                                                       b.wideId.p, b.wide.p);
+    const int internal = b.n - 1, words = blocksFor(internal, 64);
+    int* word = pinnedInts();
+    const bool small = words <= kRadiusOffsetsMax;  // the counts' scan in one workgroup, its total to the host
+    evenDepthMask(b, small ? b.wideScan.p : b.wideBase.p, s);
+    if (small) {
+        radiusOffsets(b.wideScan.p, words, b.wideBase.p, pinnedIntsDevice(), s);
+    } else {
+        int* total = b.wideScan.p + scanScratchInts(words);
+        scanExclusive(b.wideBase.p, b.wideBase.p, words, total, b.wideScan.p, s);
+        hipCheck(hipMemcpyAsync(word, total, sizeof(int), hipMemcpyDeviceToHost, s), "wide count");
+    }
+    wideEmitKernel<<<blocksFor(internal, kBlock), kBlock, 0, s>>>(b.nodes.p, b.n, b.wideMask.p, b.wideBase.p, b.wide.p);
     hipCheck(hipGetLastError(), "wide emit");
-    int count = 0;
-    hipCheck(hipMemcpyAsync(&count, total, sizeof(int), hipMemcpyDeviceToHost, s), "wide count");
     hipCheck(hipStreamSynchronize(s), "wide sync");
+    const int count = *word;
     if (count <= 0) throw DeviceError("buildWideNodes: no wide nodes");
     b.wideCount = count;
     b.wideValid = true;
@@ -458,8 +472,7 @@ void buildBatchWide(BatchState& b, hipStream_t s) {
 void reemitWide(BvhState& b, hipStream_t s) {
     if (!b.wideValid) return;
     const int internal = b.n - 1;
-    wideEmitKernel<<<blocksFor(4LL * internal, kBlock), kBlock, 0, s>>>(b.nodes.p, b.n, b.depthArr.p,
-                                                                       b.wideId.p, b.wide.p);
+    wideEmitKernel<<<blocksFor(internal, kBlock), kBlock, 0, s>>>(b.nodes.p, b.n, b.wideMask.p, b.wideBase.p, b.wide.p);
     hipCheck(hipGetLastError(), "wide re-emit");
 }
 

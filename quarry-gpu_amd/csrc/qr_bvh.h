@@ -48,15 +48,17 @@ struct BvhState {
     DevBuf<int> primSlot;
     bool primSlotValid = false;
 
-    // per node depth (root 0); computed on demand for wide collapse and validate
+    // per node depth (root 0); computed on demand for validate
     DevBuf<int> depthArr;
     bool depthValid = false;
     DevBuf<unsigned long long> jump;  // pointer-jumping scratch of the depth pass
 
     // 4-wide collapse
     DevBuf<Wide4> wide;
-    DevBuf<int> wideId;             // per internal node: wide index or -1
-    DevBuf<int> wideFlags, wideScan;  // collapse scratch (flags, scan partials + total)
+    // which internal nodes are 4-wide nodes (one bit each) and, per 64 of them, how many
+    // come before: a node's wide index is its word's count plus the bits below its own
+    DevBuf<unsigned long long> wideMask;
+    DevBuf<int> wideBase, wideScan;  // (wideScan: scan scratch + total)
     int wideCount = 0;
     bool wideValid = false;
 
@@ -127,6 +129,9 @@ void buildSahDevice(BvhState& b, int kind, const void* dItems, int n, hipStream_
 
 // Per-node depth by pointer jumping over the parent array (root 0).
 void computeDepth(BvhState& b, hipStream_t s);
+// b.wideMask (bit i: internal node i lies at an even depth) and, in counts, the set bits of
+// each of its words.
+void evenDepthMask(BvhState& b, int* counts, hipStream_t s);
 
 // Leaf init + bottom-up box propagation for all leaves, given items already in
 // leaf order (refit path shares it).

@@ -96,6 +96,11 @@ struct QuietFree {
     bool on = false;
 };
 
+// A few pinned host words of the calling thread, kept for the process: a small read from
+// the device into pageable memory goes through a driver bounce buffer.
+int* pinnedInts();
+int* pinnedIntsDevice();  // the same words as the device addresses them
+
 // Plain device allocation owned by a scope (or a borrowed view of memory someone
 // else owns: borrow() makes release() forget the pointer instead of freeing it).
 template <typename T>

@@ -70,9 +70,10 @@ bool launchRadiusCapture(const TraverseArgs& a, const V3* pts, int count, float 
 // nothing was captured: cap 0); counts are those of the capture / count pass.
 void launchRadiusFill(const TraverseArgs& a, const V3* pts, int count, float r2, const int* counts,
                       int cap, const int* offsets, uint64_t* keys, hipStream_t s);
-// Offsets of the segments, and the total and the largest count straight into hostDev[0] and
-// hostDev[1] (device view of pinned host words), in one launch; false, doing nothing, above
-// kRadiusOffsetsMax queries (scanExclusive and radiusSummary serve those).
+// Offsets of the segments (exclusive sums of n counts, and the total behind them), and the
+// total and the largest count straight into hostDev[0] and hostDev[1] (device view of
+// pinned host words), in one launch; false, doing nothing, above kRadiusOffsetsMax counts
+// (scanExclusive and radiusSummary serve those).  counts and offsets must not alias.
 constexpr int kRadiusOffsetsMax = 32768;
 bool radiusOffsets(const int* counts, int n, int* offsets, int* hostDev, hipStream_t s);
 // Whether radiusCompact leaves every segment sorted when the largest has maxSeg hits.

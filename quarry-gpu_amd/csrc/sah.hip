@@ -1611,8 +1611,8 @@ static void buildSahT(BvhState& b, const typename L::Item* dSrc, int n, hipStrea
 
     finishTopology(b, dSrc, order, s, &T.ctl[kCtlError]);
     hipCheck(hipMemcpyAsync(hw, T.ctl, kCtlWords * sizeof(int), hipMemcpyDeviceToHost, s), "sah control");
-    int depth = 0;
-    hipCheck(hipMemcpyAsync(&depth, b.height.p, sizeof(int), hipMemcpyDeviceToHost, s), "depth");
+    int* depth = pinnedInts();
+    hipCheck(hipMemcpyAsync(depth, b.height.p, sizeof(int), hipMemcpyDeviceToHost, s), "depth");
     ev.record(5, s);
     ev.sync(5);
     if (hw[kCtlError] != 0) {
@@ -1620,7 +1620,7 @@ static void buildSahT(BvhState& b, const typename L::Item* dSrc, int n, hipStrea
         b.nodeCount = 0;
         failed();
     }
-    b.depth = depth;
+    b.depth = *depth;
     SahBuildStats st;
     st.levels = hw[kCtlMaxLevel] + 1;
     st.binnedSlots = static_cast<unsigned int>(hw[kCtlBinned]);

@@ -214,3 +214,47 @@ def test_radius_segment_lengths(A, orc, nq):  # noqa: F811
         for _ in range(2):  # the second call moves the hits before the host knows their number
             _, offs, keys = pb.radius(b, 1.0, keep=True)
             assert eq(offs, want[0]) and eq(keys, want[1])
+
+
+# one mask word, its edges, one and two blocks of 1,024 internal nodes, and more words than the
+# one-workgroup scan takes (32,768)
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 66, 1025, 1026, 5000, (1 << 21) + 70])
+@pytest.mark.parametrize("builder", [0, 1])
+def test_wide_nodes_are_the_even_depth_nodes(A, n, builder):  # noqa: F811
+    print(f"n={n} builder={builder}", flush=True)
+    items = np.random.default_rng(n).uniform(-9, 9, (n, 3)).astype(np.float32)
+    b = A.Bvh(1, items, builder)
+    b.build_wide()
+    raw, _ = b.read()
+    nodes = raw.view(np.int32).reshape(-1, 8)
+    kids = nodes[: n - 1, 6:8]
+    depth = np.full(n - 1, -1)
+    level, d = np.array([0]), 0
+    while level.size:
+        depth[level] = d
+        level = kids[level].reshape(-1)
+        level, d = level[level < n - 1], d + 1
+    even = np.nonzero(depth % 2 == 0)[0]
+    index = np.full(n - 1, -1)
+    index[even] = np.arange(even.size)
+    info = b.info()
+    assert info.wide_count == even.size
+    wide = np.zeros((even.size, 4, 8), np.int32)
+    A.check(A.lib().qr_dev_download(A.ptr(wide), info.d_wide_nodes, wide.nbytes))
+    # a child that is a leaf stands for itself, an interior one for its two children, in order
+    src = np.full((even.size, 4), -1)
+    at = np.zeros(even.size, int)
+    rows = np.arange(even.size)
+    for side in (0, 1):
+        c = kids[even, side]
+        leaf = c >= n - 1
+        pair = kids[np.where(leaf, 0, c)]
+        src[rows, at] = np.where(leaf, c, pair[:, 0])
+        two = ~leaf
+        src[rows[two], at[two] + 1] = pair[two, 1]
+        at += np.where(leaf, 1, 2)
+    used = src >= 0
+    assert eq(wide[used][:, :6], nodes[src[used], :6])
+    want = np.where(src[used] >= n - 1, nodes[src[used], 6], index[np.minimum(src[used], n - 2)])
+    assert eq(wide[used][:, 6], want)
+    assert np.all(wide[~used][:, 6] == np.iinfo(np.int32).min)
