@@ -53,7 +53,8 @@ typedef enum {
 
 typedef enum { QR_PRIM_TRIANGLE = 0, QR_PRIM_POINT = 1, QR_PRIM_GAUSSIAN = 2 } qr_prim;
 typedef enum { QR_BUILDER_LBVH = 0, QR_BUILDER_SAH = 1 } qr_builder;
-/* RayOrder / QueryOrder (src/gpu/gpu_bvh.h:224, :274) */
+/* RayOrder / QueryOrder (src/gpu/gpu_bvh.h:224, :274).  Results do not depend on it; a set
+ * too small for the reordering to pay for itself is visited in input order all the same. */
 typedef enum { QR_ORDER_INPUT = 0, QR_ORDER_MORTON = 1, QR_ORDER_MORTON_DIRECTION = 2 } qr_order;
 
 /* GpuBuildTimings (src/gpu/gpu_bvh.h:79-89) */

@@ -830,7 +830,7 @@ double raycastImpl(const qr_bvh* bvh, const Ray* rays, int n, uint64_t* out, qr_
     ev.record(0, s);
     TraverseArgs a = argsFor(bvh->s, wide != 0);
     a.stats = collectStats ? st.p : nullptr;
-    if (order != QR_ORDER_INPUT) {
+    if (order != QR_ORDER_INPUT && orderingPays(a, kWalkRays, n)) {
         const float* base = reinterpret_cast<const float*>(rays) + (order == QR_ORDER_MORTON ? 0 : 3);
         const int mode = order == QR_ORDER_MORTON_DIRECTION ? kBoxUnit
                                                             : (scratch->bbValid ? kBoxGiven : kBoxMeasure);
@@ -1284,7 +1284,7 @@ double pointQuery(const qr_bvh* bvh, const V3* pts, int n, int k, int outStride,
     ev.record(0, s);
     TraverseArgs a = argsFor(bvh->s, wide != 0);
     a.stats = collectStats ? st.p : nullptr;
-    if (order == QR_ORDER_MORTON)
+    if (order == QR_ORDER_MORTON && orderingPays(a, k <= 1 ? kWalkClosest : kWalkKnn, n))
         a.order = reorder(*work, reinterpret_cast<const float*>(pts), 3, n,
                           work->bbValid ? kBoxGiven : kBoxMeasure, s);
     ev.record(1, s);
@@ -1406,7 +1406,7 @@ int qr_knn_device_noalloc(const qr_bvh* bvh, const float* pts, int n, int k, voi
         hipStream_t s = currentStream();
         TraverseArgs a = argsFor(bvh->s, wide != 0, false);
         a.tune = false;  // timing trials would take events; shapes give the same bits
-        if (order == QR_ORDER_MORTON) {
+        if (order == QR_ORDER_MORTON && orderingPays(a, k == 1 ? kWalkClosest : kWalkKnn, n)) {
             uint32_t* w = scratchOnDevice();
             SortWorkspace ws;  // views into the fixed array, never freed
             ws.keysAlt.borrow(w + kNaAltKeys, kNaQueries);
@@ -1455,7 +1455,7 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             ev.record(0, s);
             TraverseArgs a = argsFor(bvh->s, wide != 0);
             a.stats = collectStats ? st.p : nullptr;
-            if (order == QR_ORDER_MORTON)
+            if (order == QR_ORDER_MORTON && orderingPays(a, kWalkRadius, n))
                 a.order = reorder(*p, reinterpret_cast<const float*>(p->pts.p), 3, n,
                                   p->bbValid ? kBoxGiven : kBoxMeasure, s);
             ev.record(1, s);

@@ -46,6 +46,12 @@ void mortonOrder(const float* base, int stride, int count, int boxMode, SortWork
                  uint32_t* keys, uint32_t* keysSorted, uint32_t* orderOut, uint32_t* bb,
                  hipStream_t s);
 
+// Whether a requested reordering pays for itself on a set of this size (the order steers
+// locality only; results do not depend on it).  Below the counts here ordering costs more
+// than a walk in input order loses, also when the input order is random.
+enum WalkKind : int { kWalkClosest = 0, kWalkKnn = 1, kWalkRadius = 2, kWalkRays = 3 };
+bool orderingPays(const TraverseArgs& a, WalkKind walk, int count);
+
 void launchRays(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, hipStream_t s);
 // Same, also writing the hit triangle's scene index (-1 for a miss) to hitPrim.
 void launchRaysSave(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,

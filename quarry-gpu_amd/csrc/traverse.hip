@@ -1,23 +1,25 @@
 // Traversal kernels: closest-hit rays, closest / kNN / radius point queries, over
 // binary (32 B) or 4-wide (128 B) nodes, for triangle, point and Gaussian leaves.
 //
-// One lane per ray or query, depth-first.  The pruning predicates are the
+// A ray or query is walked by one lane, by four (quads), or by a group of 8 to 64
+// lanes whose quads each open a node a round; the launchers at the end of the file
+// choose by the set's size, leaf kind and k.  The pruning predicates are the
 // reference's (src/gpu/raycast.cu:75-245, src/gpu/query.cu:52-637): padded slab
 // test against the current best t for rays, box lower bound <= bound for
 // closest / kNN (so equal-distance primitives with a smaller index are still
 // reached), box lower bound <= r^2 for radius.  Every predicate only prunes
 // subtrees that cannot hold a better (dist2, index) or a smaller t, so the result
-// is the brute-force answer whatever the tree, node width or visiting order -
+// is the brute-force answer whatever the tree, node width, walk or visiting order -
 // which is what makes binary, wide, LBVH, SAH and reordered runs bit-identical.
 //
 // Layout for gfx950:
-//   * the per-lane DFS stack lives in LDS ([depth][lane], 32 entries = 32 KB per
-//     256-lane workgroup); deeper entries spill to scratch, which only very deep
-//     or very wide traversals touch;
-//   * a node's children are ordered with a fixed compare-exchange network in
-//     registers (no dynamically indexed private arrays);
-//   * leaf children are tested as soon as their parent is opened, nearest first,
-//     against the live bound, and only interior children go on the stack;
+//   * one lane: the depth-first stack lives in LDS ([depth][lane]); deeper entries
+//     spill to scratch, which only very deep or very wide traversals touch;
+//   * groups: one LDS stack per query, shared by its quads; a binary node is opened
+//     together with its interior children, so both node widths feed four entries to
+//     a quad; the k-best list is one entry per lane;
+//   * leaf children are tested as soon as their parent is opened, against the live
+//     bound, and only interior children go on the stack, nearest on top;
 //   * closest is kNN with k = 1 (identical record and tie rule).
 //
 // Queries may be visited in a permuted order (Morton reordering): lane i works
@@ -2232,6 +2234,7 @@ static void launchRayShape(int shape, const TraverseArgs& a, const Ray* rays, in
 // icosphere 64k 186 / 61 / 68, 262k 245 / 191 / 220.  Binary nodes cross over alike.  Mode
 // 1 forces one lane, mode 3 one wave; mode 4 times one lane against one wave on the first
 // call for a 4-wide tree, save flag and ray-count octave.
+constexpr int kRayLaneFrom = 393216;
 template <bool kSave>
 static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,
                     hipStream_t s) {
@@ -2241,7 +2244,7 @@ static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t*
         if (count < 3072) return kShapeWave;
         if (count < 12288) return kShapeGroup32;
         if (count < 49152) return kShapeGroup16;
-        return count < 393216 ? kShapeGroup8 : kShapeLane;
+        return count < kRayLaneFrom ? kShapeGroup8 : kShapeLane;
     }
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
@@ -2554,6 +2557,27 @@ static void launchNearestT(const TraverseArgs& a, const V3* pts, int count, int 
     } else {
         launchNearestTK<L, 32>(a, pts, count, k, outStride, out, s);
     }
+}
+
+// Ordering is four to six launches, 25-30 us up to 262,144 elements and 80 us at a million.
+// With a group of lanes on each query neighbouring queries share little that input order
+// does not find in the caches too.  Measured on queries and rays in random order (call in
+// us, input order / ordered):
+//   4-wide nodes: closest, 2M-triangle terrain 60k 163 / 184, 100k 230 / 246, 200k 391 /
+//   378; 131k terrain 60k 202 / 209, 131k 364 / 350; 1M points 100k 92 / 116; icosphere 60k
+//   405 / 400, 100k 449 / 429.  kNN16, 131k terrain 60k 415 / 405, 100k 562 / 513;
+//   icosphere 60k 774 / 771, 80k 880 / 734; 2M terrain 100k 328 / 343.  Radius, 1M points 60k
+//   659 / 678, 131k 1061 / 918; 2M terrain 131k 160 / 184.
+//   Binary nodes: terrain closest 8k 146 / 153, 16k 251 / 234; points kNN16 16k 121 / 140,
+//   32k 184 / 165.
+//   Rays, 4-wide: city, cosine 131k 99 / 127, 380k 195 / 242, down 380k 163 / 205; one lane
+//   per ray (larger sets) profits: 1M down 370 / 341, 131k terrain 629 / 386.  Binary:
+//   terrain cosine 131k 227 / 216, 33k 87 / 102.
+bool orderingPays(const TraverseArgs& a, WalkKind walk, int count) {
+    if (gTraversalMode != 0 || a.depth > kGroupDepth) return true;  // forced shapes keep their order
+    if (walk == kWalkRays) return count >= (a.wide ? kRayLaneFrom : 98304);
+    if (!a.wide) return count >= (a.kind == 0 ? 12288 : 24576);
+    return count >= (walk == kWalkClosest ? 131072 : 65536);
 }
 
 static void launchNearest(const TraverseArgs& a, const V3* pts, int count, int k, int outStride,

@@ -258,3 +258,26 @@ def test_wide_nodes_are_the_even_depth_nodes(A, n, builder):  # noqa: F811
     want = np.where(src[used] >= n - 1, nodes[src[used], 6], index[np.minimum(src[used], n - 2)])
     assert eq(wide[used][:, 6], want)
     assert np.all(wide[~used][:, 6] == np.iinfo(np.int32).min)
+
+
+# both sides of every count from which a requested order is made
+@pytest.mark.parametrize("count", [12287, 12288, 24576, 65535, 65536, 98304, 131072])
+def test_order_is_made_or_not(A, orc, count):  # noqa: F811
+    print(f"count={count}", flush=True)
+    rng = np.random.default_rng(count)
+    tris, pts = random_tris(rng, 300), scene(1, 300, 5)
+    q = rng.uniform(-40, 40, (count, 3)).astype(np.float32)
+    rays = unusual_rays(rng, tris, count)
+    for kind, items in ((0, tris), (1, pts)):
+        b = A.Bvh(kind, items)
+        b.build_wide()
+        for wide in (False, True):
+            assert eq(b.closest(q, order=A.ORDER_MORTON, wide=wide)[0], orc.knn_brute(kind, items, q, 0, threads=16))
+            assert eq(b.knn(q, 3, order=A.ORDER_MORTON, wide=wide)[0], orc.knn_brute(kind, items, q, 3, threads=16))
+            o, k, _, _ = b.radius(q, 2.0, order=A.ORDER_MORTON, wide=wide)
+            wo, wk = orc.radius_brute(kind, items, q, 2.0, threads=16)
+            assert eq(o, wo) and eq(k, wk)
+            if kind == 0:
+                want = orc.ray_brute(tris, rays, threads=16)
+                for order in (A.ORDER_MORTON, A.ORDER_MORTON_DIRECTION):
+                    assert eq(b.raycast(rays, order=order, wide=wide)[0], want)
