@@ -4,12 +4,12 @@
 // driver), :2043-2122 (entry points).  The reference bins 16 ways with one global
 // bin table per task; this build bins 32 ways and keeps the histograms in LDS:
 //   * tasks above kChunk primitives are cut into kChunk-position chunks; each
-//     workgroup builds its chunk's histogram (3 axes x 32 bins x {count, box,
-//     centroid box}) with LDS atomics and flushes it once with global atomics;
-//     one wave per task then scores the 3 x 31 planes, and a one-pass stable
-//     partition moves the primitive records (the bin pass also counts each
-//     quarter-chunk part's bins, a per-task scan of the parts' left counts gives
-//     every partition wave its destinations);
+//     workgroup builds its chunk's histogram (3 axes x 32 bins x {count, box}) with
+//     LDS atomics and flushes it once with global atomics; one wave per task then
+//     scores the 3 x 31 planes, and a one-pass stable partition moves the primitive
+//     records and reduces the two sides' centroid boxes into the child tasks (the bin
+//     pass also counts each quarter-chunk part's bins, a per-task scan of the parts'
+//     left counts gives every partition wave its destinations);
 //   * tasks of kSerial+1 .. kChunk primitives are handled by one workgroup each:
 //     histogram, plane choice and stable partition never leave the workgroup;
 //   * ranges of kSerial or fewer primitives get balanced count/2 splits in their
@@ -44,7 +44,7 @@ constexpr int kChunk = 4096;
 constexpr int kSerial = 64;
 constexpr int kMedianLevel = 32;
 constexpr int kBlock = 256;
-constexpr int kBinVals = 13;  // count, box lo xyz, box hi xyz, centroid lo xyz, centroid hi xyz
+constexpr int kBinVals = 7;  // count, box lo xyz, box hi xyz
 constexpr int kHist = 3 * kBins * kBinVals;
 constexpr int kParts = 4;                   // a chunk's parts: one partition wave each
 constexpr int kPartLen = kChunk / kParts;   // records per part
@@ -62,6 +62,47 @@ struct SahTask {
     float cLo[4], cHi[4];
 };
 
+// A task in the global tables: the centroid box as ordered bits, which the partition
+// kernel lowers and raises by atomics for the children of a split by plane.
+struct StoredTask {
+    int start, count, node, meta;
+    uint32_t cLo[4], cHi[4];
+};
+
+__device__ __forceinline__ StoredTask packTask(const SahTask& t) {
+    StoredTask p;
+    p.start = t.start;
+    p.count = t.count;
+    p.node = t.node;
+    p.meta = t.meta;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        p.cLo[k] = orderedBits(t.cLo[k]);
+        p.cHi[k] = orderedBits(t.cHi[k]);
+    }
+    return p;
+}
+
+__device__ __forceinline__ SahTask unpackTask(const StoredTask& p) {
+    SahTask t;
+    t.start = p.start;
+    t.count = p.count;
+    t.node = p.node;
+    t.meta = p.meta;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        t.cLo[k] = fromOrderedBits(p.cLo[k]);
+        t.cHi[k] = fromOrderedBits(p.cHi[k]);
+    }
+    return t;
+}
+
+// Where the children of a split by plane keep their centroid boxes (null: a serial
+// range, or a box that is already there).
+struct ChildBoxes {
+    StoredTask* task[2];
+};
+
 struct SahResult {
     int axis, plane, nL, pad;
     float lLo[4], lHi[4], rLo[4], rHi[4];
@@ -71,16 +112,9 @@ struct Chunk {
     int task, start, count, pad;
 };
 
+// A histogram keeps no centroid bounds: a split's children take their centroid boxes
+// from the records as the partition moves them.
 __device__ __forceinline__ int hidx(int a, int b, int v) { return (a * kBins + b) * kBinVals + v; }
-// Histograms that keep no centroid bounds (kCent = false: the subtree tiers, which
-// take their children's centroid boxes from the records) store 7 values per bin
-// (count, box lo xyz, box hi xyz) in a smaller LDS array.
-template <bool kCent>
-constexpr int binVals() { return kCent ? kBinVals : 7; }
-template <bool kCent>
-constexpr int histWords() { return 3 * kBins * binVals<kCent>(); }
-template <bool kCent>
-__device__ __forceinline__ int hidxT(int a, int b, int v) { return (a * kBins + b) * binVals<kCent>() + v; }
 
 struct AxisMap {
     float lo[3], scale[3];
@@ -107,21 +141,19 @@ __device__ __forceinline__ int binOf(float c, float lo, float scale) {
     return static_cast<int>(f);
 }
 
-// The empty value of histogram word i: count 0, box and centroid bounds inverted.
+// The empty value of histogram word i: count 0, box bounds inverted.
 __device__ __forceinline__ uint32_t binInit(int i) {
     const int v = i % kBinVals;
-    return v == 0 ? 0u : ((v >= 1 && v <= 3) || (v >= 7 && v <= 9)) ? orderedBits(kInf) : orderedBits(-kInf);
+    return v == 0 ? 0u : v <= 3 ? orderedBits(kInf) : orderedBits(-kInf);
 }
 
-template <bool kCent = true>
 __device__ __forceinline__ void histInit(uint32_t* h) {
-    // (word v of a bin: the same empty values for both layouts, v < 7 being shared)
-    for (int i = threadIdx.x; i < histWords<kCent>(); i += blockDim.x) h[i] = binInit(i % binVals<kCent>());
+    for (int i = threadIdx.x; i < kHist; i += blockDim.x) h[i] = binInit(i);
 }
 
 // Bins of a contiguous range of records.  Each thread takes a run of consecutive
 // records and keeps, per axis, the values of its current bin in registers, flushing
-// them to the LDS histogram with 13 atomics only when the bin changes: neighbouring
+// them to the LDS histogram with 7 atomics only when the bin changes: neighbouring
 // records (a mesh in scene order, the halves of a partition) mostly share a bin,
 // and one-record-per-lane atomics on one shared bin serialize across the wave.
 // Count, min and max are exact and order-free, so the histogram is the same bits as
@@ -129,26 +161,19 @@ __device__ __forceinline__ void histInit(uint32_t* h) {
 struct BinRun {
     int bin;
     uint32_t cnt;
-    uint32_t v[12];  // box lo xyz, box hi xyz, centroid lo xyz, centroid hi xyz
+    uint32_t v[6];  // box lo xyz, box hi xyz
 };
 
 // Adds a finished run to the histogram (and its count to part[a * kBins + bin] when
 // part is given: the counts of the current part of a chunk).
-// kCent = false leaves the centroid bounds out (a caller that takes its children's
-// centroid boxes from the records themselves).
-template <bool kCent = true>
 __device__ __forceinline__ void binRunFlush(uint32_t* h, int a, const BinRun& r, uint32_t* part = nullptr) {
     if (r.cnt == 0u) return;
-    atomicAdd(&h[hidxT<kCent>(a, r.bin, 0)], r.cnt);
+    atomicAdd(&h[hidx(a, r.bin, 0)], r.cnt);
     if (part) atomicAdd(&part[a * kBins + r.bin], r.cnt);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        atomicMin(&h[hidxT<kCent>(a, r.bin, 1 + k)], r.v[k]);
-        atomicMax(&h[hidxT<kCent>(a, r.bin, 4 + k)], r.v[3 + k]);
-        if constexpr (kCent) {
-            atomicMin(&h[hidxT<kCent>(a, r.bin, 7 + k)], r.v[6 + k]);
-            atomicMax(&h[hidxT<kCent>(a, r.bin, 10 + k)], r.v[9 + k]);
-        }
+        atomicMin(&h[hidx(a, r.bin, 1 + k)], r.v[k]);
+        atomicMax(&h[hidx(a, r.bin, 4 + k)], r.v[3 + k]);
     }
 }
 
@@ -162,53 +187,50 @@ __device__ __forceinline__ void binRunsInit(BinRun* run) {
 
 // One record into the thread's runs (a run is flushed when its bin changes); one
 // instantiation per axis, so that the runs and the axis map stay in registers.
-template <int a, bool kCent, typename R>
+template <int a, typename R>
 __device__ __forceinline__ void binRunAddAxis(uint32_t* h, BinRun& u, const R& r, const AxisMap& m,
                                               uint32_t* part) {
     if (!m.use[a]) return;
     const int b = binOf(r.c[a], m.lo[a], m.scale[a]);
     if (b != u.bin) {
-        binRunFlush<kCent>(h, a, u, part);
+        binRunFlush(h, a, u, part);
         u.bin = b;
         u.cnt = 0u;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            u.v[k] = u.v[6 + k] = 0xFFFFFFFFu;
-            u.v[3 + k] = u.v[9 + k] = 0u;
+            u.v[k] = 0xFFFFFFFFu;
+            u.v[3 + k] = 0u;
         }
     }
     ++u.cnt;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const uint32_t lo = orderedBits(r.lo[k]), hi = orderedBits(r.hi[k]), c = orderedBits(r.c[k]);
+        const uint32_t lo = orderedBits(r.lo[k]), hi = orderedBits(r.hi[k]);
         u.v[k] = lo < u.v[k] ? lo : u.v[k];
         u.v[3 + k] = hi > u.v[3 + k] ? hi : u.v[3 + k];
-        u.v[6 + k] = c < u.v[6 + k] ? c : u.v[6 + k];
-        u.v[9 + k] = c > u.v[9 + k] ? c : u.v[9 + k];
     }
 }
 
 // r is taken by value: loaded once, not re-read after the flushes' LDS atomics.
-template <bool kCent = true, typename R = PrimRec>
+template <typename R = PrimRec>
 __device__ __forceinline__ void binRunAdd(uint32_t* h, BinRun* run, const R r, const AxisMap& m,
                                           uint32_t* part = nullptr) {
-    binRunAddAxis<0, kCent>(h, run[0], r, m, part);
-    binRunAddAxis<1, kCent>(h, run[1], r, m, part);
-    binRunAddAxis<2, kCent>(h, run[2], r, m, part);
+    binRunAddAxis<0>(h, run[0], r, m, part);
+    binRunAddAxis<1>(h, run[1], r, m, part);
+    binRunAddAxis<2>(h, run[2], r, m, part);
 }
 
-template <bool kCent = true>
 __device__ __forceinline__ void binRunsFlush(uint32_t* h, const BinRun* run, const AxisMap& m,
                                              uint32_t* part = nullptr) {
 #pragma unroll
     for (int a = 0; a < 3; ++a)
-        if (m.use[a]) binRunFlush<kCent>(h, a, run[a], part);
+        if (m.use[a]) binRunFlush(h, a, run[a], part);
 }
 
 // Bins a contiguous range of records: each of the kBT threads takes a run of
 // consecutive records (neighbouring records mostly share a bin, so the runs flush
 // rarely).
-template <int kBT, bool kCent = true>
+template <int kBT>
 __device__ __forceinline__ void histAddRange(uint32_t* h, const PrimRec* __restrict__ rec, int count,
                                              const AxisMap& m) {
     const int per = (count + kBT - 1) / kBT;
@@ -220,11 +242,11 @@ __device__ __forceinline__ void histAddRange(uint32_t* h, const PrimRec* __restr
         PrimRec cur = rec[beg];
         for (int i = beg; i < end; ++i) {
             const PrimRec nxt = rec[i + 1 < end ? i + 1 : i];
-            binRunAdd<kCent>(h, run, cur, m);
+            binRunAdd(h, run, cur, m);
             cur = nxt;
         }
     }
-    binRunsFlush<kCent>(h, run, m);
+    binRunsFlush(h, run, m);
 }
 
 __device__ __forceinline__ float areaOf(float lx, float ly, float lz, float hx, float hy, float hz) {
@@ -240,9 +262,6 @@ __device__ __forceinline__ float areaOf(float lx, float ly, float lz, float hx, 
 // bits as summing the bins plane by plane.  The (cost, axis * 32 + plane) minimum
 // is reduced across the lanes, then the chosen plane's side counts and centroid
 // boxes; lane 0 writes the result.  h is the task's histogram (LDS or global).
-// kCent = false: a histogram without centroid bounds; the chosen plane's side
-// centroid boxes are then left 0 for the caller to fill from the records.
-template <bool kCent = true>
 __device__ void chooseSplit(const uint32_t* h, const SahTask& t, const AxisMap& m, SahResult* out) {
     const int lane = threadIdx.x & 63;
     const int bin = lane & (kBins - 1);
@@ -253,12 +272,12 @@ __device__ void chooseSplit(const uint32_t* h, const SahTask& t, const AxisMap& 
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         if (!m.use[a]) continue;
-        const int c = static_cast<int>(h[hidxT<kCent>(a, bin, 0)]);
+        const int c = static_cast<int>(h[hidx(a, bin, 0)]);
         float v[6];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
-            v[k] = fromOrderedBits(h[hidxT<kCent>(a, bin, 1 + k)]);
-            v[3 + k] = fromOrderedBits(h[hidxT<kCent>(a, bin, 4 + k)]);
+            v[k] = fromOrderedBits(h[hidx(a, bin, 1 + k)]);
+            v[3 + k] = fromOrderedBits(h[hidx(a, bin, 4 + k)]);
         }
         const int pc = prefixAdd32(c, lane);
         const int total = __builtin_amdgcn_readlane(pc, 31);
@@ -319,35 +338,15 @@ __device__ void chooseSplit(const uint32_t* h, const SahTask& t, const AxisMap& 
     // right of it (a min / max of ordered bits is exact and order-free; empty bins
     // take the identities)
     const int a = bestKey / kBins, plane = bestKey % kBins;
-    const uint32_t c = h[hidxT<kCent>(a, bin, 0)];
+    const uint32_t c = h[hidx(a, bin, 0)];
     const bool isLeft = bin < plane;
     const uint32_t nL = reduce32<AddU>(isLeft ? c : 0u);
-    uint32_t v[12];  // left min xyz, left max xyz, right min xyz, right max xyz
-#pragma unroll
-    for (int k = 0; k < 12; ++k) v[k] = 0u;
-    if constexpr (kCent) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const uint32_t lo = c ? h[hidxT<kCent>(a, bin, 7 + k)] : 0xFFFFFFFFu;
-            const uint32_t hi = c ? h[hidxT<kCent>(a, bin, 10 + k)] : 0u;
-            v[k] = reduce32<MinU>(isLeft ? lo : 0xFFFFFFFFu);
-            v[3 + k] = reduce32<MaxU>(isLeft ? hi : 0u);
-            v[6 + k] = reduce32<MinU>(isLeft ? 0xFFFFFFFFu : lo);
-            v[9 + k] = reduce32<MaxU>(isLeft ? 0u : hi);
-        }
-    }
     if (lane != 0) return;
     res.axis = a;
     res.plane = plane;
     res.nL = static_cast<int>(nL);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        res.lLo[k] = fromOrderedBits(v[k]);
-        res.lHi[k] = fromOrderedBits(v[3 + k]);
-        res.rLo[k] = fromOrderedBits(v[6 + k]);
-        res.rHi[k] = fromOrderedBits(v[9 + k]);
-    }
-    res.lLo[3] = res.lHi[3] = res.rLo[3] = res.rHi[3] = 0.0f;
+    for (int k = 0; k < 4; ++k) res.lLo[k] = res.lHi[k] = res.rLo[k] = res.rHi[k] = 0.0f;
     *out = res;
 }
 
@@ -382,6 +381,25 @@ __device__ __forceinline__ int blockExclusive(int v, int* lds, int* total) {
     __syncthreads();
     *total = all;
     return base + x - v;
+}
+
+// Two sides' centroid boxes as ordered bits: left min xyz, max xyz, right min xyz,
+// max xyz.
+__device__ __forceinline__ bool sideBoxIsMin(int k) { return k < 3 || (k >= 6 && k < 9); }
+
+// One record's centroid (as float bits) into its side's box.
+__device__ __forceinline__ void sideBoxAdd(uint32_t* bx, bool left, uint32_t x, uint32_t y, uint32_t z) {
+    const uint32_t u[3] = {orderedBits(__uint_as_float(x)), orderedBits(__uint_as_float(y)),
+                           orderedBits(__uint_as_float(z))};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const uint32_t lo = left ? bx[k] : bx[6 + k], hi = left ? bx[3 + k] : bx[9 + k];
+        const uint32_t nlo = u[k] < lo ? u[k] : lo, nhi = u[k] > hi ? u[k] : hi;
+        bx[k] = left ? nlo : bx[k];
+        bx[6 + k] = left ? bx[6 + k] : nlo;
+        bx[3 + k] = left ? nhi : bx[3 + k];
+        bx[9 + k] = left ? bx[9 + k] : nhi;
+    }
 }
 
 // Stable partition of the records [begin, begin + cnt) of task t by split s into
@@ -442,18 +460,7 @@ __device__ __forceinline__ void partitionRange(const PrimRec* __restrict__ src, 
             const float c = ax == 0 ? __uint_as_float(w0.x) : ax == 1 ? __uint_as_float(w0.y) : __uint_as_float(w1.x);
             left = goesLeft(c, begin + i, t, s, m);
             if (kBoxes) {
-                const uint32_t u[3] = {orderedBits(__uint_as_float(w0.x)), orderedBits(__uint_as_float(w0.y)),
-                                       orderedBits(__uint_as_float(w1.x))};
-#pragma unroll
-                for (int k = 0; k < 3; ++k) {
-                    const int o = left ? 0 : 6;
-                    const uint32_t lo = left ? bx[k] : bx[6 + k], hi = left ? bx[3 + k] : bx[9 + k];
-                    const uint32_t nlo = u[k] < lo ? u[k] : lo, nhi = u[k] > hi ? u[k] : hi;
-                    bx[k] = o == 0 ? nlo : bx[k];
-                    bx[6 + k] = o == 6 ? nlo : bx[6 + k];
-                    bx[3 + k] = o == 0 ? nhi : bx[3 + k];
-                    bx[9 + k] = o == 6 ? nhi : bx[9 + k];
-                }
+                sideBoxAdd(bx, left, w0.x, w0.y, w1.x);
             }
         }
         const unsigned long long lm = __ballot(valid && left);
@@ -492,10 +499,10 @@ __device__ __forceinline__ void partitionRange(const PrimRec* __restrict__ src, 
 // Stable partition of the records [begin, begin + cnt) by one wave whose left and
 // right destinations are known (from the counts of the range's bins): one pass,
 // lane-strided reads, ballot ranks.  Destinations outside the task's sides are
-// reported through err, never written.
+// reported through err, never written.  The sides' centroid boxes are added to bx.
 __device__ __forceinline__ void partitionWaveRange(const PrimRec* __restrict__ src, PrimRec* __restrict__ dst,
                                                    int begin, int cnt, int leftDst, int rightDst, const SahTask& t,
-                                                   const SahResult& s, const AxisMap& m, int* err) {
+                                                   const SahResult& s, const AxisMap& m, int* err, uint32_t* bx) {
     const int lane = threadIdx.x & 63;
     const int ax = s.axis < 0 ? 0 : s.axis;
     const unsigned long long below = (1ull << lane) - 1ull;
@@ -516,6 +523,7 @@ __device__ __forceinline__ void partitionWaveRange(const PrimRec* __restrict__ s
             w4 = sw[4];
             const float c = ax == 0 ? __uint_as_float(w0.x) : ax == 1 ? __uint_as_float(w0.y) : __uint_as_float(w1.x);
             left = goesLeft(c, begin + i, t, s, m);
+            sideBoxAdd(bx, left, w0.x, w0.y, w1.x);
         }
         const unsigned long long lm = __ballot(valid && left);
         const unsigned long long rm = __ballot(valid && !left);
@@ -642,9 +650,9 @@ __device__ __forceinline__ int metaOf(int buf, int level) { return buf | (level 
 // kSerial primitives, serial ranges are disjoint and non-empty).
 struct SahTables {
     PrimRec* rec[2];
-    SahTask* big[2];
-    SahTask* local;
-    SahTask* small;
+    StoredTask* big[2];
+    StoredTask* local;
+    StoredTask* small;
     SerialTask* serial;
     Chunk* chunks;
     int* first;
@@ -652,6 +660,7 @@ struct SahTables {
     int* chunkOff;   // per chunk part: lefts of the task's earlier parts
     uint32_t* bins;
     SahResult* results;
+    ChildBoxes* childBoxes;
     int* ctl;
     int maxBig, maxLocal, maxSerial, maxChunks;
 };
@@ -676,7 +685,7 @@ __device__ __forceinline__ void writeSplit(int n, int start, int count, int node
 // The tables' two-entry arrays indexed by a selection, not a dynamic subscript (the
 // tables are a kernel argument; a subscript would copy them to scratch).
 __device__ __forceinline__ PrimRec* recOf(const SahTables& T, int buf) { return buf ? T.rec[1] : T.rec[0]; }
-__device__ __forceinline__ SahTask* bigOf(const SahTables& T, int cur) { return cur ? T.big[1] : T.big[0]; }
+__device__ __forceinline__ StoredTask* bigOf(const SahTables& T, int cur) { return cur ? T.big[1] : T.big[0]; }
 
 __device__ __forceinline__ void pushSerial(const SahTables& T, int start, int count, int node, int buf) {
     const int at = atomicAdd(&T.ctl[kCtlSerial], 1);
@@ -722,32 +731,31 @@ __device__ __forceinline__ SahTask makeTask(int start, int count, int node, int 
 constexpr int kSmallTask = 512;
 
 // A child of a big task: serial range, small or local task, or next-level big task.
-__device__ __forceinline__ void routeChild(const SahTables& T, int nextBuf, int start, int count, int node, int buf,
-                                           int level, const float* lo, const float* hi) {
+// Returns where the task is stored (null: a serial range, or a full table).
+__device__ __forceinline__ StoredTask* routeChild(const SahTables& T, int nextBuf, int start, int count, int node,
+                                                  int buf, int level, const float* lo, const float* hi) {
     if (count <= kSerial) {
         pushSerial(T, start, count, node, buf);
-    } else if (count <= kSmallTask) {
-        const int at = atomicAdd(&T.ctl[kCtlSmall], 1);
-        if (at < T.maxLocal) {
-            T.small[at] = makeTask(start, count, node, metaOf(buf, level), lo, hi);
-        } else {
-            atomicOr(&T.ctl[kCtlError], 1);
-        }
-    } else if (count <= kChunk) {
-        const int at = atomicAdd(&T.ctl[kCtlLocal], 1);
-        if (at < T.maxLocal) {
-            T.local[at] = makeTask(start, count, node, metaOf(buf, level), lo, hi);
-        } else {
-            atomicOr(&T.ctl[kCtlError], 1);
-        }
-    } else {
-        const int at = atomicAdd(&T.ctl[kCtlBig0 + nextBuf], 1);
-        if (at < T.maxBig) {
-            bigOf(T, nextBuf)[at] = makeTask(start, count, node, metaOf(buf, level), lo, hi);
-        } else {
-            atomicOr(&T.ctl[kCtlError], 1);
-        }
+        return nullptr;
     }
+    int word = kCtlBig0 + nextBuf, room = T.maxBig;
+    StoredTask* table = bigOf(T, nextBuf);
+    if (count <= kSmallTask) {
+        word = kCtlSmall;
+        room = T.maxLocal;
+        table = T.small;
+    } else if (count <= kChunk) {
+        word = kCtlLocal;
+        room = T.maxLocal;
+        table = T.local;
+    }
+    const int at = atomicAdd(&T.ctl[word], 1);
+    if (at >= room) {
+        atomicOr(&T.ctl[kCtlError], 1);
+        return nullptr;
+    }
+    table[at] = packTask(makeTask(start, count, node, metaOf(buf, level), lo, hi));
+    return table + at;
 }
 
 // The root: one task over [0, n) with the centroid bounds of the prep kernel.
@@ -801,7 +809,7 @@ __global__ __launch_bounds__(kBlock) void sahPlanKernel(SahTables T, int cur, in
         const int i = base + threadIdx.x;
         int c = 0;
         if (i < nt) {
-            const SahTask t = bigOf(T, cur)[i];
+            const StoredTask t = bigOf(T, cur)[i];
             c = (t.count + kChunk - 1) / kChunk;
             sStart[threadIdx.x] = t.start;
             sCount[threadIdx.x] = t.count;
@@ -846,20 +854,29 @@ __device__ __forceinline__ uint32_t* binsOf(const SahTables& T, int cur) {
 // Wave w bins the chunk's part w (kPartLen records); besides the task's histogram it
 // records each part's bin counts, from which the chunk scan gives every part its
 // partition offsets without a counting pass.
+// Bound by the LDS atomics: a record whose bins differ from its neighbour's costs 21 of
+// them (39 while the bins also kept centroid bounds), and lanes of a wave that meet in one
+// bin take turns.  Even and odd lanes have a histogram each.  Measured (us a build, all
+// levels; 13 values / 7 values with 1 / 2 / 4 / 8 copies): city, 1.3M triangles 582 / 393 /
+// 364 / 350 / 359, 2M-triangle terrain, whose neighbours share bins, 472 / 411 / 404 / 409 /
+// 422, 300k Gaussians 224 / 175 / 181 / 185 / 191.  More waves a chunk (512 and 1,024
+// threads) were no faster: city 449 and 539 with one copy.
+constexpr int kBinCopies = 2;
 __global__ __launch_bounds__(kBlock) void sahBinKernel(SahTables T, int cur) {
     static_assert(kChunk == kParts * kPartLen, "a chunk is its parts");
     static_assert(kBlock / 64 == kParts, "one wave per part");
     if (static_cast<int>(blockIdx.x) >= T.ctl[kCtlChunks]) return;
-    __shared__ uint32_t h[kHist];
+    __shared__ uint32_t h[kBinCopies * kHist];
     __shared__ uint32_t part[kParts][3 * kBins];
     const Chunk ch = T.chunks[blockIdx.x];
-    const SahTask t = bigOf(T, cur)[ch.task];
+    const SahTask t = unpackTask(bigOf(T, cur)[ch.task]);
     const AxisMap m = axisMap(t);
-    histInit(h);
+    for (int i = threadIdx.x; i < kBinCopies * kHist; i += kBlock) h[i] = binInit(i);
     for (int i = threadIdx.x; i < kParts * 3 * kBins; i += kBlock) (&part[0][0])[i] = 0u;
     __syncthreads();
     // wave w bins part w, each lane a run of consecutive records
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    uint32_t* hl = h + (lane % kBinCopies) * kHist;
     const int pBeg = w * kPartLen;
     const int pCnt = ch.count - pBeg < kPartLen ? ch.count - pBeg : kPartLen;
     if (pCnt > 0) {
@@ -873,11 +890,11 @@ __global__ __launch_bounds__(kBlock) void sahBinKernel(SahTables T, int cur) {
             PrimRec cur = src[beg];
             for (int i = beg; i < end; ++i) {
                 const PrimRec nxt = src[i + 1 < end ? i + 1 : i];
-                binRunAdd(h, run, cur, m, part[w]);
+                binRunAdd(hl, run, cur, m, part[w]);
                 cur = nxt;
             }
         }
-        binRunsFlush(h, run, m, part[w]);
+        binRunsFlush(hl, run, m, part[w]);
     }
     __syncthreads();
     uint32_t* g = binsOf(T, cur) + static_cast<size_t>(ch.task) * kHist;
@@ -886,11 +903,16 @@ __global__ __launch_bounds__(kBlock) void sahBinKernel(SahTables T, int cur) {
         T.chunkBins[static_cast<size_t>(blockIdx.x) * kParts * 3 * kBins + i] = static_cast<int>((&part[0][0])[i]);
     for (int i = threadIdx.x; i < kHist; i += kBlock) {
         const int v = i % kBinVals;
-        if (h[i - v] == 0u) continue;  // empty bin
-        const uint32_t x = h[i];
+        uint32_t x = h[i];
+#pragma unroll
+        for (int c = 1; c < kBinCopies; ++c) {
+            const uint32_t y = h[c * kHist + i];
+            x = v == 0 ? x + y : v <= 3 ? MinU::op(x, y) : MaxU::op(x, y);
+        }
+        if (x == binInit(v)) continue;  // nothing to add: an empty bin
         if (v == 0) {
             atomicAdd(&g[i], x);
-        } else if ((v >= 1 && v <= 3) || (v >= 7 && v <= 9)) {
+        } else if (v <= 3) {
             atomicMin(&g[i], x);
         } else {
             atomicMax(&g[i], x);
@@ -927,7 +949,7 @@ __global__ __launch_bounds__(kBlock) void sahSplitKernel(SahTables T, int cur, i
     __shared__ SahResult sres;
     const int ti = blockIdx.x;
     if (ti >= T.ctl[kCtlBig0 + cur]) return;
-    const SahTask t = bigOf(T, cur)[ti];
+    const SahTask t = unpackTask(bigOf(T, cur)[ti]);
     uint32_t* h = binsOf(T, cur) + static_cast<size_t>(ti) * kHist;
     if (median) {
         if (threadIdx.x == 0) sres = medianResult(t);
@@ -936,7 +958,10 @@ __global__ __launch_bounds__(kBlock) void sahSplitKernel(SahTables T, int cur, i
     }
     __syncthreads();
     const SahResult r = sres;
-    if (threadIdx.x == 0) T.results[ti] = r;
+    if (threadIdx.x == 0) {
+        T.results[ti] = r;
+        T.childBoxes[ti] = {{nullptr, nullptr}};
+    }
     if (!median)
         for (int i = threadIdx.x; i < kHist; i += kBlock) h[i] = binInit(i);
 
@@ -985,28 +1010,61 @@ __global__ __launch_bounds__(kBlock) void sahSplitKernel(SahTables T, int cur, i
         atomicMax(&T.ctl[kCtlMaxLevel], level);
         int l, rr;
         writeSplit(n, t.start, t.count, t.node, nL, nodes, parent, farEnd, &l, &rr);
-        routeChild(T, 1 - cur, t.start, nL, l, buf, level + 1, r.lLo, r.lHi);
-        routeChild(T, 1 - cur, t.start + nL, t.count - nL, rr, buf, level + 1, r.rLo, r.rHi);
+        // a split by plane: the children's centroid boxes start empty and are filled by
+        // the partition; one by position hands down the task's own box
+        const float eLo[3] = {kInf, kInf, kInf}, eHi[3] = {-kInf, -kInf, -kInf};
+        const bool plane = r.axis >= 0;
+        StoredTask* tl = routeChild(T, 1 - cur, t.start, nL, l, buf, level + 1, plane ? eLo : r.lLo, plane ? eHi : r.lHi);
+        StoredTask* tr = routeChild(T, 1 - cur, t.start + nL, t.count - nL, rr, buf, level + 1, plane ? eLo : r.rLo,
+                                    plane ? eHi : r.rHi);
+        if (plane) T.childBoxes[ti] = {{tl, tr}};
     }
 }
 
 // One workgroup per chunk, one wave per part: each part's records go to their
-// sides at the offsets the chunk scan gave it, in one pass.
+// sides at the offsets the chunk scan gave it, in one pass.  The centroid boxes of the
+// two sides are reduced on the way (registers, then the workgroup's four waves) and
+// go to the child tasks with one atomic per word and workgroup: 252 -> 285 us a build of
+// the 1.3M-triangle city, for 582 -> 364 in the bins that then need no centroid bounds.
 __global__ __launch_bounds__(kBlock) void sahPartScatterKernel(SahTables T, int cur) {
     if (static_cast<int>(blockIdx.x) >= T.ctl[kCtlChunks]) return;
     const Chunk ch = T.chunks[blockIdx.x];
-    const SahTask t = bigOf(T, cur)[ch.task];
+    const SahTask t = unpackTask(bigOf(T, cur)[ch.task]);
     const SahResult s = T.results[ch.task];
     const AxisMap m = axisMap(t);
+    __shared__ uint32_t waveBox[kParts][12];
     const int w = threadIdx.x >> 6;
     const int pBeg = w * kPartLen;
     const int pCnt = ch.count - pBeg < kPartLen ? ch.count - pBeg : kPartLen;
+    uint32_t bx[12];
+#pragma unroll
+    for (int k = 0; k < 12; ++k) bx[k] = sideBoxIsMin(k) ? 0xFFFFFFFFu : 0u;
     if (pCnt > 0) {
         const int e = blockIdx.x * kParts + w;
         const int partLeft = T.chunkOff[e];  // lefts of the task's earlier parts
         const int partPos = ch.start + pBeg - t.start;
         partitionWaveRange(recOf(T, t.meta & 1), recOf(T, 1 - (t.meta & 1)), ch.start + pBeg, pCnt,
-                           t.start + partLeft, t.start + s.nL + (partPos - partLeft), t, s, m, &T.ctl[kCtlError]);
+                           t.start + partLeft, t.start + s.nL + (partPos - partLeft), t, s, m, &T.ctl[kCtlError], bx);
+    }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+        bx[k] = sideBoxIsMin(k) ? reduce64<MinU>(bx[k]) : reduce64<MaxU>(bx[k]);
+        if ((threadIdx.x & 63) == 0) waveBox[w][k] = bx[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 12) {
+        const int k = threadIdx.x, side = k / 6, c = k % 3;
+        StoredTask* child = T.childBoxes[ch.task].task[side];
+        if (child != nullptr) {
+            const bool isMin = sideBoxIsMin(k);
+            uint32_t x = waveBox[0][k];
+            for (int v = 1; v < kParts; ++v) x = isMin ? MinU::op(x, waveBox[v][k]) : MaxU::op(x, waveBox[v][k]);
+            if (isMin) {
+                atomicMin(&child->cLo[c], x);
+            } else {
+                atomicMax(&child->cHi[c], x);
+            }
+        }
     }
     if (threadIdx.x == 0) atomicAdd(&T.ctl[kCtlParted], ch.count);
 }
@@ -1038,7 +1096,7 @@ __device__ __forceinline__ void flushSerial(const SahTables& T, const SerialTask
 template <int kBT>
 __global__ __launch_bounds__(kBT) void sahSubtreeKernel(SahTables T, int n, Node2* __restrict__ nodes,
                                                         int* __restrict__ parent, int* __restrict__ farEnd) {
-    __shared__ uint32_t h[histWords<false>()];
+    __shared__ uint32_t h[kHist];
     __shared__ SahResult sres;
     __shared__ SahTask stk[kSubtreeStack];
     __shared__ SahTask curTask;
@@ -1052,7 +1110,7 @@ __global__ __launch_bounds__(kBT) void sahSubtreeKernel(SahTables T, int n, Node
     const int listLen = T.ctl[kCtlLocal];
     for (int task = blockIdx.x; task < listLen; task += gridDim.x) {
     if (threadIdx.x == 0) {
-        stk[0] = T.local[task];
+        stk[0] = unpackTask(T.local[task]);
         ssp = 1;
     }
     __syncthreads();
@@ -1073,11 +1131,11 @@ __global__ __launch_bounds__(kBT) void sahSubtreeKernel(SahTables T, int n, Node
         PrimRec* dst = recOf(T, 1 - buf);
         const AxisMap m = axisMap(t);
         if (!median) {
-            histInit<false>(h);
+            histInit(h);
             __syncthreads();
-            histAddRange<kBT, false>(h, src + t.start, t.count, m);
+            histAddRange<kBT>(h, src + t.start, t.count, m);
             __syncthreads();
-            if (threadIdx.x < 64) chooseSplit<false>(h, t, m, &sres);
+            if (threadIdx.x < 64) chooseSplit(h, t, m, &sres);
         } else if (threadIdx.x == 0) {
             sres = medianResult(t);
         }
@@ -1133,7 +1191,8 @@ __global__ __launch_bounds__(kBT) void sahSubtreeKernel(SahTables T, int n, Node
                     } else if (cc[side] <= kSmallTask) {
                         const int at = atomicAdd(&T.ctl[kCtlSmall], 1);
                         if (at < T.maxLocal) {
-                            T.small[at] = childTask(cs[side], cc[side], ci[side], metaOf(childBuf, level + 1), s, side);
+                            T.small[at] =
+                                packTask(childTask(cs[side], cc[side], ci[side], metaOf(childBuf, level + 1), s, side));
                         } else {
                             atomicOr(&T.ctl[kCtlError], 1);
                         }
@@ -1189,8 +1248,8 @@ __device__ __forceinline__ void histAddLds(uint32_t* h, const PrimBox* recL, con
     const int end = beg + per < count ? beg + per : count;
     BinRun run[3];
     binRunsInit(run);
-    for (int i = beg; i < end; ++i) binRunAdd<false>(h, run, recL[idx[i]], m);
-    binRunsFlush<false>(h, run, m);
+    for (int i = beg; i < end; ++i) binRunAdd(h, run, recL[idx[i]], m);
+    binRunsFlush(h, run, m);
 }
 
 template <int kBT>
@@ -1201,7 +1260,7 @@ __global__ __launch_bounds__(kBT) void sahSmallKernel(SahTables T, int n, uint32
     __shared__ PrimBox recL[kSmallTask];
     __shared__ unsigned char finalBuf[kSmallTask];  // index buffer holding the final serial ranges' positions
     __shared__ unsigned short idxL[2][kSmallTask];
-    __shared__ uint32_t h[histWords<false>()];
+    __shared__ uint32_t h[kHist];
     __shared__ SahResult sres;
     __shared__ SahTask stk[kSmallStack];
     __shared__ SerialTask serBuf[kSmallSerialBatch];
@@ -1214,7 +1273,7 @@ __global__ __launch_bounds__(kBT) void sahSmallKernel(SahTables T, int n, uint32
     int* err = &T.ctl[kCtlError];
     const int listLen = T.ctl[kCtlSmall];
     for (int task = blockIdx.x; task < listLen; task += gridDim.x) {
-        const SahTask root = T.small[task];
+        const SahTask root = unpackTask(T.small[task]);
         if (root.count > kSmallTask) {  // the list holds tasks of at most kSmallTask primitives
             if (threadIdx.x == 0) atomicOr(err, 4);
             continue;
@@ -1240,11 +1299,11 @@ __global__ __launch_bounds__(kBT) void sahSmallKernel(SahTables T, int n, uint32
             const unsigned short* idxS = idxL[buf] + ls;
             const AxisMap m = axisMap(t);
             if (!median) {
-                histInit<false>(h);
+                histInit(h);
                 __syncthreads();
                 histAddLds<kBT>(h, recL, idxS, t.count, m);
                 __syncthreads();
-                if (threadIdx.x < 64) chooseSplit<false>(h, t, m, &sres);
+                if (threadIdx.x < 64) chooseSplit(h, t, m, &sres);
             } else if (threadIdx.x == 0) {
                 sres = medianResult(t);
             }
@@ -1500,7 +1559,7 @@ static void buildSahT(BvhState& b, const typename L::Item* dSrc, int n, hipStrea
             ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(reinterpret_cast<uintptr_t>(base) + off);
             off += count * sizeof(*ptr);
         };
-        SahTask* big = nullptr;
+        StoredTask* big = nullptr;
         take(T.rec[0], static_cast<size_t>(n));
         take(T.rec[1], static_cast<size_t>(n));
         take(order, static_cast<size_t>(n));
@@ -1515,8 +1574,9 @@ static void buildSahT(BvhState& b, const typename L::Item* dSrc, int n, hipStrea
         take(T.ctl, static_cast<size_t>(kCtlWords));
         take(T.bins, 2 * static_cast<size_t>(T.maxBig) * kHist);
         take(T.results, static_cast<size_t>(T.maxBig));
+        take(T.childBoxes, static_cast<size_t>(T.maxBig));
         T.big[0] = big;
-        T.big[1] = reinterpret_cast<SahTask*>(reinterpret_cast<uintptr_t>(big) + T.maxBig * sizeof(SahTask));
+        T.big[1] = reinterpret_cast<StoredTask*>(reinterpret_cast<uintptr_t>(big) + T.maxBig * sizeof(StoredTask));
         return off;
     };
     b.sahArena.reserve(carve(nullptr));

@@ -160,3 +160,68 @@ def test_build_phase_timing_levels(A, scenes):
     finally:
         A.check(L.qr_set_build_phase_timing(1))
     assert all(len(h) == 1 for h in hashes.values())
+
+
+def _split32(p):
+    """The 32-bin split of a range of points (float32, the builder's operation order):
+    (left count, side of each point, or None for a split by position)."""
+    f = np.float32
+    lo, hi = p.min(0), p.max(0)
+    n = len(p)
+    side = max(n // 8, 1)
+    best, found = np.inf, None
+    for a in range(3):
+        ext = f(hi[a] - lo[a])
+        if not ext > 0:
+            continue
+        scale = f(32) / ext
+        if not scale < 3.0e38:
+            continue
+        b = np.clip((p[:, a] - lo[a]) * scale, f(0), f(31)).astype(np.int32)
+        for plane in range(1, 32):
+            m = b < plane
+            nl = int(m.sum())
+            if nl < side or n - nl < side:
+                continue
+
+            def area(q):
+                d = q.max(0) - q.min(0)
+                return f(f(d[0] * d[1] + d[1] * d[2]) + d[2] * d[0])
+
+            cost = f(area(p[m]) * f(nl) + area(p[~m]) * f(n - nl))
+            if cost < best:
+                best, found = cost, m
+    return (n // 2, None) if found is None else (int(found.sum()), found)
+
+
+# 4,097: one split level by chunks; 12,289: a last chunk of one record; 20,000 clustered:
+# uneven sides; the flat cloud has an axis without extent
+@pytest.mark.parametrize("n,shape", [(4097, "box"), (12289, "box"), (20000, "clustered"), (9000, "flat")])
+def test_sah_level_splits(A, n, shape):
+    """Every split of the ranges above 4,096 points is the one that numpy finds, so the
+    children's centroid boxes, from which their bins follow, are exact."""
+    print(f"sah level splits n={n} {shape}", flush=True)
+    rng = np.random.default_rng(n)
+    pts = rng.uniform(-20, 20, (n, 3)).astype(np.float32)
+    if shape == "clustered":
+        pts[n // 3:] = rng.normal(3.0, 0.2, (n - n // 3, 3)).astype(np.float32)
+    if shape == "flat":
+        pts[:, 1] = 2.5
+    b = A.Bvh(1, pts, A.BUILDER_SAH)
+    nodes, ids = b.read()
+    leaf = pts[ids]
+    left = nodes.view(np.int32).reshape(-1, 8)[:, 6]
+    todo, seen = [(0, 0, n)], 0
+    while todo:
+        node, start, count = todo.pop()
+        if count <= 4096:
+            continue
+        l = int(left[node])  # an internal left child is numbered by its range's last slot
+        nl = (l - (n - 1) if l >= n - 1 else l) - start + 1
+        want, m = _split32(leaf[start:start + count])
+        assert nl == want, (start, count)
+        if m is not None:
+            assert m[:nl].all() and not m[nl:].any(), (start, count)
+        todo += [(start + nl - 1, start, nl), (start + nl, start + nl, count - nl)]
+        seen += 1
+    assert seen >= 1
