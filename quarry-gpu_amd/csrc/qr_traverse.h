@@ -69,7 +69,7 @@ constexpr int kMaxCopies = 64;
 // Radius, one walk: counts hits per query and keeps the first `cap` of each query in
 // its slot of `capture` (count * cap keys); returns false when the tree or mode takes
 // the per-lane kernels, which only count (nothing is captured).
-int radiusCaptureCap(int count);  // hits kept per query: 64, fewer for huge query sets
+int radiusCaptureCap(int count);  // hits kept per query: 64 to 2,048 by the set, fewer for huge sets
 bool launchRadiusCapture(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
                          uint64_t* capture, int cap, int* maxCount, hipStream_t s);
 // Writes the CSR segments of the queries the capture does not hold (all queries when
