@@ -337,14 +337,18 @@ QR_API int qr_adjoint_ray(qr_bvh* bvh, const void* rays_dev, int n, const uint64
                           const int* hit_prim_dev, const float* grad_t_dev, float* grad_origins_dev,
                           float* grad_dirs_dev, float* grad_tris_dev);
 /* The same for a mesh of shared vertices: faces_dev holds three vertex indices per
- * triangle (prim_count x 3 i32, scene order, in range), and the triangles' gradients go
- * straight to grad_vertices_dev (3 floats per vertex, accumulated, may be NULL). */
+ * triangle (prim_count x 3 i32, scene order, in range), and the triangles' gradients are
+ * added to grad_vertices_dev (3 floats per vertex, accumulated, may be NULL).  The
+ * per-triangle sums in between take prim_count x 36 bytes of stream-ordered memory. */
 QR_API int qr_adjoint_closest_mesh(qr_bvh* bvh, const float* points_dev, int n, const void* results_dev,
                                    const int* aux_dev, const float* grad_dist2_dev, const int* faces_dev,
                                    float* grad_points_dev, float* grad_vertices_dev);
 QR_API int qr_adjoint_ray_mesh(qr_bvh* bvh, const void* rays_dev, int n, const uint64_t* results_dev,
                                const int* hit_prim_dev, const float* grad_t_dev, const int* faces_dev,
                                float* grad_origins_dev, float* grad_dirs_dev, float* grad_vertices_dev);
+/* The second half of those two, for a caller that keeps the per-triangle gradients: adds n
+ * triangles' corner gradients (n x 9) to their vertices. */
+QR_API int qr_adjoint_vertices(const float* grad_tris_dev, const int* faces_dev, int n, float* grad_vertices_dev);
 
 #ifdef __cplusplus
 }

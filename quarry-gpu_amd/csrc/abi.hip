@@ -904,7 +904,7 @@ int qr_adjoint_closest(qr_bvh* bvh, const float* points, int n, const void* resu
         need(n >= 0, "negative point count");
         need(n == 0 || (points && results && grad_dist2), "null device pointer");
         need(n == 0 || bvh->s.kind == kPrimPoint || aux != nullptr, "saved region / root required");
-        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_items, nullptr, currentStream());
+        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_items, currentStream());
     });
 }
 
@@ -916,7 +916,14 @@ int qr_adjoint_closest_mesh(qr_bvh* bvh, const float* points, int n, const void*
         need(bvh->s.kind == kPrimTri, "mesh adjoint needs a triangle BVH");
         need(faces != nullptr, "null face array");
         need(n == 0 || (points && results && aux && grad_dist2), "null device pointer");
-        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, grad_vertices, faces, currentStream());
+        hipStream_t s = currentStream();
+        if (n == 0 || !grad_vertices) {
+            adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, nullptr, s);
+            return;
+        }
+        CornerScratch corners(bvh->s.n, s);
+        adjointClosest(bvh->s, points, n, results, aux, grad_dist2, grad_points, corners.p, s);
+        addCornersToVertices(corners.p, faces, bvh->s.n, grad_vertices, s);
     });
 }
 
@@ -926,8 +933,7 @@ int qr_adjoint_ray(qr_bvh* bvh, const void* rays, int n, const uint64_t* results
         checkTree(bvh, false);
         need(n >= 0, "negative ray count");
         need(n == 0 || (rays && results && hit_prim && grad_t), "null device pointer");
-        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_tris, nullptr,
-                   currentStream());
+        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_tris, currentStream());
     });
 }
 
@@ -939,8 +945,22 @@ int qr_adjoint_ray_mesh(qr_bvh* bvh, const void* rays, int n, const uint64_t* re
         need(n >= 0, "negative ray count");
         need(faces != nullptr, "null face array");
         need(n == 0 || (rays && results && hit_prim && grad_t), "null device pointer");
-        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, grad_vertices, faces,
-                   currentStream());
+        hipStream_t s = currentStream();
+        if (n == 0 || !grad_vertices) {
+            adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, nullptr, s);
+            return;
+        }
+        CornerScratch corners(bvh->s.n, s);
+        adjointRay(bvh->s, rays, n, results, hit_prim, grad_t, grad_origins, grad_dirs, corners.p, s);
+        addCornersToVertices(corners.p, faces, bvh->s.n, grad_vertices, s);
+    });
+}
+
+int qr_adjoint_vertices(const float* grad_tris, const int* faces, int n, float* grad_vertices) {
+    return guard([&] {
+        need(n >= 0, "negative triangle count");
+        need(n == 0 || (grad_tris && faces && grad_vertices), "null device pointer");
+        addCornersToVertices(grad_tris, faces, n, grad_vertices, currentStream());
     });
 }
 

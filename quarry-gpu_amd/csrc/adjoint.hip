@@ -25,7 +25,8 @@
 //   ray hit t with n = (b - a) x (c - a), w the hit's barycentrics:
 //     dt/do = -n / (n.d),  dt/dd = -t n / (n.d),  dt/dv_i = w_i n / (n.d).
 // Scene-order gradient arrays are accumulated with atomics (several queries may
-// share a primitive), for a mesh straight into its shared vertices.
+// share a primitive).  A mesh's shared vertices take two levels of sums: queries into
+// their triangle's corners, then each triangle's corners once into its vertices.
 #include "qr_adjoint.h"
 
 namespace qr {
@@ -40,21 +41,35 @@ __device__ __forceinline__ void atomicAdd3(float* dst, V3 v) {
     atomicAdd(dst + 2, v.z);
 }
 
-// Adds a triangle's three vertex gradients: to the triangle's nine words, or, with faces
-// (three vertex indices per triangle, scene order), to the shared vertices.  A vertex
-// without weight -- two of the three when the closest point is a vertex -- adds zeros and
-// is passed over: the atomics bound these kernels (262k queries around an icosphere 231
-// us with all nine, 82 into its vertices).
-__device__ __forceinline__ void addVertices(float* __restrict__ dst, const int* __restrict__ faces, int prim, V3 a,
-                                            V3 b, V3 c) {
+__device__ __forceinline__ bool isZero(V3 v) { return (v.x == 0.0f) & (v.y == 0.0f) & (v.z == 0.0f); }
+
+// Adds a triangle's three corner gradients to its nine words.  A corner without weight
+// -- two of the three when the closest point is a vertex -- adds zeros and is passed
+// over: the atomics bound this kernel (262k queries around a 328k-triangle icosphere, us:
+// 231 with all nine words, 81 here).
+__device__ __forceinline__ void addCorners(float* __restrict__ dst, int prim, V3 a, V3 b, V3 c) {
     const V3 v[3] = {a, b, c};
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const bool zero = (v[k].x == 0.0f) & (v[k].y == 0.0f) & (v[k].z == 0.0f);
-        if (zero) continue;
-        const size_t at = static_cast<size_t>(prim) * 3 + k;
-        atomicAdd3(dst + 3 * (faces ? static_cast<size_t>(faces[at]) : at), v[k]);
-    }
+    for (int k = 0; k < 3; ++k)
+        if (!isZero(v[k])) atomicAdd3(dst + (static_cast<size_t>(prim) * 3 + k) * 3, v[k]);
+}
+
+// The triangles' corner gradients into the shared vertices: a thread per corner.  Not the
+// queries straight into the vertices: one flat FP32 sum per vertex carries the rounding of
+// all the queries around it (262,144 queries, relative error against FP64: 320 faces 8.8e-7
+// against 2.5e-7 here, 5,120 faces 2.5e-7 against 1.1e-7) and was no faster (328k
+// triangles: 82 us against 81 and 7 for this pass).
+__global__ void cornersToVerticesKernel(const V3* __restrict__ corners, const int* __restrict__ faces,
+                                        long long count, float* __restrict__ gverts) {
+    const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= count) return;
+    const V3 v = corners[i];
+    if (!isZero(v)) atomicAdd3(gverts + 3 * static_cast<size_t>(faces[i]), v);
+}
+
+__global__ void zeroFloatsKernel(float* __restrict__ p, long long n) {
+    const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < n) p[i] = 0.0f;
 }
 
 // Barycentric weights (of a, b, c) of the closest point for a known region,
@@ -144,8 +159,7 @@ __global__ void saveAuxKernel(const typename L::Item* __restrict__ items, const 
 __global__ void adjTriKernel(const Tri* __restrict__ items, const int* __restrict__ primSlot,
                              const V3* __restrict__ pts, const ClosestResult* __restrict__ res,
                              const int* __restrict__ aux, const float* __restrict__ gout, int n,
-                             float* __restrict__ gpts, float* __restrict__ gitems,
-                             const int* __restrict__ faces) {
+                             float* __restrict__ gpts, float* __restrict__ gitems) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const ClosestResult r = res[i];
@@ -159,7 +173,7 @@ __global__ void adjTriKernel(const Tri* __restrict__ items, const int* __restric
         const V3 p = add(add(scale(tri.a, wa), scale(tri.b, wb)), scale(tri.c, wc));
         const V3 d = scale(sub(q, p), 2.0f * g);
         gq = d;
-        if (gitems) addVertices(gitems, faces, r.prim, scale(d, -wa), scale(d, -wb), scale(d, -wc));
+        if (gitems) addCorners(gitems, r.prim, scale(d, -wa), scale(d, -wb), scale(d, -wc));
     }
     if (gpts) {
         gpts[3 * i + 0] = gq.x;
@@ -291,8 +305,7 @@ __global__ void adjGaussKernel(const Gaussian* __restrict__ items, const int* __
 __global__ void adjRayKernel(const Tri* __restrict__ items, const int* __restrict__ primSlot,
                              const Ray* __restrict__ rays, const uint64_t* __restrict__ res,
                              const int* __restrict__ hitPrim, const float* __restrict__ gout, int n,
-                             float* __restrict__ gorig, float* __restrict__ gdir, float* __restrict__ gitems,
-                             const int* __restrict__ faces) {
+                             float* __restrict__ gorig, float* __restrict__ gdir, float* __restrict__ gitems) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const uint64_t rv = res[i];
@@ -318,7 +331,7 @@ __global__ void adjRayKernel(const Tri* __restrict__ items, const int* __restric
         const V3 k = scale(nrm, g / nd);
         go = scale(k, -1.0f);
         gd = scale(k, -t);
-        if (gitems) addVertices(gitems, faces, prim, scale(k, 1.0f - bu - bv), scale(k, bu), scale(k, bv));
+        if (gitems) addCorners(gitems, prim, scale(k, 1.0f - bu - bv), scale(k, bu), scale(k, bv));
     }
     if (gorig) {
         gorig[3 * i + 0] = go.x;
@@ -366,9 +379,8 @@ int saveClosestAux(BvhState& b, const float* pts, int n, const void* results, in
 }
 
 void adjointClosest(BvhState& b, const float* pts, int n, const void* results, const int* aux,
-                    const float* gout, float* gpts, float* gitems, const int* faces, hipStream_t s) {
+                    const float* gout, float* gpts, float* gitems, hipStream_t s) {
     if (n <= 0) return;
-    if (faces && b.kind != kPrimTri) throw ArgError("mesh adjoint: the tree does not hold triangles");
     ensurePrimSlot(b, s);
     const int grid = blocksFor(n, kBlock);
     const auto* P = reinterpret_cast<const V3*>(pts);
@@ -376,7 +388,7 @@ void adjointClosest(BvhState& b, const float* pts, int n, const void* results, c
     switch (b.kind) {
         case kPrimTri:
             adjTriKernel<<<grid, kBlock, 0, s>>>(reinterpret_cast<const Tri*>(b.items.p), b.primSlot.p, P, R, aux,
-                                                 gout, n, gpts, gitems, faces);
+                                                 gout, n, gpts, gitems);
             break;
         case kPrimPoint:
             adjPointKernel<<<grid, kBlock, 0, s>>>(reinterpret_cast<const V3*>(b.items.p), b.primSlot.p, P, R, gout,
@@ -391,14 +403,37 @@ void adjointClosest(BvhState& b, const float* pts, int n, const void* results, c
 }
 
 void adjointRay(BvhState& b, const void* rays, int n, const uint64_t* results, const int* hitPrim,
-                const float* gout, float* gorig, float* gdir, float* gitems, const int* faces, hipStream_t s) {
+                const float* gout, float* gorig, float* gdir, float* gitems, hipStream_t s) {
     if (n <= 0) return;
     if (b.kind != kPrimTri) throw ArgError("ray adjoint: the tree does not hold triangles");
     ensurePrimSlot(b, s);
     adjRayKernel<<<blocksFor(n, kBlock), kBlock, 0, s>>>(reinterpret_cast<const Tri*>(b.items.p), b.primSlot.p,
                                                          static_cast<const Ray*>(rays), results, hitPrim, gout, n,
-                                                         gorig, gdir, gitems, faces);
+                                                         gorig, gdir, gitems);
     hipCheck(hipGetLastError(), "adjoint ray");
+}
+
+void addCornersToVertices(const float* gcorners, const int* faces, int triangles, float* gverts, hipStream_t s) {
+    if (triangles <= 0) return;
+    const long long corners = 3LL * triangles;
+    cornersToVerticesKernel<<<blocksFor(corners, kBlock), kBlock, 0, s>>>(reinterpret_cast<const V3*>(gcorners), faces,
+                                                                          corners, gverts);
+    hipCheck(hipGetLastError(), "corners to vertices");
+}
+
+CornerScratch::CornerScratch(int triangles, hipStream_t stream) : s(stream) {
+    const long long n = 9LL * triangles;
+    const hipError_t e = hipMallocAsync(reinterpret_cast<void**>(&p), sizeof(float) * static_cast<size_t>(n), s);
+    if (e != hipSuccess) {
+        p = nullptr;
+        (void)hipGetLastError();
+        throw OomError(std::string("hipMallocAsync failed: ") + hipGetErrorString(e));
+    }
+    zeroFloatsKernel<<<blocksFor(n, kBlock), kBlock, 0, s>>>(p, n);
+}
+
+CornerScratch::~CornerScratch() {
+    if (p) (void)hipFreeAsync(p, s);
 }
 
 }  // namespace qr

@@ -158,6 +158,7 @@ def lib():
             "qr_adjoint_ray": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
             "qr_adjoint_closest_mesh": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
             "qr_adjoint_ray_mesh": ([_vp, _vp, _ip, _vp, _vp, _vp, _vp, _vp, _vp, _vp], _ip),
+            "qr_adjoint_vertices": ([_vp, _vp, _ip, _vp], _ip),
         }
         for name, (args, res) in sig.items():
             fn = getattr(L, name)

@@ -102,10 +102,17 @@ class _ClosestDist2(torch.autograd.Function):
         return gp, gi, None, None, None, None
 
 
+def _vertex_grad(shape, idx: torch.Tensor, corners: torch.Tensor) -> torch.Tensor:
+    """The triangles' corner gradients (F, 9) summed into their vertices."""
+    gv = torch.zeros(shape, dtype=torch.float32, device=idx.device)
+    A.check(A.lib().qr_adjoint_vertices(_p(corners), _p(idx), idx.shape[0], _p(gv)))
+    return gv
+
+
 class _MeshDist2(torch.autograd.Function):
-    """Closest points on a mesh of shared vertices: gathers the triangles itself, and the
-    adjoint adds each query's gradient straight to the vertices (a per-triangle gradient
-    and the gather's own sorted backward took three times as long as the adjoint)."""
+    """Closest points on a mesh of shared vertices: gathers the triangles itself, and adds
+    the triangles' gradients to the vertices with one kernel (the gather's own backward
+    sorts its indices first)."""
 
     @staticmethod
     def forward(ctx, points, vertices, faces, order, wide, builder):
@@ -121,10 +128,10 @@ class _MeshDist2(torch.autograd.Function):
         n = points.shape[0]
         g = g_dist2.contiguous().to(torch.float32)
         gp = torch.empty_like(points) if ctx.needs_input_grad[0] else None
-        gv = torch.zeros(ctx.vertices, dtype=torch.float32, device=points.device) if ctx.needs_input_grad[1] else None
+        gt = torch.zeros((idx.shape[0], 9), dtype=torch.float32, device=points.device) if ctx.needs_input_grad[1] else None
         _on_stream()
-        A.check(A.lib().qr_adjoint_closest_mesh(ctx.bvh.h, _p(points), n, _p(res), _p(aux), _p(g), _p(idx), _p(gp),
-                                                _p(gv)))
+        A.check(A.lib().qr_adjoint_closest(ctx.bvh.h, _p(points), n, _p(res), _p(aux), _p(g), _p(gp), _p(gt)))
+        gv = _vertex_grad(ctx.vertices, idx, gt) if gt is not None else None
         return gp, gv, None, None, None, None
 
 
@@ -162,10 +169,10 @@ class _MeshRayHitT(torch.autograd.Function):
         g = torch.nan_to_num(g_t.contiguous().to(torch.float32), nan=0.0, posinf=0.0, neginf=0.0)
         go = torch.empty((n, 3), dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[0] else None
         gd = torch.empty((n, 3), dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[1] else None
-        gv = torch.zeros(ctx.vertices, dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[2] else None
+        gt = torch.zeros((idx.shape[0], 9), dtype=torch.float32, device=rays.device) if ctx.needs_input_grad[2] else None
         _on_stream()
-        A.check(A.lib().qr_adjoint_ray_mesh(ctx.bvh.h, _p(rays), n, _p(res), _p(hit), _p(g), _p(idx), _p(go), _p(gd),
-                                            _p(gv)))
+        A.check(A.lib().qr_adjoint_ray(ctx.bvh.h, _p(rays), n, _p(res), _p(hit), _p(g), _p(go), _p(gd), _p(gt)))
+        gv = _vertex_grad(ctx.vertices, idx, gt) if gt is not None else None
         return go, gd, gv, None, None, None, None, None
 
 
