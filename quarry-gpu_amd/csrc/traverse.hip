@@ -218,6 +218,10 @@ __device__ __forceinline__ bool closer(float d, int id, float bd, int bid) {
     return d < bd || (d == bd && id < bid);
 }
 
+// A query with a NaN coordinate has no closest primitive (index -1) and is not walked: its
+// box distances are 0 and no distance of it ever bounds them, so every node would be opened.
+__device__ __forceinline__ bool hasNaN(V3 p) { return (p.x != p.x) | (p.y != p.y) | (p.z != p.z); }
+
 // ---- k best so far ------------------------------------------------------------------
 // Capacity-K list sorted by (dist2, index) in registers, for any k <= K.  It keeps
 // the K best seen so far and prunes with the K-th: the first k entries are then
@@ -557,7 +561,8 @@ __device__ __forceinline__ void writeList(const KnnList<K>& list, int k, Closest
     for (int s = 0; s < K; ++s) {
         if (s < k) {
             ClosestResult r{0u, -1};
-            if (s < list.n) r = {floatBits(list.d[s]), list.id[s]};
+            // (the fill's id: a NaN distance was counted, not kept)
+            if (s < list.n && list.id[s] != 0x7fffffff) r = {floatBits(list.d[s]), list.id[s]};
             dst[s] = r;
         }
     }
@@ -573,7 +578,7 @@ __device__ __forceinline__ void nearestBinaryWalk(const Node2* __restrict__ node
                                                   KnnList<K>& list, Stack& st, SpillArea& spill,
                                                   int& nodeTests, int& leafTests, int& overflow,
                                                   int& opened, int idBits) {
-    int id = 0;
+    int id = hasNaN(p) ? -1 : 0;
     while (id >= 0) {
         if (kStats) ++opened;
         const Node2 nd = nodes[id];
@@ -714,7 +719,7 @@ __device__ __forceinline__ void nearestWideWalk(const Wide4* __restrict__ wide,
                                                 const int* __restrict__ primIds, V3 p, KnnList<K>& list,
                                                 Stack& st, SpillArea& spill, int& nodeTests, int& leafTests,
                                                 int& overflow, int& opened, int idBits) {
-    int id = 0;
+    int id = hasNaN(p) ? -1 : 0;
     while (id >= 0) {
         if (kStats) ++opened;
         WideEntry e[4];
@@ -883,7 +888,7 @@ struct QuadKnnList {
             const int g = slot * E + j;
             if (g < k) {
                 ClosestResult r{0u, -1};
-                if (g < n) r = {floatBits(d[j]), id[j]};
+                if (g < n && id[j] != 0x7fffffff) r = {floatBits(d[j]), id[j]};
                 dst[g] = r;
             }
         }
@@ -938,7 +943,8 @@ __global__ __launch_bounds__(kBlock) void nearestQuadKernel(
         // with the top of the stack -- that one is requested speculatively and the
         // entry is reloaded only when the offers pruned it.
         WideEntry e = wide[0].c[slot];
-        while (true) {
+        const bool walk = !hasNaN(p);
+        while (walk) {
             if (kStats && slot == 0) ++opened;
             const int ch = e.child;
             const bool leaf = ch < 0 && ch != kWideEmpty;
@@ -1347,7 +1353,7 @@ struct GroupNearest {
         ld = kd = kInfBits;
         lid = kid = kNoPrim;
         if (gl == 0) stk[0] = 0;
-        int sp = 1;
+        int sp = hasNaN(p) ? 0 : 1;
         while (sp > 0) {
             int take = takeOf(sp);
             int node = -1;

@@ -281,3 +281,46 @@ def test_order_is_made_or_not(A, orc, count):  # noqa: F811
                 want = orc.ray_brute(tris, rays, threads=16)
                 for order in (A.ORDER_MORTON, A.ORDER_MORTON_DIRECTION):
                     assert eq(b.raycast(rays, order=order, wide=wide)[0], want)
+
+
+@pytest.mark.parametrize("mode", [0, 1, 2, 3, 5, 6])
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_nan_queries_are_not_walked(A, orc, kind, mode):  # noqa: F811
+    """A NaN coordinate makes every distance NaN: no answer, in any shape, and no node opened
+    (a NaN's box distance is 0 and never bounded by a k-th distance)."""
+    items = scene(kind, 3000, 3)
+    q = np.random.default_rng(4).uniform(-40, 40, (130, 3)).astype(np.float32)
+    nan = q.copy()
+    nan[np.arange(130), np.arange(130) % 3] = np.nan
+    some = q.copy()
+    some[::3] = nan[::3]
+    b = A.Bvh(kind, items)
+    b.build_wide()
+    A.lib().qr_set_traversal_mode(mode)
+    try:
+        for k in (0, 5):
+            want = orc.knn_brute(kind, items, q, k, threads=8)
+            want[::3] = (0, 0xffffffff)
+            for wide in (False, True):
+                def run(p):
+                    return b.knn(p, k, wide=wide, stats=True) if k else b.closest(p, wide=wide, stats=True)
+                got, _, st = run(nan)
+                assert st.nodes_opened == 0, (k, wide)
+                assert np.all(got == np.array([0, 0xffffffff], np.uint32)), (k, wide)
+                assert eq(run(some)[0], want), (k, wide)
+    finally:
+        A.lib().qr_set_traversal_mode(0)
+
+
+def test_nan_queries_of_a_batch(A, orc):  # noqa: F811
+    items = scene(1, 600, 3)
+    q = np.random.default_rng(4).uniform(-40, 40, (100, 3)).astype(np.float32)
+    want = np.concatenate([orc.knn_brute(1, items[a:b], q[c:d], 3, threads=8)
+                           for a, b, c, d in ((0, 200, 0, 50), (200, 600, 50, 100))])
+    q[::7, 2] = np.nan
+    want[::7] = (0, 0xffffffff)
+    batch = A.Batch(1, items, np.array([0, 200, 600], np.int32))
+    for v, name in enumerate(A.BATCH_VARIANTS):
+        plan = A.BatchPlan(batch, q, np.array([0, 50, 100], np.int32), 3, tune=(v, True))
+        plan.run()
+        assert eq(plan.read(), want), name
