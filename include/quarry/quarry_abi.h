@@ -98,7 +98,8 @@ QR_API const char* qr_last_error(void);
 QR_API int qr_describe(char* buf, int len);
 /* warmupBuildGPU / warmupQueryGPU (src/gpu/gpu_bvh.h:122, :343) */
 QR_API int qr_warmup(void);
-/* Shape of the 4-wide traversal, process-wide: 0 automatic (closest / kNN below
+/* Shape of the traversal, process-wide (modes 2 to 6 name shapes of the 4-wide walks; 0 and
+ * 1 hold for binary nodes too): 0 automatic (closest / kNN below
  * 65,536 queries by query count, leaf kind and k; from 65,536 on, the first call
  * for a tree, k class and query-count octave times 16 and 32 lanes and one wave per
  * query on its own queries and keeps the fastest; radius 64 to 16 lanes per query by

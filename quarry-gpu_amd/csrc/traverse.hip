@@ -2151,7 +2151,7 @@ bool batchQueryOrder(const V3* points, const int* qOff, int n, int scenes, int m
 }
 
 // 0 automatic, 1 one lane per query, 2 four lanes per query, 3 one wave per query,
-// 4 closest / kNN and rays tuned whatever the query count
+// 4 closest / kNN and rays tuned whatever the query count, 5 / 6 16 / 32 lanes per query
 int gTraversalMode = 0;
 
 // Shapes of a walk over 4-wide nodes.
@@ -2420,7 +2420,7 @@ static void launchShape(int shape, const TraverseArgs& a, const V3* pts, int cou
 // terrain closest 257 queries 675 us against 22, 100k 937 against 221, 400k 1150 against
 // 656; 262k Gaussians kNN8 100k 1527 against 480) and ahead for points, whose leaf test is
 // the cheapest, from about 131,072 queries (1M points closest 100k 215 us against 171, 400k
-// 344 against 591).
+// 344 against 591).  Mode 1 forces one lane here too.
 template <typename L>
 static int binaryLaneFrom() {
     return L::kKind == 1 ? 131072 : INT_MAX;
@@ -2513,7 +2513,7 @@ static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int
                             ClosestResult* out, hipStream_t s) {
     const auto* prims = static_cast<const typename L::Item*>(a.items);
     const bool deep = a.depth > kGroupDepth;
-    if (!a.wide && !deep && count < binaryLaneFrom<L>()) {
+    if (!a.wide && !deep && gTraversalMode != 1 && count < binaryLaneFrom<L>()) {
         launchShape<L, K>(defaultShape<L, K>(count), a, pts, count, k, outStride, out, a.stats, s);
         return;
     }

@@ -324,3 +324,22 @@ def test_nan_queries_of_a_batch(A, orc):  # noqa: F811
         plan = A.BatchPlan(batch, q, np.array([0, 50, 100], np.int32), 3, tune=(v, True))
         plan.run()
         assert eq(plan.read(), want), name
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_lane_mode_on_binary_nodes(A, orc, kind):  # noqa: F811
+    """Mode 1 walks binary nodes one lane per query too.  That walk counts a test per opened
+    node; the groups count the entries that pass."""
+    items = scene(kind, 3000, 3)
+    q = np.random.default_rng(4).uniform(-40, 40, (500, 3)).astype(np.float32)
+    b = A.Bvh(kind, items)
+    for k in (0, 5):
+        want = orc.knn_brute(kind, items, q, k, threads=8)
+        for mode in (0, 1):
+            A.lib().qr_set_traversal_mode(mode)
+            try:
+                got, _, st = b.knn(q, k, stats=True) if k else b.closest(q, stats=True)
+            finally:
+                A.lib().qr_set_traversal_mode(0)
+            assert eq(got, want)
+            assert (st.node_tests == st.nodes_opened) == (mode == 1), (k, mode)
