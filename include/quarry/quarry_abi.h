@@ -246,7 +246,8 @@ QR_API int qr_radius_read(const qr_csr* r, int* offsets_host, uint64_t* keys_hos
  * (src/gpu/gpu_bvh.h:255-262, :296-301). */
 QR_API int qr_points_device_ptrs(const qr_points* pts, float** points_dev, void** results_dev);
 QR_API int qr_radius_device_ptrs(const qr_csr* r, int** offsets_dev, uint64_t** keys_dev);
-/* destroyRadiusBufferGPU */
+/* destroyRadiusBufferGPU.  Waits for the device if the device pointers were asked for (their
+ * readers may still be queued), for nothing otherwise. */
 QR_API int qr_radius_destroy(qr_csr* r);
 /* lastQueryStatsGPU */
 QR_API int qr_last_query_stats(qr_traversal_stats* out);

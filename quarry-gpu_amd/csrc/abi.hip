@@ -2,6 +2,7 @@
 // management, host<->device transfers, timing and error mapping around the HIP
 // kernels.  No kernel math lives here.
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -54,6 +55,9 @@ struct qr_csr {
     DevBuf<uint64_t> keys;
     int count = 0;
     int total = 0;
+    // whether the device pointers were handed out: only then can work that this library
+    // has not waited for read the buffers
+    mutable std::atomic<bool> shared{false};
 };
 
 // Pinned host words for the small device-to-host reads of a call (per host thread).
@@ -600,6 +604,7 @@ int qr_points_device_ptrs(const qr_points* p, float** points_dev, void** results
 int qr_radius_device_ptrs(const qr_csr* r, int** offsets_dev, uint64_t** keys_dev) {
     return guard([&] {
         need(r != nullptr, "null radius result");
+        r->shared = true;
         if (offsets_dev) *offsets_dev = r->offsets.p;
         if (keys_dev) *keys_dev = r->keys.p;
     });
@@ -1513,7 +1518,10 @@ int qr_radius(const qr_bvh* bvh, qr_points* p, float radius, int collectStats, i
             if (total < 0 || maxSeg < 0) throw DeviceError("radius: summary words not written");
             res->total = total;
             const bool compacted = guess > 0 && total <= guess;
-            if (!compacted) res->keys.alloc(static_cast<size_t>(total > 0 ? total : 1));
+            if (!compacted) {
+                QuietFree quiet(true);  // only this stream has touched a short guess's keys
+                res->keys.alloc(static_cast<size_t>(total > 0 ? total : 1));
+            }
             p->rKeysGuess = total + total / 8 + 64;
             kev.record(2, s);
             if (total > 0) {
@@ -1571,7 +1579,12 @@ int qr_radius_read(const qr_csr* r, int* offsets, uint64_t* keys) {
 }
 
 int qr_radius_destroy(qr_csr* r) {
-    return guard([&] { destroyHandle(r); });
+    return guard([&] {
+        if (!r) return;
+        // qr_radius and qr_radius_read return with their work done
+        QuietFree quiet(!r->shared || hipDeviceSynchronize() == hipSuccess);
+        delete r;
+    });
 }
 
 int qr_last_query_stats(qr_traversal_stats* out) {

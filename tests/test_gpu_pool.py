@@ -87,3 +87,50 @@ def test_threads_and_streams(A, orc):  # noqa: F811
     for t in threads:
         t.join()
     assert not wrong, wrong
+
+
+def side_stream_work(stream, ms=300):
+    """Queues about that much work on the stream: products of one size, timed once."""
+    with torch.cuda.stream(stream):
+        m = torch.ones((4096, 4096), device="cuda")
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        out = torch.mm(m, m)
+        a.record()
+        torch.mm(m, m, out=out)
+        b.record()
+        b.synchronize()
+        for _ in range(int(ms / max(a.elapsed_time(b), 0.05)) + 1):
+            torch.mm(m, m, out=out)
+        done = torch.cuda.Event()
+        done.record()
+    return done
+
+
+def test_radius_results_do_not_wait_for_other_streams(A, orc):  # noqa: F811
+    """A radius result whose device pointers nobody asked for has no reader left once the call
+    returned: neither destroying it nor a grown key buffer inside the call waits for the work
+    of other streams."""
+    L = A.lib()
+    rng = np.random.default_rng(5)
+    items = rng.uniform(-10, 10, (20000, 3)).astype(np.float32)
+    q = rng.uniform(-10, 10, (500, 3)).astype(np.float32)
+    b = A.Bvh(1, items)
+    pb = A.PointBuffer(q)
+    want = {r: orc.radius_brute(1, items, q, r, threads=8) for r in (0.5, 1.5)}
+    pb.radius(b, 1.5, wide=False)  # (the call's own buffers have grown)
+    pb.radius(b, 0.5, wide=False)  # (and its guess of the number of hits is small)
+    stream = torch.cuda.Stream()
+    done = side_stream_work(stream)
+    for r in (0.5, 1.5, 1.5, 0.5):
+        _, offs, keys = pb.radius(b, r, wide=False, keep=True)
+        assert eq(offs, want[r][0]) and eq(keys, want[r][1])
+    assert not done.query()
+    done.synchronize()
+
+    done = side_stream_work(stream)  # asked for, they may have readers on any stream
+    csr, ms, offs, keys = (ctypes.c_void_p(), ctypes.c_double(), ctypes.c_void_p(), ctypes.c_void_p())
+    A.check(L.qr_radius(b.h, pb.h, 0.5, 0, A.ORDER_INPUT, 0, ctypes.byref(csr), ctypes.byref(ms)))
+    A.check(L.qr_radius_device_ptrs(csr, ctypes.byref(offs), ctypes.byref(keys)))
+    assert not done.query()
+    A.check(L.qr_radius_destroy(csr))
+    assert done.query()
