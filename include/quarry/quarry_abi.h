@@ -133,8 +133,10 @@ QR_API int qr_set_stream(void* hip_stream);
  * counterpart: the reference API only takes host arrays. */
 QR_API int qr_dev_alloc(size_t bytes, void** out);
 QR_API int qr_dev_free(void* ptr);
-/* Buffers the library frees are kept for its next ones, at most 4 GiB a device and none
- * much longer than 10 s; this gives the current device's back to the runtime now. */
+/* Buffers the library frees are kept for its next ones, at most 4 GiB a device; those unused
+ * for 10 s go back to the runtime when the library next allocates or frees one, and all of
+ * the current device's now with this call (a program that falls idle, or goes on with
+ * queries of resident buffers only, calls it to release them). */
 QR_API int qr_dev_trim(void);
 QR_API int qr_dev_upload(void* dst, const void* src_host, size_t bytes);
 QR_API int qr_dev_download(void* dst_host, const void* src, size_t bytes);

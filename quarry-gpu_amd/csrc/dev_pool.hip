@@ -13,9 +13,11 @@
 //     waited itself (QuietFree).  A cached block may therefore be handed to any thread and
 //     used on any stream at once;
 //   * blocks are kept per device and handed out again on that device only;
-//   * at most kMaxCached bytes per device stay cached (the longest unused go first), none
-//     longer than kMaxIdle beyond the next call, and an allocation that fails gives all of
-//     them back before it tries again; qr_dev_trim gives them back on request;
+//   * at most kMaxCached bytes per device stay cached (the longest unused go first).  Every
+//     allocation and every free gives back the blocks that have lain for longer than
+//     kMaxIdle (there is no thread that does: a program that only queries resident buffers,
+//     or stops, keeps them until then); an allocation that fails gives all of them back
+//     before it tries again; qr_dev_trim gives them back on request;
 //   * sizes are rounded up by at most an eighth, and a request takes a cached block of up
 //     to one and a half times its size;
 //   * nothing is kept for a pointer the cache did not hand out: devFree passes it on.
@@ -23,6 +25,7 @@
 #include <list>
 #include <map>
 #include <mutex>
+#include <new>
 #include <unordered_map>
 
 #include "qr_internal.h"
@@ -78,18 +81,22 @@ void uncache(Cached& c, Block& b) {
 }
 
 // Cached blocks to give back now, taken off the books: all of the device's, or those idle
-// for too long and, while more than kMaxCached are cached, the longest unused.
+// for too long and, while more than kMaxCached are cached, the longest unused.  (Without
+// memory for the list the rest stays cached.)
 std::vector<void*> excess(Pool& P, int dev, bool all) {
     std::vector<void*> out;
     Cached& c = P.cached[dev];
     const auto now = Clock::now();
-    while (!c.byAge.empty()) {
-        void* p = c.byAge.front();
-        const auto it = P.blocks.find(p);
-        if (!all && c.bytes <= kMaxCached && now - it->second.since <= kMaxIdle) break;
-        uncache(c, it->second);
-        P.blocks.erase(it);
-        out.push_back(p);
+    try {
+        while (!c.byAge.empty()) {
+            void* p = c.byAge.front();
+            const auto it = P.blocks.find(p);
+            if (!all && c.bytes <= kMaxCached && now - it->second.since <= kMaxIdle) break;
+            out.push_back(p);
+            uncache(c, it->second);
+            P.blocks.erase(it);
+        }
+    } catch (const std::bad_alloc&) {
     }
     return out;
 }
@@ -115,17 +122,20 @@ void* devAlloc(size_t bytes) {
     hipCheck(hipGetDevice(&dev), "get device");
     const size_t want = roundUp(bytes > 0 ? bytes : 1);
     Pool& P = pool();
+    void* p = nullptr;
+    std::vector<void*> back;
     {
         std::lock_guard<std::mutex> lock(P.m);
         Cached& c = P.cached[dev];
         const auto it = c.bySize.lower_bound(want);
         if (it != c.bySize.end() && it->first <= want + want / 2) {
-            void* p = it->second;
+            p = it->second;
             uncache(c, P.blocks[p]);
-            return p;
         }
+        back = excess(P, dev, false);
     }
-    void* p = nullptr;
+    giveBack(back);
+    if (p) return p;
     hipError_t e = hipMalloc(&p, want);
     if (e != hipSuccess) {
         (void)hipGetLastError();

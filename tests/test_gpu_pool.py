@@ -2,6 +2,7 @@
 uses them, also with several threads and streams, and are given back."""
 import ctypes
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -134,3 +135,44 @@ def test_radius_results_do_not_wait_for_other_streams(A, orc):  # noqa: F811
     assert not done.query()
     A.check(L.qr_radius_destroy(csr))
     assert done.query()
+
+
+def used(torch_free_before):
+    return torch_free_before - torch.cuda.mem_get_info()[0]
+
+
+def alloc(A, n):  # noqa: F811
+    p = ctypes.c_void_p()
+    A.check(A.lib().qr_dev_alloc(n, ctypes.byref(p)))
+    return p
+
+
+def test_cached_blocks_are_bounded_and_given_back(A):  # noqa: F811
+    """Freed blocks are kept (the same address comes back), at most 4 GiB of them, none past
+    10 s once another buffer is allocated, and trim returns them to the runtime."""
+    L = A.lib()
+    A.check(L.qr_dev_trim())
+    p = alloc(A, 64 << 20)
+    A.check(L.qr_dev_free(p))
+    q = alloc(A, 64 << 20)
+    assert p.value == q.value
+    A.check(L.qr_dev_free(q))
+    A.check(L.qr_dev_trim())
+    free0 = torch.cuda.mem_get_info()[0]
+
+    held = [alloc(A, 1 << 30) for _ in range(6)]
+    slack = 64 << 20  # other allocations on the card
+    assert used(free0) >= (6 << 30) - slack
+    for h in held:
+        A.check(L.qr_dev_free(h))
+    assert (3 << 30) - slack <= used(free0) <= (4 << 30) + slack
+    A.check(L.qr_dev_trim())
+    assert used(free0) <= slack
+
+    A.check(L.qr_dev_free(alloc(A, 1 << 30)))
+    assert used(free0) >= (1 << 30) - slack
+    print("idle", flush=True)
+    time.sleep(10.5)
+    small = alloc(A, 4096)  # nothing is freed here: allocating is enough
+    assert used(free0) <= slack
+    A.check(L.qr_dev_free(small))
