@@ -18,8 +18,8 @@
 //     kMaxIdle (there is no thread that does: a program that only queries resident buffers,
 //     or stops, keeps them until then); an allocation that fails gives all of them back
 //     before it tries again; qr_dev_trim gives them back on request;
-//   * sizes are rounded up by at most an eighth, and a request takes a cached block of up
-//     to one and a half times its size;
+//   * sizes are rounded up to multiples of 512 bytes and, from 4 KiB on, by at most an
+//     eighth; a request takes a cached block of up to one and a half times its size;
 //   * nothing is kept for a pointer the cache did not hand out: devFree passes it on.
 #include <chrono>
 #include <list>
@@ -68,7 +68,7 @@ Pool& pool() {
 
 size_t roundUp(size_t bytes) {
     size_t step = 512;
-    while (step * 8 < bytes) step <<= 1;
+    while (step * 16 <= bytes) step <<= 1;
     return (bytes + step - 1) / step * step;
 }
 

@@ -176,3 +176,15 @@ def test_cached_blocks_are_bounded_and_given_back(A):  # noqa: F811
     small = alloc(A, 4096)  # nothing is freed here: allocating is enough
     assert used(free0) <= slack
     A.check(L.qr_dev_free(small))
+
+
+# from 4 KiB on a block is at most an eighth larger than asked for
+@pytest.mark.parametrize("n", [4097, 131073, (1 << 20) + 1, (9 << 20) + 1])
+def test_rounding(A, n):  # noqa: F811
+    L = A.lib()
+    A.check(L.qr_dev_trim())
+    p = alloc(A, n)
+    A.check(L.qr_dev_free(p))
+    q = alloc(A, n + n // 8 + 512)  # more than the block can hold: another one
+    assert q.value != p.value
+    A.check(L.qr_dev_free(q))
