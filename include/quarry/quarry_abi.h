@@ -111,6 +111,9 @@ QR_API int qr_warmup(void);
  * every count (6), other queries as in mode 0.  Results are identical in every
  * mode.  No reference counterpart (a tuning knob of this backend). */
 QR_API int qr_set_traversal_mode(int mode);
+/* How many shapes chosen by timing are kept now; a tree's go when it is rebuilt, edited in
+ * its topology or destroyed.  (Tests use it to see what a call chose by itself.) */
+QR_API int qr_kept_shapes(int* out);
 /* LBVH build: how many frontier nodes a workgroup (or group of workgroups) may hand
  * up to the next level, process-wide, 0..32 (default 32).  Units with more send
  * their nodes through the device-wide arrival protocol instead; 0 sends every node

@@ -201,6 +201,7 @@ TraverseArgs argsFor(const BvhState& b, bool wide, bool arm = true) {
     a.nodes = b.nodes.p;
     a.nodeCount = b.nodeCount;
     a.depth = b.depth;
+    a.serial = b.serial;
     a.wideNodes = b.wide.p;
     a.wideCount = b.wideCount;
     a.items = b.items.p;
@@ -319,6 +320,13 @@ int qr_set_traversal_mode(int mode) {
     return guard([&] {
         need(mode >= 0 && mode <= 6, "traversal mode must be 0 to 6");
         setTraversalMode(mode);
+    });
+}
+
+int qr_kept_shapes(int* out) {
+    return guard([&] {
+        need(out != nullptr, "null output pointer");
+        *out = keptShapes();
     });
 }
 
@@ -448,7 +456,10 @@ int qr_bvh_build_device(int prim, int builder, const void* items, int n, qr_buil
 }
 
 int qr_bvh_destroy(qr_bvh* bvh) {
-    return guard([&] { destroyHandle(bvh); });
+    return guard([&] {
+        if (bvh) forgetShapes(bvh->s.serial);
+        destroyHandle(bvh);
+    });
 }
 
 int qr_bvh_get_info(const qr_bvh* bvh, qr_bvh_info* out) {

@@ -1473,10 +1473,7 @@ static void buildLbvhT(BvhState& b, const typename L::Item* dSrc, int n, hipStre
         t->sahBinMs = t->sahSplitMs = t->sahPartMs = 0.0;
         t->totalMs = ev.ms(0, 4);
     }
-    b.primSlotValid = false;
-    b.depthValid = false;
-    b.wideValid = false;
-    b.wideCount = 0;
+    newTopology(b);
 }
 
 void setFrontierCap(int cap) {

@@ -4,6 +4,7 @@
 #include "qr_traverse.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace qr {
 
@@ -295,6 +296,16 @@ __global__ void checkDepthKernel(const Node2* __restrict__ nodes, const int* __r
 }
 
 }  // namespace
+
+void newTopology(BvhState& b) {
+    static std::atomic<uint64_t> last{0};
+    forgetShapes(b.serial);
+    b.serial = ++last;
+    b.primSlotValid = false;
+    b.depthValid = false;
+    b.wideValid = false;
+    b.wideCount = 0;
+}
 
 void reserveWide(BvhState& b) {
     if (b.n < 2) throw ArgError("buildWideNodes: tree is empty");

@@ -35,6 +35,7 @@ struct BvhState {
     int n = 0;
     int nodeCount = 0;
     int depth = 0;
+    uint64_t serial = 0;            // another one for every topology ever built in the process
 
     DevBuf<Node2> nodes;            // 2n-1
     DevBuf<unsigned char> items;    // leaf order, n * itemSize(kind)
@@ -126,6 +127,9 @@ void buildLbvhDevice(BvhState& b, int kind, const void* dItems, int n, hipStream
                      BuildTimingsC* t);
 void buildSahDevice(BvhState& b, int kind, const void* dItems, int n, hipStream_t s,
                     BuildTimingsC* t);
+
+// A builder has written a new topology: what was derived from the old one no longer holds.
+void newTopology(BvhState& b);
 
 // Per-node depth by pointer jumping over the parent array (root 0).
 void computeDepth(BvhState& b, hipStream_t s);

@@ -16,6 +16,7 @@ struct TraverseArgs {
     const void* items = nullptr;        // leaf-ordered primitives
     const int* primIds = nullptr;       // leaf slot -> scene index
     int depth = 0;                      // of the binary tree
+    uint64_t serial = 0;                // of its topology
     const uint32_t* order = nullptr;    // optional visiting order (lane i -> query order[i])
     unsigned long long* stats = nullptr;  // optional [node tests, leaf tests, overflows]
     // false: the walk shape comes from an earlier tuning of the same tree and size
@@ -51,6 +52,11 @@ void mortonOrder(const float* base, int stride, int count, int boxMode, SortWork
 // than a walk in input order loses, also when the input order is random.
 enum WalkKind : int { kWalkClosest = 0, kWalkKnn = 1, kWalkRadius = 2, kWalkRays = 3 };
 bool orderingPays(const TraverseArgs& a, WalkKind walk, int count);
+
+// Walk shapes chosen by timing are kept by the topology's serial number; its tree drops
+// them when it is rebuilt or destroyed.
+void forgetShapes(uint64_t serial);
+int keptShapes();
 
 void launchRays(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, hipStream_t s);
 // Same, also writing the hit triangle's scene index (-1 for a miss) to hitPrim.

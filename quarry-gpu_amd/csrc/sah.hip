@@ -1709,10 +1709,7 @@ static void buildSahT(BvhState& b, const typename L::Item* dSrc, int n, hipStrea
         t->totalMs = ev.ms(0, 5);
     }
     for (hipEvent_t e : lev) giveEvent(e);
-    b.primSlotValid = false;
-    b.depthValid = false;
-    b.wideValid = false;
-    b.wideCount = 0;
+    newTopology(b);
 }
 
 void buildSahDevice(BvhState& b, int kind, const void* dItems, int n, hipStream_t s, BuildTimingsC* t) {

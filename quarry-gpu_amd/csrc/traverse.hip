@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -2174,18 +2175,24 @@ constexpr int kGroupDepth = 64;
 constexpr int kTuneFrom = 65536;
 
 struct TuneKey {
-    const void* tree;
-    int wideCount, kind, K, octave;
+    uint64_t tree;  // the topology's serial number: the next tree in the same memory is another one
+    int kind, K, octave;
     bool operator<(const TuneKey& o) const {
-        if (tree != o.tree) return tree < o.tree;
-        if (wideCount != o.wideCount) return wideCount < o.wideCount;
-        if (kind != o.kind) return kind < o.kind;
-        if (K != o.K) return K < o.K;
-        return octave < o.octave;
+        return std::tie(tree, kind, K, octave) < std::tie(o.tree, o.kind, o.K, o.octave);
     }
 };
 static std::mutex gTuneMutex;
 static std::map<TuneKey, int> gTuned;
+
+void forgetShapes(uint64_t serial) {
+    std::lock_guard<std::mutex> lock(gTuneMutex);
+    gTuned.erase(gTuned.lower_bound({serial, 0, 0, 0}), gTuned.lower_bound({serial + 1, 0, 0, 0}));
+}
+
+int keptShapes() {
+    std::lock_guard<std::mutex> lock(gTuneMutex);
+    return static_cast<int>(gTuned.size());
+}
 
 // G lanes per ray, over the 4-wide nodes or, with a.wide false, the binary ones.
 template <int G, bool kSave, typename Nodes>
@@ -2254,7 +2261,7 @@ static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t*
     }
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.wideNodes, a.wideCount, 100 + (kSave ? 1 : 0), 0, octave};
+    const TuneKey key{a.serial, 100 + (kSave ? 1 : 0), 0, octave};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
         const auto it = gTuned.find(key);
@@ -2450,7 +2457,7 @@ static TunedShape tunedShape(const TraverseArgs& a, const V3* pts, int count, in
                              ClosestResult* out, hipStream_t s) {
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.wideNodes, a.wideCount, L::kKind, K, octave};
+    const TuneKey key{a.serial, L::kKind, K, octave};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
         const auto it = gTuned.find(key);
@@ -2499,7 +2506,7 @@ template <typename L, int K>
 static int cachedShape(const TraverseArgs& a, int count) {
     int octave = 0;
     while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.wideNodes, a.wideCount, L::kKind, K, octave};
+    const TuneKey key{a.serial, L::kKind, K, octave};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
         const auto it = gTuned.find(key);

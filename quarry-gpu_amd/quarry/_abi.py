@@ -94,6 +94,7 @@ def lib():
             "qr_last_error": ([], ctypes.c_char_p),
             "qr_describe": ([ctypes.c_char_p, _ip], _ip),
             "qr_warmup": ([], _ip),
+            "qr_kept_shapes": ([_vp], _ip),
             "qr_set_stream": ([_vp], _ip),
             "qr_dev_alloc": ([ctypes.c_size_t, _vp], _ip),
             "qr_dev_free": ([_vp], _ip),

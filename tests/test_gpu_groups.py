@@ -1,5 +1,7 @@
 """The walks that give a query a group of lanes, at the sizes where a group, a wave or the
 k-best list is only partly filled; results against the brute-force oracle, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -123,8 +125,6 @@ def unusual_rays(rng, items, n):
 # the counts at which the lanes per ray change, and one ray
 @pytest.mark.parametrize("count", [1, 3071, 3072, 12289, 49153, 393217])
 def test_ray_group_edges(A, orc, count):  # noqa: F811
-    import ctypes
-
     print(f"rays={count}", flush=True)
     rng = np.random.default_rng(count)
     items = random_tris(rng, 400, size=8.0)
@@ -343,3 +343,33 @@ def test_lane_mode_on_binary_nodes(A, orc, kind):  # noqa: F811
                 A.lib().qr_set_traversal_mode(0)
             assert eq(got, want)
             assert (st.node_tests == st.nodes_opened) == (mode == 1), (k, mode)
+
+
+def test_timed_shapes_belong_to_one_tree(A, orc):  # noqa: F811
+    """The next tree in the memory of a destroyed, rebuilt or edited one is timed again."""
+    def kept():
+        n = ctypes.c_int()
+        A.check(A.lib().qr_kept_shapes(ctypes.byref(n)))
+        return n.value
+
+    items = scene(1, 3000, 3)
+    q = np.random.default_rng(4).uniform(-40, 40, (65536, 3)).astype(np.float32)
+    want = orc.knn_brute(1, items, q, 0, threads=16)
+    before = kept()
+    for _ in range(2):  # the second tree gets the first one's memory
+        b = A.Bvh(1, items)
+        b.build_wide()
+        for _ in range(2):
+            assert eq(b.closest(q, wide=True)[0], want)
+            assert kept() == before + 1
+        b.build_wide()  # the same topology: nothing to time again
+        assert kept() == before + 1
+        b.knn(q, 3, wide=True)
+        assert kept() == before + 2
+        b.update(items[:2000], deleted=np.arange(2000, 3000))
+        assert kept() == before
+        b.build_wide()
+        assert eq(b.closest(q, wide=True)[0], orc.knn_brute(1, items[:2000], q, 0, threads=16))
+        assert kept() == before + 1
+        b.close()
+        assert kept() == before
