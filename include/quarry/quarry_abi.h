@@ -100,9 +100,10 @@ QR_API int qr_describe(char* buf, int len);
 QR_API int qr_warmup(void);
 /* Shape of the traversal, process-wide (modes 2 to 6 name shapes of the 4-wide walks; 0 and
  * 1 hold for binary nodes too): 0 automatic (closest / kNN below
- * 65,536 queries by query count, leaf kind and k; from 65,536 on, the first call
- * for a tree, k class and query-count octave times 16 and 32 lanes and one wave per
- * query on its own queries and keeps the fastest; radius 64 to 16 lanes per query by
+ * 65,536 queries by query count, leaf kind and k; from 65,536 on, the second call
+ * for a tree, k class and query-count octave (the first, if no like call on a tree of
+ * that leaf kind and size was timed yet) times 16 and 32 lanes and one wave per query
+ * on its own queries and keeps the fastest; radius 64 to 16 lanes per query by
  * query count; rays 64 to 8 lanes per ray by ray count, one lane from 393,216 on), 1 one lane per
  * query or ray, 2 four lanes per query, 3 one wave per query or ray, 4 as 0 but closest
  * / kNN and rays tuned at every count (rays: one lane or one wave), 5 / 6

@@ -2170,8 +2170,13 @@ constexpr int kGroupDepth = 64;
 // the query count alone does not tell: 262,144 closest queries on the terrain run fastest
 // 16 lanes per query (410 us, one wave per query 597), as many in and around an icosphere
 // -- long walks of very different lengths -- one wave per query (970 us against 1312).
-// From kTuneFrom queries on, the first call for a (tree, k class, query count octave)
-// times the three group shapes on its own queries and keeps the fastest (tunedShape).
+// From kTuneFrom queries on a call for a (tree, k class, query count octave) times the
+// three group shapes on its own queries and keeps the fastest (tunedShape): the second such
+// call, or the first when no like call -- a tree of that leaf kind and size octave, that k
+// class and count octave -- has been timed yet.  The first call else takes the shape of the
+// last like call that was: a mesh that moves is a new tree every step, walked once (262,144
+// queries around a 328k-triangle icosphere rebuilt each step: 2780 us a step with the
+// timing in it, 1600 without).
 constexpr int kTuneFrom = 65536;
 
 struct TuneKey {
@@ -2182,7 +2187,35 @@ struct TuneKey {
     }
 };
 static std::mutex gTuneMutex;
-static std::map<TuneKey, int> gTuned;
+static std::map<TuneKey, int> gTuned;  // by tree: the shape, or kCalledOnce (not timed yet)
+static std::map<TuneKey, int> gLike;   // by the tree's size octave: the last shape timed
+constexpr int kCalledOnce = -1;
+constexpr size_t kKeptMax = 4096;  // entries of gTuned; more are of trees in their thousands, all forgotten
+
+static int octaveOf(int count) {
+    int octave = 0;
+    while ((2LL << octave) <= count) ++octave;
+    return octave;
+}
+
+// The shape kept for this call (gTuneMutex held), or that of the last like call, or kCalledOnce.
+static int keptShape(const TuneKey& key, int wideCount) {
+    const auto own = gTuned.find(key);
+    if (own != gTuned.end() && own->second != kCalledOnce) return own->second;
+    TuneKey like = key;
+    like.tree = static_cast<uint64_t>(octaveOf(wideCount));
+    const auto it = gLike.find(like);
+    return it != gLike.end() ? it->second : kCalledOnce;
+}
+
+static void keepShape(const TuneKey& key, int wideCount, int shape) {
+    std::lock_guard<std::mutex> lock(gTuneMutex);
+    if (gTuned.size() >= kKeptMax) gTuned.clear();
+    gTuned[key] = shape;
+    TuneKey like = key;
+    like.tree = static_cast<uint64_t>(octaveOf(wideCount));
+    gLike[like] = shape;
+}
 
 void forgetShapes(uint64_t serial) {
     std::lock_guard<std::mutex> lock(gTuneMutex);
@@ -2191,7 +2224,9 @@ void forgetShapes(uint64_t serial) {
 
 int keptShapes() {
     std::lock_guard<std::mutex> lock(gTuneMutex);
-    return static_cast<int>(gTuned.size());
+    int kept = 0;
+    for (const auto& e : gTuned) kept += e.second != kCalledOnce ? 1 : 0;
+    return kept;
 }
 
 // G lanes per ray, over the 4-wide nodes or, with a.wide false, the binary ones.
@@ -2259,9 +2294,7 @@ static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t*
         if (count < 49152) return kShapeGroup16;
         return count < kRayLaneFrom ? kShapeGroup8 : kShapeLane;
     }
-    int octave = 0;
-    while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.serial, 100 + (kSave ? 1 : 0), 0, octave};
+    const TuneKey key{a.serial, 100 + (kSave ? 1 : 0), 0, octaveOf(count)};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
         const auto it = gTuned.find(key);
@@ -2278,7 +2311,7 @@ static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t*
     ev.sync(3);
     const int best = ev.ms(2, 3) < ev.ms(0, 1) ? kShapeWave : kShapeLane;
     std::lock_guard<std::mutex> lock(gTuneMutex);
-    if (gTuned.size() >= 4096) gTuned.clear();
+    if (gTuned.size() >= kKeptMax) gTuned.clear();
     gTuned[key] = best;
     return best;
 }
@@ -2440,8 +2473,8 @@ static int defaultShape(int count) {
     return lanes == 64 ? kShapeWave : (lanes == 32 ? kShapeGroup32 : kShapeGroup16);
 }
 
-// The shape for this tree and size class, timed on the first call's own queries; that call's
-// results are then written already (done), every shape writing the same.  From
+// The shape for this tree and size class (see kTuneFrom); a call that times has its results
+// written already (done), every shape writing the same.  From
 // kTuneSplitFrom queries on each shape walks a third of the queries, so that the first call
 // on a new tree costs about what a later one does -- a mesh that moves is a new tree every
 // step; below, a third would not fill the device and say little, and each shape walks all.
@@ -2455,13 +2488,16 @@ struct TunedShape {
 template <typename L, int K>
 static TunedShape tunedShape(const TraverseArgs& a, const V3* pts, int count, int k, int outStride,
                              ClosestResult* out, hipStream_t s) {
-    int octave = 0;
-    while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.serial, L::kKind, K, octave};
+    const TuneKey key{a.serial, L::kKind, K, octaveOf(count)};
     {
         std::lock_guard<std::mutex> lock(gTuneMutex);
-        const auto it = gTuned.find(key);
-        if (it != gTuned.end()) return {it->second, false};
+        const bool again = gTuned.count(key) != 0 && gTuned[key] == kCalledOnce;
+        const int shape = keptShape(key, a.wideCount);
+        if (shape != kCalledOnce && !again) {
+            if (gTuned.size() >= kKeptMax) gTuned.clear();
+            gTuned.emplace(key, kCalledOnce);
+            return {shape, false};
+        }
     }
     constexpr int kShapes = K <= 16 ? 3 : 2;
     const int shapes[3] = {kShapeGroup32, kShapeWave, kShapeGroup16};
@@ -2494,25 +2530,17 @@ static TunedShape tunedShape(const TraverseArgs& a, const V3* pts, int count, in
             bestMs = ms;
         }
     }
-    std::lock_guard<std::mutex> lock(gTuneMutex);
-    if (gTuned.size() >= 4096) gTuned.clear();  // trees come and go; keep the table small
-    gTuned[key] = best;
+    keepShape(key, a.wideCount, best);
     return {best, true};
 }
 
-// The shape an earlier tuning chose for this tree and size class, else the measured
+// The shape an earlier tuning chose for this tree or a like call, else the measured
 // crossovers' (no timing trials).
 template <typename L, int K>
 static int cachedShape(const TraverseArgs& a, int count) {
-    int octave = 0;
-    while ((2LL << octave) <= count) ++octave;
-    const TuneKey key{a.serial, L::kKind, K, octave};
-    {
-        std::lock_guard<std::mutex> lock(gTuneMutex);
-        const auto it = gTuned.find(key);
-        if (it != gTuned.end()) return it->second;
-    }
-    return defaultShape<L, K>(count);
+    std::lock_guard<std::mutex> lock(gTuneMutex);
+    const int shape = keptShape({a.serial, L::kKind, K, octaveOf(count)}, a.wideCount);
+    return shape != kCalledOnce ? shape : defaultShape<L, K>(count);
 }
 
 template <typename L, int K>
