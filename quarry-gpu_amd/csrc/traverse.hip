@@ -219,8 +219,9 @@ __device__ __forceinline__ bool closer(float d, int id, float bd, int bid) {
     return d < bd || (d == bd && id < bid);
 }
 
-// A query with a NaN coordinate has no closest primitive (index -1) and is not walked: its
-// box distances are 0 and no distance of it ever bounds them, so every node would be opened.
+// A query with a NaN coordinate has no closest primitive (index -1) and is not walked (by
+// groups of lanes: not beyond the root): its box distances are 0 and no distance of it ever
+// bounds them, so every node would be opened.
 __device__ __forceinline__ bool hasNaN(V3 p) { return (p.x != p.x) | (p.y != p.y) | (p.z != p.z); }
 
 // ---- k best so far ------------------------------------------------------------------
@@ -1354,8 +1355,11 @@ struct GroupNearest {
         ld = kd = kInfBits;
         lid = kid = kNoPrim;
         if (gl == 0) stk[0] = 0;
-        int sp = hasNaN(p) ? 0 : 1;
-        while (sp > 0) {
+        // A NaN query ends at the root, however many children wait.  (A check before the walk
+        // holds the root's read until the query's: closest, 100k queries, 1 % more.)
+        const int done = hasNaN(p) ? INT_MAX : 0;
+        int sp = 1;
+        do {
             int take = takeOf(sp);
             int node = -1;
             bool cut = false;
@@ -1437,7 +1441,7 @@ struct GroupNearest {
                     sp = top;
                 }
             }
-        }
+        } while (sp > done);
     }
 
     // Nodes to take from a stack of sp entries: one per quad, fewer when the stack could
