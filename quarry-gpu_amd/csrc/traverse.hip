@@ -2478,13 +2478,39 @@ static int defaultShape(int count) {
 }
 
 // The shape for this tree and size class (see kTuneFrom); a call that times has its results
-// written already (done), every shape writing the same.  From
-// kTuneSplitFrom queries on each shape walks a third of the queries, so that the first call
-// on a new tree costs about what a later one does -- a mesh that moves is a new tree every
-// step; below, a third would not fill the device and say little, and each shape walks all.
-// The first to run finds the tree outside the caches; 32 lanes, seldom far from the better
-// of the other two, goes first.
+// written already (done), every shape writing the same.  From kTuneSplitFrom queries on
+// each shape walks a part of its own, so that such a call costs about what a later one does.
+// A part is every fourth run of 256 visits: contiguous parts of ordered queries are regions
+// of the scene, and the emptiest one's shape would win.  The first part is walked untimed,
+// since it finds the tree outside the caches.  With fewer queries a part would not fill the
+// device and say little: each shape walks all, after the first part.  (The parts are an
+// order made for this call: as a mapping inside the walks they cost every other call 1 %.)
 constexpr int kTuneSplitFrom = 3 * 65536;
+constexpr int kPartRun = 256;
+struct Parts {
+    int n;
+    int first[5];  // where each part begins in the order, and the end
+};
+static Parts partsOf(int count, int n) {
+    Parts p{n, {0}};
+    for (int i = 0; i < n; ++i) {  // whole rounds of n runs, then what is left
+        const int round = n * kPartRun, rest = count % round - i * kPartRun;
+        p.first[i + 1] = p.first[i] + count / round * kPartRun + std::min(std::max(rest, 0), kPartRun);
+    }
+    return p;
+}
+// The visits part by part.
+__global__ void partOrderKernel(const uint32_t* __restrict__ order, int count, Parts parts,
+                                uint32_t* __restrict__ out) {
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= count) return;
+    const int run = i / kPartRun, part = run % parts.n;
+    int first = 0;
+#pragma unroll
+    for (int p = 1; p < 4; ++p) first = part == p ? parts.first[p] : first;
+    out[first + run / parts.n * kPartRun + i % kPartRun] = order ? order[i] : static_cast<uint32_t>(i);
+}
+
 struct TunedShape {
     int shape;
     bool done;
@@ -2505,26 +2531,30 @@ static TunedShape tunedShape(const TraverseArgs& a, const V3* pts, int count, in
     }
     constexpr int kShapes = K <= 16 ? 3 : 2;
     const int shapes[3] = {kShapeGroup32, kShapeWave, kShapeGroup16};
+    QuietFree quiet;
+    DevBuf<uint32_t> visits;
+    try {
+        visits.alloc(static_cast<size_t>(count));
+    } catch (const OomError&) {  // the call itself needs no memory
+        return {defaultShape<L, K>(count), false};
+    }
+    const Parts parts = partsOf(count, kShapes + 1);
+    partOrderKernel<<<blocksFor(count, kBlock), kBlock, 0, s>>>(a.order, count, parts, visits.p);
     const bool split = count >= kTuneSplitFrom;
+    TraverseArgs part = a;
+    part.order = visits.p;
+    launchShape<L, K>(shapes[0], part, pts, parts.first[1], k, outStride, out, nullptr, s);
     EventSet<kShapes + 1> ev;
     ev.record(0, s);
     for (int i = 0; i < kShapes; ++i) {
-        const int begin = split ? static_cast<int>(static_cast<long long>(count) * i / kShapes) : 0;
-        const int end = split ? static_cast<int>(static_cast<long long>(count) * (i + 1) / kShapes) : count;
-        TraverseArgs part = a;
-        const V3* p = pts;
-        ClosestResult* o = out;
-        if (a.order) {
-            part.order = a.order + begin;
-        } else {
-            p += begin;
-            o += static_cast<size_t>(begin) * outStride;
-        }
-        launchShape<L, K>(shapes[i], part, p, end - begin, k, outStride, o, nullptr, s);
+        part.order = visits.p + parts.first[i + 1];
+        if (split) launchShape<L, K>(shapes[i], part, pts, parts.first[i + 2] - parts.first[i + 1], k, outStride, out, nullptr, s);
+        else launchShape<L, K>(shapes[i], a, pts, count, k, outStride, out, nullptr, s);
         ev.record(i + 1, s);
     }
     hipCheck(hipGetLastError(), "nearest tuning");
     ev.sync(kShapes);
+    quiet.begin();
     int best = shapes[0];
     float bestMs = 0.0f;
     for (int i = 0; i < kShapes; ++i) {

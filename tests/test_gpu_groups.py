@@ -383,3 +383,21 @@ def test_timed_shapes_belong_to_one_tree(A, orc):  # noqa: F811
     b.build_wide()
     assert eq(b.closest(q, wide=True)[0], want)
     assert kept() == before
+
+
+# every visit belongs to one part, whole runs of 256 or a piece of one at the end: below, at
+# and above the count from which the timed shapes share the queries
+@pytest.mark.parametrize("count", [65536, 196607, 196608, 196609, 197631, 200000])
+def test_timed_calls_answer_every_query(A, orc, count):  # noqa: F811
+    print(f"count={count}", flush=True)
+    items = scene(1, 700, 3)
+    q = np.random.default_rng(count).uniform(-40, 40, (count, 3)).astype(np.float32)
+    for k in (0, 3, 17):  # three shapes to time, and two
+        want = orc.knn_brute(1, items, q, k, threads=16)
+        for order in (A.ORDER_INPUT, A.ORDER_MORTON):
+            b = A.Bvh(1, items)
+            b.build_wide()
+            for _ in range(3):  # one of the first two times
+                got = (b.knn(q, k, order=order, wide=True) if k else b.closest(q, order=order, wide=True))[0]
+                assert eq(got, want), (k, order)
+            b.close()
