@@ -170,6 +170,15 @@ QR_HD RayPre rayPrepare(const Ray& ray) {
     return p;
 }
 
+// The farthest box entry that a hit no farther than t may lie behind: where the box test
+// with tMax = t ends.  A triangle's hit may come up to 1e-6 (relative and absolute) before
+// its own box's entry (tInsideBox), rounding on top: one slack alone is too short by an
+// ulp or two for grazing hits at t about 1,000.
+QR_HD float rayReach(float t) {
+    const float t1 = t * (1.0f + 1e-6f) + 1e-6f;
+    return t1 * (1.0f + 1e-6f) + 1e-6f;
+}
+
 QR_HD bool rayBoxPre(const RayPre& r, const Box& box, float tMax, float& tEnter) {
     float ax = (box.lo.x - r.o.x) * r.inv.x, bx = (box.hi.x - r.o.x) * r.inv.x;
     float ay = (box.lo.y - r.o.y) * r.inv.y, by = (box.hi.y - r.o.y) * r.inv.y;

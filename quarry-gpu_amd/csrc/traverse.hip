@@ -449,10 +449,9 @@ __device__ __forceinline__ int descend(const int (&c)[4], const bool (&ok)[4], L
     return next;
 }
 
-// The farthest entry distance, as ray stacks keep them (not below zero), that a hit
-// nearer than `best` may still lie behind: the box tests' slack; a negative best (a ray
-// whose tMin is negative) drops nothing at zero.
-__device__ __forceinline__ float stackReach(float best) { return fmaxf(best * (1.0f + 1e-6f) + 1e-6f, 0.0f); }
+// The same for entry distances as ray stacks keep them (not below zero): a negative best (a
+// ray whose tMin is negative) drops nothing at zero.
+__device__ __forceinline__ float stackReach(float best) { return fmaxf(rayReach(best), 0.0f); }
 
 // One lane per ray over 4-wide nodes, for large ray sets.  The leaves of an opened node are
 // tested one per lane and step, not slot by slot: the wave runs the triangle test (the
@@ -1692,7 +1691,7 @@ __global__ __launch_bounds__(kBlock) void rayWaveKernel(Nodes nodes, const Tri* 
                 best = t;
                 any |= got;
             }
-            const bool push = adm & !leaf & (tEnter <= best * (1.0f + 1e-6f) + 1e-6f);
+            const bool push = adm & !leaf & (tEnter <= rayReach(best));
             const unsigned long long pb = __ballot(push);
             if (pb != 0) {
                 const typename GroupBits<G>::Word pm = gb.of(pb);
