@@ -200,7 +200,6 @@ TraverseArgs argsFor(const BvhState& b, bool wide, bool arm = true) {
     a.wide = wide;
     a.nodes = b.nodes.p;
     a.nodeCount = b.nodeCount;
-    a.depth = b.depth;
     a.serial = b.serial;
     a.wideNodes = b.wide.p;
     a.wideCount = b.wideCount;

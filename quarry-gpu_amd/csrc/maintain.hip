@@ -305,6 +305,10 @@ void newTopology(BvhState& b) {
     b.depthValid = false;
     b.wideValid = false;
     b.wideCount = 0;
+    if (b.depth > kMaxTreeDepth) {
+        b.n = b.nodeCount = 0;
+        throw DeviceError("build: the tree is deeper than its builder's bound");
+    }
 }
 
 void reserveWide(BvhState& b) {

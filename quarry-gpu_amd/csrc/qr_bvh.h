@@ -128,6 +128,9 @@ void buildLbvhDevice(BvhState& b, int kind, const void* dItems, int n, hipStream
 void buildSahDevice(BvhState& b, int kind, const void* dItems, int n, hipStream_t s,
                     BuildTimingsC* t);
 
+// Levels of the deepest tree a builder makes, for the stacks of the walks: LBVH one per code
+// bit (30) and per bit of an index among equal codes (31), SAH 32 and log2(n).
+constexpr int kMaxTreeDepth = 64;
 // A builder has written a new topology: what was derived from the old one no longer holds.
 void newTopology(BvhState& b);
 

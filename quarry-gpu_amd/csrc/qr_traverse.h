@@ -15,8 +15,7 @@ struct TraverseArgs {
     int wideCount = 0;
     const void* items = nullptr;        // leaf-ordered primitives
     const int* primIds = nullptr;       // leaf slot -> scene index
-    int depth = 0;                      // of the binary tree
-    uint64_t serial = 0;                // of its topology
+    uint64_t serial = 0;                // of the tree's topology
     const uint32_t* order = nullptr;    // optional visiting order (lane i -> query order[i])
     unsigned long long* stats = nullptr;  // optional [node tests, leaf tests, overflows]
     // false: the walk shape comes from an earlier tuning of the same tree and size

@@ -823,7 +823,7 @@ __device__ __forceinline__ float quadGetF(float v) {
     return __int_as_float(quadGet<S>(__float_as_int(v)));
 }
 
-constexpr int kQuadDepth = 96;  // 3 x the deepest 4-wide level a tree here can have
+constexpr int kQuadDepth = 96;  // 3 x the deepest 4-wide level a tree here can have (kMaxTreeDepth / 2)
 
 // DPP quad permutation: lane s of each quad receives lane P[s] (2 bits per lane).
 template <int P>
@@ -1176,7 +1176,7 @@ __device__ __forceinline__ void waveSortPairs(float& k, int& v, int lane, int wi
 // its queries.  A round pops w entries and pushes at most 4w, and w is held to
 // (stack - kWaveHeadroom - sp) / 3 (at least 1), so sp stays below stack - kWaveHeadroom
 // except while popping one entry per round, which adds at most 3 per 4-wide level -- within
-// the headroom for trees up to 32 levels deep (the quad kernels' stack assumes the same).
+// the headroom for 32 levels, half of kMaxTreeDepth (the quad kernels' stack assumes the same).
 constexpr int kWaveStack = 1024;
 constexpr int kWaveHeadroom = 3 * 32 + 4;
 
@@ -1624,7 +1624,7 @@ __global__ __launch_bounds__(kBlock) void rayWaveKernel(Nodes nodes, const Tri* 
                                                         const int* __restrict__ primIds,
                                                         int* __restrict__ hitPrim, uint32_t idMask) {
     constexpr int kQuads = G / 4;
-    constexpr int kStack = G == 4 ? 96 : kWaveStack / (64 / G);
+    constexpr int kStack = kWaveStack / (64 / G);
     __shared__ int lds[kStack * (kBlock / G)];
     const int lane = threadIdx.x & 63;
     const int gl = lane & (G - 1);
@@ -1646,11 +1646,9 @@ __global__ __launch_bounds__(kBlock) void rayWaveKernel(Nodes nodes, const Tri* 
         int sp = 1;
         while (sp > 0) {
             int take = kQuads;
-            if constexpr (G > 4) {
-                const int room = kStack - kWaveHeadroom - sp;
-                if (room < 3 * kQuads) take = room < 3 ? 1 : room / 3;
-                take = take < sp ? take : sp;
-            }
+            const int room = kStack - kWaveHeadroom - sp;
+            if (room < 3 * kQuads) take = room < 3 ? 1 : room / 3;
+            take = take < sp ? take : sp;
             int node = -1;
             if (quad < take) {
                 const uint32_t v = static_cast<uint32_t>(stk[sp - 1 - quad]);
@@ -2164,11 +2162,6 @@ enum NearestShape : int {
     kShapeLane = 0, kShapeQuad = 1, kShapeWave = 2, kShapeGroup16 = 3, kShapeGroup32 = 4, kShapeGroup8 = 5
 };
 
-// Deepest binary tree the group walks take: their stacks have room for three entries on
-// each of 32 4-wide levels above what a round pushes.  Deeper trees (none of the builders
-// makes one from distinct boxes) go one lane per query, whose stack spills to scratch.
-constexpr int kGroupDepth = 64;
-
 // Tuned shapes.  The best shape depends on how long and how uneven the walks are, which
 // the query count alone does not tell: 262,144 closest queries on the terrain run fastest
 // 16 lanes per query (410 us, one wave per query 597), as many in and around an icosphere
@@ -2289,7 +2282,7 @@ constexpr int kRayLaneFrom = 393216;
 template <bool kSave>
 static int rayShape(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,
                     hipStream_t s) {
-    if (a.depth > kGroupDepth || gTraversalMode == 1) return kShapeLane;
+    if (gTraversalMode == 1) return kShapeLane;
     if (gTraversalMode == 3) return a.wide ? kShapeWave : kShapeLane;
     if (gTraversalMode != 4 || !a.wide) {
         if (count < 3072) return kShapeWave;
@@ -2346,10 +2339,6 @@ void launchRays(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out
 void launchRaysSave(const TraverseArgs& a, const Ray* rays, int count, uint64_t* out, int* hitPrim,
                     hipStream_t s) {
     launchRaysT<true>(a, rays, count, out, hitPrim, s);
-}
-
-namespace {
-
 }
 
 void setTraversalMode(int mode) { gTraversalMode = mode; }
@@ -2580,8 +2569,7 @@ template <typename L, int K>
 static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int k, int outStride,
                             ClosestResult* out, hipStream_t s) {
     const auto* prims = static_cast<const typename L::Item*>(a.items);
-    const bool deep = a.depth > kGroupDepth;
-    if (!a.wide && !deep && gTraversalMode != 1 && count < binaryLaneFrom<L>()) {
+    if (!a.wide && gTraversalMode != 1 && count < binaryLaneFrom<L>()) {
         launchShape<L, K>(defaultShape<L, K>(count), a, pts, count, k, outStride, out, a.stats, s);
         return;
     }
@@ -2595,7 +2583,7 @@ static void launchNearestTK(const TraverseArgs& a, const V3* pts, int count, int
     }
     int shape;
     bool tune = false;
-    switch (deep ? 1 : gTraversalMode) {
+    switch (gTraversalMode) {
         case 1: shape = kShapeLane; break;
         case 2: shape = kShapeQuad; break;
         case 3: shape = kShapeWave; break;
@@ -2648,7 +2636,7 @@ static void launchNearestT(const TraverseArgs& a, const V3* pts, int count, int 
 //   per ray (larger sets) profits: 1M down 370 / 341, 131k terrain 629 / 386.  Binary:
 //   terrain cosine 131k 227 / 216, 33k 87 / 102.
 bool orderingPays(const TraverseArgs& a, WalkKind walk, int count) {
-    if (gTraversalMode != 0 || a.depth > kGroupDepth) return true;  // forced shapes keep their order
+    if (gTraversalMode != 0) return true;  // forced shapes keep their order
     if (walk == kWalkRays) return count >= (a.wide ? kRayLaneFrom : 98304);
     if (!a.wide) return count >= (a.kind == 0 ? 12288 : 24576);
     return count >= (walk == kWalkClosest ? 131072 : 65536);
@@ -2676,8 +2664,8 @@ void launchKnn(const TraverseArgs& a, const V3* pts, int count, int k, int outSt
 }
 
 // Whether a radius call captures its hits in one walk (by groups of lanes, or on quads):
-// unless one lane per query is forced or the tree is deeper than those walks' stacks take.
-static bool radiusCaptures(const TraverseArgs& a) { return gTraversalMode != 1 && a.depth <= kGroupDepth; }
+// unless one lane per query is forced.
+static bool radiusCaptures() { return gTraversalMode != 1; }
 
 // cap > 0: a fill on quads after a capture (only the queries the capture could not
 // hold are walked); cap == 0: the per-lane count / fill kernels.
@@ -2776,7 +2764,7 @@ int radiusCaptureCap(int count) {
 bool launchRadiusCapture(const TraverseArgs& a, const V3* pts, int count, float r2, int* counts,
                          uint64_t* capture, int cap, int* maxCount, hipStream_t s) {
     if (count <= 0) return false;
-    if (!radiusCaptures(a) || cap <= 0) {
+    if (!radiusCaptures() || cap <= 0) {
         switch (a.kind) {
             case 0: launchRadiusT<TriLeaf, false>(a, pts, count, r2, counts, nullptr, nullptr, maxCount, 0, s); break;
             case 1: launchRadiusT<PointLeaf, false>(a, pts, count, r2, counts, nullptr, nullptr, maxCount, 0, s); break;

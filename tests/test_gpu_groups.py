@@ -154,6 +154,7 @@ def test_deep_tree(A, orc):  # noqa: F811
     b = A.Bvh(1, items, A.BUILDER_SAH)
     b.build_wide()
     print("depth", b.info().depth, flush=True)
+    assert 2 * 15 <= b.info().depth <= 64  # (15 if balanced; the walks' stacks are proven for 64)
     q = np.zeros((100, 3), np.float32)
     q[:, 0] = np.exp2(np.linspace(-100, 1, 100))
     for k in (0, 5):
@@ -401,3 +402,32 @@ def test_timed_calls_answer_every_query(A, orc, count):  # noqa: F811
                 got = (b.knn(q, k, order=order, wide=True) if k else b.closest(q, order=order, wide=True))[0]
                 assert eq(got, want), (k, order)
             b.close()
+
+
+@pytest.mark.parametrize("count", [100, 70000])  # by query count, and timed
+def test_deepest_lbvh(A, orc, count):  # noqa: F811
+    """One point per leading bit of the Morton code and 20,000 in one place, told apart by their
+    index: 30 + 15 levels, every 4-wide level with something to come back to."""
+    corner = np.zeros((31, 3), np.float32)
+    for bit in range(30):  # bit 3 i + a of the code is bit i of axis a's 10
+        corner[bit, bit % 3] = 2.0 ** (bit // 3)
+    corner[30] = 1023.0
+    items = np.concatenate([corner, np.zeros((20000, 3), np.float32)])
+    b = A.Bvh(1, items)
+    b.build_wide()
+    print("depth", b.info().depth, flush=True)
+    assert 40 < b.info().depth <= 64
+    q = np.random.default_rng(1).uniform(-1, 1, (count, 3)).astype(np.float32)
+    q *= np.exp2(np.random.default_rng(2).uniform(-2, 10, (count, 1))).astype(np.float32)
+    for mode in (0, 1):
+        A.lib().qr_set_traversal_mode(mode)
+        try:
+            for k in (0, 5):
+                for wide in (False, True):
+                    got = (b.knn(q, k, wide=wide) if k else b.closest(q, wide=wide))[0]
+                    assert eq(got[:100], orc.knn_brute(1, items, q[:100], k, threads=8)), (mode, k, wide)
+            o, keys, _, _ = b.radius(q[:100], 3.0, wide=True)
+            wo, wk = orc.radius_brute(1, items, q[:100], 3.0, threads=8)
+            assert eq(o, wo) and eq(keys, wk), mode
+        finally:
+            A.lib().qr_set_traversal_mode(0)
