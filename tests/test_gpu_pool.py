@@ -13,6 +13,33 @@ from test_gpu_parity import A, eq, random_tris  # noqa: F401
 pytestmark = pytest.mark.gpu
 
 
+def used(torch_free_before):
+    return torch_free_before - torch.cuda.mem_get_info()[0]
+
+
+def alloc(A, n):  # noqa: F811
+    p = ctypes.c_void_p()
+    A.check(A.lib().qr_dev_alloc(n, ctypes.byref(p)))
+    return p
+
+
+def side_stream_work(stream, ms=300):
+    """Queues about that much work on the stream: products of one size, timed once."""
+    with torch.cuda.stream(stream):
+        m = torch.ones((4096, 4096), device="cuda")
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        out = torch.mm(m, m)
+        a.record()
+        torch.mm(m, m, out=out)
+        b.record()
+        b.synchronize()
+        for _ in range(int(ms / max(a.elapsed_time(b), 0.05)) + 1):
+            torch.mm(m, m, out=out)
+        done = torch.cuda.Event()
+        done.record()
+    return done
+
+
 def test_alloc_free_trim(A):  # noqa: F811
     L = A.lib()
     held = []
@@ -38,27 +65,79 @@ def test_alloc_free_trim(A):  # noqa: F811
 
 
 def test_free_waits_for_queued_work(A, orc):  # noqa: F811
-    """The adjoint call returns before its kernel ends; the tree destroyed right after it
-    must not give its arrays to the next build early."""
+    """A buffer and a tree freed while kernels that read them are still queued on a
+    non-blocking stream: their memory must not reach the next owner before those end."""
+    L = A.lib()
     rng = np.random.default_rng(2)
     items = random_tris(rng, 20000)
     q = rng.uniform(-30, 30, (60000, 3)).astype(np.float32)
-    dq, ones = A.DeviceArray(q), A.DeviceArray(np.ones(q.shape[0], np.float32))
-    res, aux = A.DeviceArray.empty((q.shape[0], 2), np.uint32), A.DeviceArray.empty(q.shape[0], np.int32)
+    n = q.shape[0]
+    stream = torch.cuda.Stream()
     want = None
-    for _ in range(5):
+    for late in (False, True):
         b = A.Bvh(0, items)
-        b.build_wide()
+        ones = A.DeviceArray(np.ones(n, np.float32))
+        res, aux = A.DeviceArray.empty((n, 2), np.uint32), A.DeviceArray.empty(n, np.int32)
+        pts = alloc(A, q.nbytes)
+        A.check(L.qr_dev_upload(pts, A.ptr(q), q.nbytes))
         ms = ctypes.c_double()
-        A.check(A.lib().qr_closest_device(b.h, dq.ptr, q.shape[0], res.ptr, A.ORDER_MORTON, 1, ctypes.byref(ms)))
-        A.check(A.lib().qr_closest_save_aux(b.h, dq.ptr, q.shape[0], res.ptr, aux.ptr))
-        g = A.DeviceArray.empty((q.shape[0], 3), np.float32)
-        A.check(A.lib().qr_adjoint_closest(b.h, dq.ptr, q.shape[0], res.ptr, aux.ptr, ones.ptr, g.ptr, None))
-        b.close()
-        A.Bvh(0, items[::-1].copy()).close()
+        A.check(L.qr_closest_device(b.h, pts, n, res.ptr, A.ORDER_MORTON, 0, ctypes.byref(ms)))
+        A.check(L.qr_closest_save_aux(b.h, pts, n, res.ptr, aux.ptr))
+        g = A.DeviceArray.empty((n, 3), np.float32)
+        A.check(L.qr_dev_trim())
+        A.check(L.qr_set_stream(ctypes.c_void_p(stream.cuda_stream)))
+        try:
+            done = side_stream_work(stream) if late else None
+            A.check(L.qr_adjoint_closest(b.h, pts, n, res.ptr, aux.ptr, ones.ptr, g.ptr, None))
+        finally:
+            A.check(L.qr_set_stream(None))
+        if late:
+            assert not done.query()  # the adjoint has not begun
+            A.check(L.qr_dev_free(pts))
+            other = alloc(A, q.nbytes)
+            assert other.value == pts.value
+            A.check(L.qr_dev_upload(other, A.ptr(np.zeros_like(q)), q.nbytes))
+            b.close()
+            A.Bvh(0, items[::-1].copy()).close()
+        torch.cuda.synchronize()
         got = g.download()
         want = got if want is None else want
-        assert eq(got, want)
+        assert eq(got, want), late
+        A.check(L.qr_dev_free(pts))  # (late: the block's second owner)
+
+
+def test_destroying_a_tree_waits_for_queued_work(A, orc):  # noqa: F811
+    L = A.lib()
+    rng = np.random.default_rng(2)
+    items = random_tris(rng, 20000)
+    q = rng.uniform(-30, 30, (60000, 3)).astype(np.float32)
+    n = q.shape[0]
+    dq, ones = A.DeviceArray(q), A.DeviceArray(np.ones(n, np.float32))
+    res, aux = A.DeviceArray.empty((n, 2), np.uint32), A.DeviceArray.empty(n, np.int32)
+    stream = torch.cuda.Stream()
+    want = None
+    for late in (False, True):
+        b = A.Bvh(0, items)
+        ms = ctypes.c_double()
+        A.check(L.qr_closest_device(b.h, dq.ptr, n, res.ptr, A.ORDER_MORTON, 0, ctypes.byref(ms)))
+        A.check(L.qr_closest_save_aux(b.h, dq.ptr, n, res.ptr, aux.ptr))
+        g = A.DeviceArray.empty((n, 3), np.float32)
+        A.check(L.qr_set_stream(ctypes.c_void_p(stream.cuda_stream)))
+        try:
+            done = side_stream_work(stream) if late else None
+            A.check(L.qr_adjoint_closest(b.h, dq.ptr, n, res.ptr, aux.ptr, ones.ptr, g.ptr, None))
+        finally:
+            A.check(L.qr_set_stream(None))
+        was = {b.info().d_nodes, b.info().d_items, b.info().d_prim_ids}
+        assert not late or not done.query()
+        b.close()
+        c = A.Bvh(0, items[::-1].copy())
+        assert not late or c.info().d_items in was  # the same memory, other contents
+        torch.cuda.synchronize()
+        got = g.download()
+        want = got if want is None else want
+        assert eq(got, want), late
+        c.close()
 
 
 def test_threads_and_streams(A, orc):  # noqa: F811
@@ -90,23 +169,6 @@ def test_threads_and_streams(A, orc):  # noqa: F811
     assert not wrong, wrong
 
 
-def side_stream_work(stream, ms=300):
-    """Queues about that much work on the stream: products of one size, timed once."""
-    with torch.cuda.stream(stream):
-        m = torch.ones((4096, 4096), device="cuda")
-        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        out = torch.mm(m, m)
-        a.record()
-        torch.mm(m, m, out=out)
-        b.record()
-        b.synchronize()
-        for _ in range(int(ms / max(a.elapsed_time(b), 0.05)) + 1):
-            torch.mm(m, m, out=out)
-        done = torch.cuda.Event()
-        done.record()
-    return done
-
-
 def test_radius_results_do_not_wait_for_other_streams(A, orc):  # noqa: F811
     """A radius result whose device pointers nobody asked for has no reader left once the call
     returned: neither destroying it nor a grown key buffer inside the call waits for the work
@@ -135,16 +197,6 @@ def test_radius_results_do_not_wait_for_other_streams(A, orc):  # noqa: F811
     assert not done.query()
     A.check(L.qr_radius_destroy(csr))
     assert done.query()
-
-
-def used(torch_free_before):
-    return torch_free_before - torch.cuda.mem_get_info()[0]
-
-
-def alloc(A, n):  # noqa: F811
-    p = ctypes.c_void_p()
-    A.check(A.lib().qr_dev_alloc(n, ctypes.byref(p)))
-    return p
 
 
 def test_cached_blocks_are_bounded_and_given_back(A):  # noqa: F811
