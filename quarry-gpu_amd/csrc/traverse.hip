@@ -2488,8 +2488,8 @@ static Parts partsOf(int count, int n) {
     return p;
 }
 // The visits part by part.
-__global__ void partOrderKernel(const uint32_t* __restrict__ order, int count, Parts parts,
-                                uint32_t* __restrict__ out) {
+static __global__ void partOrderKernel(const uint32_t* __restrict__ order, int count, Parts parts,
+                                       uint32_t* __restrict__ out) {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= count) return;
     const int run = i / kPartRun, part = run % parts.n;
