@@ -18,8 +18,8 @@ struct TraverseArgs {
     uint64_t serial = 0;                // of the tree's topology
     const uint32_t* order = nullptr;    // optional visiting order (lane i -> query order[i])
     unsigned long long* stats = nullptr;  // optional [node tests, leaf tests, overflows]
-    // false: the walk shape comes from an earlier tuning of the same tree and size
-    // class or from the measured crossovers, never from timing trials on this call
+    // false: the walk shape comes from an earlier tuning of the same tree or a like call,
+    // or from the measured crossovers, never from timing trials on this call
     bool tune = true;
 };
 

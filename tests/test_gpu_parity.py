@@ -437,8 +437,8 @@ def test_wave_walk_on_identical_items(A, orc, scenes, kind):
 
 
 def test_tuned_shape_on_large_sets(A, orc, scenes):
-    """From 65,536 queries the automatic mode tunes the shape on the first call (the
-    trials write the output); the first and later calls give the oracle's bits."""
+    """From 65,536 queries the automatic mode tunes the shape on one of the first two calls
+    (the trials write the output); all calls give the oracle's bits."""
     tris = scenes.terrain(64, 3)
     b = A.Bvh(0, tris)
     b.build_wide()
